@@ -313,3 +313,34 @@ def test_llama3_8b_parameter_set_round_trip_and_column_split(kvx, cuda):
             for b, c in zip(bounds, chunk):
                 assert torch.equal(c.view(torch.int16), m[:, b[1][0]:b[1][1]].view(torch.int16))
     ws.close()
+
+
+@pytest.mark.parametrize("use_plan", [False, True])
+def test_strided_copy_any_alignment_matches_oracle(kvx, cuda, use_plan):
+    """Entries of every size from 1 to 33 bytes and around a tile's edge, in
+    rows at odd addresses and strides, with aligned long rows in the same
+    launch: each entry moves at its own vector width, its last vector stepped
+    back to the row's end, and no byte outside the rows changes."""
+    rng = np.random.default_rng(23)
+    T = 32768
+    shapes = [(s, int(rng.integers(1, 90)), int(rng.integers(0, 9)), int(rng.integers(0, 9)))
+              for s in range(1, 34)]
+    shapes += [(s, 3, 1, 3) for s in (T - 1, T, T + 1, T + 15, 2 * T + 17, 33 * T - 5)]
+    shapes += [(2730, 700, 5462, 0), (4 * T, 1, 0, 0), (1, 1, 0, 0), (4, 5000, 0, 0)]
+    ora, s_pos, d_pos = [], 1, 3
+    for k in rng.permutation(len(shapes)):
+        size, count, s_extra, d_extra = shapes[k]
+        if size == 4 * T:
+            s_pos, d_pos = (s_pos + 15) // 16 * 16, (d_pos + 15) // 16 * 16
+        s_stride, d_stride = size + s_extra, size + d_extra
+        ora.append((s_pos, d_pos, size, count, s_stride, d_stride))
+        s_pos += (count - 1) * s_stride + size + int(rng.integers(0, 4))
+        d_pos += (count - 1) * d_stride + size + int(rng.integers(1, 4))
+    src_np = rng.integers(0, 256, s_pos, dtype=np.uint8)
+    want = rng.integers(0, 256, d_pos, dtype=np.uint8)
+    src, dst = torch.from_numpy(src_np).to(cuda), torch.from_numpy(want.copy()).to(cuda)
+    W.apply_entries(src_np, want, ora)
+    entries = [kvx.StridedEntry(src.data_ptr() + a, dst.data_ptr() + b, sz, c, ss, ds)
+               for a, b, sz, c, ss, ds in ora]
+    kvx.copy_strided(kvx.StridedPlan(entries) if use_plan else entries, device=0).Await()
+    assert np.array_equal(u8(dst), want)

@@ -183,7 +183,6 @@ class StridedCopyPlan {
  private:
   StridedCopyPlan() = default;
   int device_ = 0;
-  int vec_ = 16;
   uint32_t n_ = 0;
   uint32_t grid_ = 0;
   uint32_t long_tiles_ = 0;  // the first tiles of the grid, long rows (sliced)

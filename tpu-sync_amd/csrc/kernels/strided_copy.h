@@ -41,16 +41,21 @@ struct StridedEntryDev {
   uint32_t tile_begin;     // first workgroup of the entry
   uint32_t rows_per_tile;  // > 0: whole rows per workgroup
   uint32_t tiles_per_row;  // > 0: a row spans this many workgroups
-  uint32_t pad;
+  uint16_t vec;            // vector bytes: 16, 8, 4, 2 or 1
+  uint16_t tail;           // bytes by which a row's last vector is stepped back
 };
 static_assert(sizeof(StridedEntryDev) == 64, "device table layout");
 
-// Builds the device table for `copies` with vector width `vec_bytes`;
-// returns false if an entry violates the kernel's limits. *grid receives the
+// Builds the device table for `copies`; returns false if an entry violates
+// the kernel's limits. any_align: both sides are device memory, and each entry
+// takes the widest vectors its rows hold, at any address (a row's last vector
+// overlaps the one before it where the row is no whole number of them).
+// Otherwise (one side is host memory over PCIe, where an unaligned access
+// becomes several) every entry takes the common width `vec_bytes`. *grid receives the
 // workgroup count. Entries whose rows span more than one tile come first in
 // the table (in the copies' order, then the others in theirs); *long_tiles
 // (if not null) receives their tiles, the first of the grid.
-bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes,
+bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes, bool any_align,
                        std::vector<StridedEntryDev>* table, uint32_t* grid,
                        uint32_t* long_tiles = nullptr);
 
@@ -66,7 +71,7 @@ int StridedVectorBytes(const std::vector<StridedCopy>& copies);
 // its workgroups share a CU, and at 16-byte vectors moves the long-row tiles
 // sliced (0: every tile contiguous).
 hipError_t LaunchStridedCopy(const StridedEntryDev* table_dev, uint32_t n,
-                             uint32_t tiles, int vec_bytes, hipStream_t stream,
+                             uint32_t tiles, hipStream_t stream,
                              uint32_t max_workgroups = 0, uint32_t long_tiles = 0);
 
 }  // namespace kvx

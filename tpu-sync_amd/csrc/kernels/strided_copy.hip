@@ -12,6 +12,17 @@
 // scalar loads; lanes find their row with a multiply-shift instead of a
 // division. Loads and stores are non-temporal (every byte is touched once).
 //
+// Every entry has a vector width of its own. In HBM that is the widest power
+// of two up to 16 that a row holds, at any byte address: gfx950 serves
+// unaligned 16-byte accesses about as fast as aligned ones (a wave's accesses
+// are contiguous, so only the lines at its two ends are shared), and a row
+// that is not a whole number of vectors ends with one that is stepped back to
+// the row's last byte, rewriting a few bytes with the same values. Measured
+// against one width for the whole launch that divides every address, size and
+// stride: four bf16 [14336, 4096] split 3 ways (2730-byte rows) 511 -> 195 us,
+// 0.87 GB of 8-bit weights with a 4-byte scale each packed in 500 -> 287 us
+// (a whole call; floors 140 and 260 us at this kernel's 6.7 TB/s).
+//
 // At 16-byte vectors with one workgroup per tile, tiles go sliced: in a
 // group of 32 consecutive tiles (of one long row, or of one entry's runs of
 // short rows) the workgroup holding tile j moves the j-th 1 KiB of each of
@@ -48,11 +59,36 @@ constexpr uint32_t kLdsPerCu = 160u << 10;
 // of 8 lower at 2). While such a launch runs, its CUs' LDS is taken.
 constexpr uint32_t kWorkgroupsPerCu = 2;
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// A vector of V bytes at any byte address.
+template <int V> struct VecT;
+template <> struct VecT<16> {
+  typedef uint32_t T __attribute__((ext_vector_type(4), aligned(1)));
+};
+template <> struct VecT<8> {
+  typedef uint32_t T __attribute__((ext_vector_type(2), aligned(1)));
+};
+template <> struct VecT<4> { typedef uint32_t T __attribute__((aligned(1))); };
+template <> struct VecT<2> { typedef uint16_t T __attribute__((aligned(1))); };
+template <> struct VecT<1> { typedef uint8_t T; };
 
 #define KVX_GLOBAL __attribute__((address_space(1)))
 #define KVX_CONST __attribute__((address_space(4)))
+
+template <int V>
+__device__ __forceinline__ typename VecT<V>::T ld(uint64_t a) {
+  return __builtin_nontemporal_load((const KVX_GLOBAL typename VecT<V>::T*)a);
+}
+template <int V>
+__device__ __forceinline__ void st(uint64_t a, typename VecT<V>::T v) {
+  __builtin_nontemporal_store(v, (KVX_GLOBAL typename VecT<V>::T*)a);
+}
+
+// Byte offset of vector v of a row of `vecs` vectors, the last one stepped
+// back by `tail` bytes.
+template <int V>
+__device__ __forceinline__ uint64_t vec_offset(uint64_t v, uint32_t vecs, uint32_t tail) {
+  return v * V - (v == vecs - 1 ? tail : 0);
+}
 
 struct KArgs {
   const StridedEntryDev* table;
@@ -70,14 +106,14 @@ constexpr uint32_t kSliceVecs = 64;
 constexpr uint32_t kSliceTiles = kTileVecs / kSliceVecs;
 static_assert(kSliceTiles == kUnroll * (kThreads / 64), "one slice per wave and step");
 
-template <typename V>
+template <int V>
 __device__ __forceinline__ void copy_sliced(uint64_t src, uint64_t dst, uint32_t vecs,
-                                            uint32_t ct) {
+                                            uint32_t tail, uint32_t ct) {
   const uint32_t j = ct & (kSliceTiles - 1);
   const uint64_t first = static_cast<uint64_t>(ct - j) * kTileVecs + j * kSliceVecs;
   const uint32_t wave = threadIdx.x / 64;
   const uint32_t lane = threadIdx.x % 64;
-  V r[kUnroll];
+  typename VecT<V>::T r[kUnroll];
   uint64_t vi[kUnroll];
   // As in copy_tile: every load goes out (lanes past the row re-read its
   // last vector); only the stores are predicated.
@@ -86,12 +122,12 @@ __device__ __forceinline__ void copy_sliced(uint64_t src, uint64_t dst, uint32_t
     const uint32_t c = u * (kThreads / 64) + wave;  // tile of the group
     vi[u] = first + static_cast<uint64_t>(c) * kTileVecs + lane;
     const uint64_t vl = vi[u] < vecs ? vi[u] : vecs - 1;
-    r[u] = __builtin_nontemporal_load((const KVX_GLOBAL V*)(src + vl * sizeof(V)));
+    r[u] = ld<V>(src + vec_offset<V>(vl, vecs, tail));
   }
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
     if (vi[u] < vecs) {
-      __builtin_nontemporal_store(r[u], (KVX_GLOBAL V*)(dst + vi[u] * sizeof(V)));
+      st<V>(dst + vec_offset<V>(vi[u], vecs, tail), r[u]);
     }
   }
 }
@@ -99,7 +135,7 @@ __device__ __forceinline__ void copy_sliced(uint64_t src, uint64_t dst, uint32_t
 // Slice j of each tile of the group of kSliceTiles tiles from tile tb of an
 // entry of short rows (rows_per_tile rows per tile; only the entry's last
 // tile may hold fewer).
-template <typename V>
+template <int V>
 __device__ __forceinline__ void copy_sliced_rows(const KVX_CONST StridedEntryDev& ent,
                                                  uint32_t tb, uint32_t j) {
   const uint32_t wave = threadIdx.x / 64;
@@ -107,7 +143,7 @@ __device__ __forceinline__ void copy_sliced_rows(const KVX_CONST StridedEntryDev
   const uint32_t rpt = ent.rows_per_tile;
   const uint32_t vecs = ent.vecs;
   const uint64_t magic = ent.div_magic;
-  V r[kUnroll];
+  typename VecT<V>::T r[kUnroll];
   uint64_t doff[kUnroll];
   bool valid[kUnroll];
 #pragma unroll
@@ -122,39 +158,39 @@ __device__ __forceinline__ void copy_sliced_rows(const KVX_CONST StridedEntryDev
     const uint32_t kk = valid[u] ? k : total - 1;
     const uint32_t row = static_cast<uint32_t>((kk * magic) >> 32);
     const uint64_t r_abs = row0 + row;
-    const uint64_t col = static_cast<uint64_t>(kk - row * vecs) * sizeof(V);
-    r[u] = __builtin_nontemporal_load(
-        (const KVX_GLOBAL V*)(ent.src + r_abs * ent.src_stride + col));
+    const uint64_t col = vec_offset<V>(kk - row * vecs, vecs, ent.tail);
+    r[u] = ld<V>(ent.src + r_abs * ent.src_stride + col);
     doff[u] = r_abs * ent.dst_stride + col;
   }
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
-    if (valid[u]) __builtin_nontemporal_store(r[u], (KVX_GLOBAL V*)(ent.dst + doff[u]));
+    if (valid[u]) st<V>(ent.dst + doff[u], r[u]);
   }
 }
 
-// Moves tile `wg` (one entry's rows, or one slice of a long row).
-template <typename V>
-__device__ __forceinline__ void copy_tile(const KArgs& a, uint32_t wg) {
-  const uint32_t e = ((const KVX_CONST uint32_t*)a.tile_entry)[wg];
-  const KVX_CONST StridedEntryDev* ent = (const KVX_CONST StridedEntryDev*)a.table + e;
+// Moves tile `wg` of entry `ent` (some of its rows, or one slice of a long
+// row) in vectors of V bytes.
+template <int V>
+__device__ __forceinline__ void copy_tile_v(const KArgs& a, const KVX_CONST StridedEntryDev* ent,
+                                            uint32_t wg) {
   const uint64_t src = ent->src;
   const uint64_t dst = ent->dst;
   const uint64_t sstride = ent->src_stride;
   const uint64_t dstride = ent->dst_stride;
   const uint32_t vecs = ent->vecs;
+  const uint32_t tail = ent->tail;
   const uint32_t t = wg - ent->tile_begin;
-  if (a.sliced && ent->rows_per_tile == 0) {
+  if (V == 16 && a.sliced && ent->rows_per_tile == 0) {
     const uint32_t tpr = ent->tiles_per_row;
     const uint32_t row = t / tpr;
     const uint32_t ct = t - row * tpr;
     // Tiles in whole groups go sliced; a row's last tiles (fewer than a
     // group) stay contiguous.
     if (ct < (tpr & ~(kSliceTiles - 1))) {
-      copy_sliced<V>(src + row * sstride, dst + row * dstride, vecs, ct);
+      copy_sliced<V>(src + row * sstride, dst + row * dstride, vecs, tail, ct);
       return;
     }
-  } else if (a.sliced) {
+  } else if (V == 16 && a.sliced) {
     const uint32_t rpt = ent->rows_per_tile;
     const uint32_t ntiles = (ent->count + rpt - 1) / rpt;
     const uint32_t tb = t & ~(kSliceTiles - 1);
@@ -184,7 +220,7 @@ __device__ __forceinline__ void copy_tile(const KArgs& a, uint32_t wg) {
   const uint32_t total = nrows * nv;
   const uint32_t last = total - 1;
   const uint64_t magic = ent->div_magic;
-  V r[kUnroll];
+  typename VecT<V>::T r[kUnroll];
   uint64_t doff[kUnroll];
   // Every lane issues all kUnroll loads unconditionally (lanes past the end
   // of the tile re-read its last vector), so the loads go out back to back;
@@ -197,15 +233,28 @@ __device__ __forceinline__ void copy_tile(const KArgs& a, uint32_t wg) {
     const uint32_t row = nrows == 1 ? 0u : static_cast<uint32_t>((k * magic) >> 32);
     const uint32_t v = k - row * nv;
     const uint64_t r_abs = row0 + row;
-    const uint64_t col = static_cast<uint64_t>(v0 + v) * sizeof(V);
-    r[u] = __builtin_nontemporal_load((const KVX_GLOBAL V*)(src + r_abs * sstride + col));
+    const uint64_t col = vec_offset<V>(v0 + v, vecs, tail);
+    r[u] = ld<V>(src + r_abs * sstride + col);
     doff[u] = r_abs * dstride + col;
   }
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
     if (threadIdx.x + u * kThreads < total) {
-      __builtin_nontemporal_store(r[u], (KVX_GLOBAL V*)(dst + doff[u]));
+      st<V>(dst + doff[u], r[u]);
     }
+  }
+}
+
+// Moves tile `wg` at its entry's vector width (uniform in the workgroup).
+__device__ __forceinline__ void copy_tile(const KArgs& a, uint32_t wg) {
+  const uint32_t e = ((const KVX_CONST uint32_t*)a.tile_entry)[wg];
+  const KVX_CONST StridedEntryDev* ent = (const KVX_CONST StridedEntryDev*)a.table + e;
+  switch (ent->vec) {
+    case 16: copy_tile_v<16>(a, ent, wg); break;
+    case 8: copy_tile_v<8>(a, ent, wg); break;
+    case 4: copy_tile_v<4>(a, ent, wg); break;
+    case 2: copy_tile_v<2>(a, ent, wg); break;
+    default: copy_tile_v<1>(a, ent, wg); break;
   }
 }
 
@@ -224,15 +273,14 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t g, uint32_t tiles) {
 // The loop bound is uniform, so every wave leaves it together. With a full
 // grid the sliced tiles go in plain order (a group's workgroups on
 // consecutive ids) and the others in XCD order after them.
-template <typename V>
 __global__ __launch_bounds__(kThreads) void strided_copy_kernel(KArgs a) {
   if (gridDim.x == a.tiles) {
     const uint32_t g = blockIdx.x;
     const uint32_t L = a.sliced_tiles;
-    copy_tile<V>(a, g < L ? g : L + xcd_tile(g - L, a.tiles - L));
+    copy_tile(a, g < L ? g : L + xcd_tile(g - L, a.tiles - L));
     return;
   }
-  for (uint32_t t = blockIdx.x; t < a.tiles; t += gridDim.x) copy_tile<V>(a, t);
+  for (uint32_t t = blockIdx.x; t < a.tiles; t += gridDim.x) copy_tile(a, t);
 }
 
 }  // namespace
@@ -251,7 +299,7 @@ int StridedVectorBytes(const std::vector<StridedCopy>& copies) {
   return 1;
 }
 
-bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes,
+bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes, bool any_align,
                        std::vector<StridedEntryDev>* table, uint32_t* grid,
                        uint32_t* long_tiles) {
   table->clear();
@@ -266,8 +314,15 @@ bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes,
           c.src_stride < 0 || c.dst_stride < 0 || count > UINT32_MAX) {
         return false;
       }
-      const uint64_t vecs = static_cast<uint64_t>(c.size) / vec_bytes;
-      if (vecs > UINT32_MAX) return false;
+      // The limit on a row is the common width's, so that what a launch
+      // accepts does not depend on where it runs.
+      if (static_cast<uint64_t>(c.size) / vec_bytes > UINT32_MAX) return false;
+      uint64_t vec = static_cast<uint64_t>(vec_bytes);
+      if (any_align) {
+        vec = 16;
+        while (vec > static_cast<uint64_t>(c.size)) vec /= 2;
+      }
+      const uint64_t vecs = (static_cast<uint64_t>(c.size) + vec - 1) / vec;
       const bool long_row = vecs > kTileVecs;
       if (long_row != (pass == 0)) continue;
       StridedEntryDev d{};
@@ -279,6 +334,8 @@ bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes,
       d.vecs = static_cast<uint32_t>(vecs);
       d.div_magic = (uint64_t{1} << 32) / vecs + 1;
       d.tile_begin = static_cast<uint32_t>(tiles);
+      d.vec = static_cast<uint16_t>(vec);
+      d.tail = static_cast<uint16_t>(vecs * vec - static_cast<uint64_t>(c.size));
       uint64_t t;
       if (!long_row) {
         d.rows_per_tile = static_cast<uint32_t>(kTileVecs / vecs);
@@ -299,7 +356,7 @@ bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes,
 }
 
 hipError_t LaunchStridedCopy(const StridedEntryDev* table_dev, uint32_t n,
-                             uint32_t tiles, int vec_bytes, hipStream_t stream,
+                             uint32_t tiles, hipStream_t stream,
                              uint32_t max_workgroups, uint32_t long_tiles) {
   if (tiles == 0) return hipSuccess;
   KArgs a;
@@ -309,30 +366,12 @@ hipError_t LaunchStridedCopy(const StridedEntryDev* table_dev, uint32_t n,
   a.tiles = tiles;
   const uint32_t grid = max_workgroups > 0 && max_workgroups < tiles ? max_workgroups : tiles;
   // Slicing is measured at 16-byte vectors with one workgroup per tile.
-  a.sliced = vec_bytes == 16 && grid == tiles ? 1u : 0u;
+  a.sliced = grid == tiles ? 1u : 0u;
   a.sliced_tiles = a.sliced && long_tiles <= tiles ? long_tiles : 0;
   // HBM-bound launches take the occupancy cap; PCIe-bound ones (a capped
   // grid) keep their few workgroups spread without it.
   const uint32_t lds = max_workgroups == 0 ? kLdsPerCu / kWorkgroupsPerCu : 0;
-  switch (vec_bytes) {
-    case 16:
-      hipLaunchKernelGGL(strided_copy_kernel<u32x4>, dim3(grid), dim3(kThreads), lds, stream, a);
-      break;
-    case 8:
-      hipLaunchKernelGGL(strided_copy_kernel<u32x2>, dim3(grid), dim3(kThreads), lds, stream, a);
-      break;
-    case 4:
-      hipLaunchKernelGGL(strided_copy_kernel<uint32_t>, dim3(grid), dim3(kThreads), lds, stream, a);
-      break;
-    case 2:
-      hipLaunchKernelGGL(strided_copy_kernel<uint16_t>, dim3(grid), dim3(kThreads), lds, stream, a);
-      break;
-    case 1:
-      hipLaunchKernelGGL(strided_copy_kernel<uint8_t>, dim3(grid), dim3(kThreads), lds, stream, a);
-      break;
-    default:
-      return hipErrorInvalidValue;
-  }
+  hipLaunchKernelGGL(strided_copy_kernel, dim3(grid), dim3(kThreads), lds, stream, a);
   return hipGetLastError();
 }
 
