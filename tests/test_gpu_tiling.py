@@ -352,3 +352,65 @@ def test_weight_sync_rejects_small_tiled_buffers_and_chunks(kvx, cuda):
     ok = torch.zeros(L.tiled_bytes, dtype=torch.uint8, device=cuda)
     with pytest.raises(kvx.KvxError, match="tile row"):
         kvx.WeightSynchronizer([[ok]], layouts=[[L]], chunk_bytes=2000)
+
+
+@pytest.mark.parametrize("itemsize,P", [(1, 1), (1, 4), (2, 1), (2, 2), (4, 1), (8, 1)])
+def test_widths_that_are_no_whole_number_of_vectors(kvx, oracle, cuda, itemsize, P):
+    """Rows of every width around a vector's and a tile's edge, whose rows
+    start at any element and end inside a vector, in matrices of one row up
+    to past a tile row, from buffers off by one element: the last vector of a
+    row is stepped back when tiling and stored in part when detiling."""
+    rng = np.random.default_rng(31)
+    tiles = [[8, 128]] + ([[P, 1]] if P > 1 else [])
+    for W in (1, 2, 3, 5, 7, 8, 9, 15, 16, 17, 31, 33, 127, 129, 130, 143, 257, 1021):
+        for H, batch in ((1, []), (7, []), (8, [2]), (17, [])):
+            lay = dict(itemsize=itemsize, dims=batch + [H, W],
+                       minor_to_major=list(range(len(batch) + 1, -1, -1)), tiles=tiles)
+            print("tiling case", lay, flush=True)
+            check_layout(kvx, oracle, cuda, lay, rng, lin_off=itemsize * (W % 3),
+                         tiled_off=itemsize * (W % 2))
+
+
+def test_odd_width_larger_than_a_sliced_group(kvx, cuda):
+    """Odd-width packed matrices of more than 8 workgroups (sliced slots with
+    partial vectors), against the numpy formulation."""
+    for itemsize, P, H, W in ((2, 2, 1037, 2049), (1, 4, 1029, 4099)):
+        rng = np.random.default_rng(W)
+        dt = np.uint16 if itemsize == 2 else np.uint8
+        x = rng.integers(0, 1 << (8 * itemsize), (H, W), dtype=dt)
+        L = kvx.tiling.TiledLayout(itemsize, (H, W), [(8, 128), (P, 1)])
+        lin = torch.from_numpy(x.view(np.uint8).reshape(-1).copy()).to(cuda)
+        til = torch.full((L.tiled_bytes,), 0x5A, dtype=torch.uint8, device=cuda)
+        kvx.tiling.tile_buffer(L, lin, til).Await()
+        assert np.array_equal(u8(til), numpy_tile_2d(x, 8, 128, P).view(np.uint8))
+        out = torch.zeros_like(lin)
+        kvx.tiling.detile_buffer(L, til, out).Await()
+        assert torch.equal(out, lin)
+
+
+@pytest.mark.parametrize("chunk", [1 << 10, 20 << 10, 0])
+def test_weight_sync_odd_widths(kvx, oracle, cuda, chunk):
+    """Odd-width packed weights through staging chunks that hold no tile row
+    (cut between elements, moved element by element), a few, or all."""
+    rng = np.random.default_rng(chunk + 5)
+    lays = [dict(itemsize=2, dims=[37, 301], minor_to_major=[1, 0], tiles=[[8, 128], [2, 1]]),
+            dict(itemsize=1, dims=[2, 19, 135], minor_to_major=[2, 1, 0],
+                 tiles=[[8, 128], [4, 1]])]
+    layouts = [as_layout(kvx, l) for l in lays]
+    tensors = [torch.from_numpy(rng.integers(0, 256, L.tiled_bytes, dtype=np.uint8)).to(cuda)
+               for L in layouts]
+    dev0 = [u8(t) for t in tensors]
+    ws = kvx.WeightSynchronizer([[t] for t in tensors], layouts=[[l] for l in layouts],
+                                chunk_bytes=chunk)
+    ws.d2h().Await()
+    img = ws.host_image()
+    for k, lay in enumerate(lays):
+        _, n, off = ws.host_buffer_info(k, 0)
+        assert np.array_equal(img[off:off + n], oracle.detile(lay, dev0[k])), k
+        img[off:off + n] = rng.integers(0, 256, n, dtype=np.uint8)
+        tensors[k].fill_(0xA5)
+    ws.h2d().Await()
+    for k, lay in enumerate(lays):
+        _, n, off = ws.host_buffer_info(k, 0)
+        assert np.array_equal(u8(tensors[k]), oracle.tile(lay, img[off:off + n].copy())), k
+    ws.close()

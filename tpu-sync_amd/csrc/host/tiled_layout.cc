@@ -88,6 +88,18 @@ int WidestVector(uint64_t acc, int cap) {
   return 1;
 }
 
+// Vector width of a standard form's units: the widest that divides a row of a
+// tile (so that a vector never straddles two tiles) and that a row of the
+// matrix holds. The rows themselves may start at any address and end inside a
+// vector: a bf16 [4096, 32003] tiled into T(8,128)(2,1) takes 8-byte vectors
+// in 119 us a call (floor 78 at 6.7 TB/s), element by element with a clearing
+// pass 2066.
+int UnitVector(uint64_t W, uint64_t tW, uint64_t s) {
+  int v = WidestVector(tW * s, 16);
+  while (v > 1 && static_cast<uint64_t>(v) > W * s) v /= 2;
+  return v;
+}
+
 }  // namespace
 
 Status ValidateTiledLayout(const TiledLayout& l) {
@@ -160,6 +172,30 @@ int64_t TiledPlan::CutAtOrBelow(int64_t x) const {
   return (b * static_cast<int64_t>(H) + h / th * th) * row_bytes;
 }
 
+// Whether the standard form's units at vector width v stay within the
+// kernels' 32-bit unit indices and FastDivU32 divisors: linear order counts
+// B * ceil(H / P) * ceil(W * s / v) units, tiled order tiled_bytes / (P * v).
+static bool StdUnitsFit(const TiledPlan& p, int v, bool tile) {
+  if (v <= 0) return false;
+  const uint64_t s = static_cast<uint64_t>(p.layout.itemsize);
+  const uint64_t ng = (p.H + p.P - 1) / p.P;
+  const uint64_t ncv = (p.W * s + static_cast<uint64_t>(v) - 1) / static_cast<uint64_t>(v);
+  uint64_t units = 0;
+  if (ncv >= static_cast<uint64_t>(kDivLimit) || ng >= static_cast<uint64_t>(kDivLimit) ||
+      __builtin_mul_overflow(p.B * ng, ncv, &units) ||
+      units >= static_cast<uint64_t>(kU32Limit)) {
+    return false;
+  }
+  if (tile) {
+    const uint64_t ncvt = p.tW * s / static_cast<uint64_t>(v);
+    const uint64_t tunits = static_cast<uint64_t>(p.tiled_bytes) / (p.P * static_cast<uint64_t>(v));
+    if (ncvt >= static_cast<uint64_t>(kDivLimit) || tunits >= static_cast<uint64_t>(kU32Limit)) {
+      return false;
+    }
+  }
+  return true;
+}
+
 StatusOr<TiledPlan> PlanTiled(const TiledLayout& l) {
   KVX_RETURN_IF_ERROR(ValidateTiledLayout(l));
   TiledPlan p;
@@ -199,37 +235,35 @@ StatusOr<TiledPlan> PlanTiled(const TiledLayout& l) {
   } else {
     standard = false;
   }
+  bool geom = false;
   if (standard) {
     const uint64_t W = static_cast<uint64_t>(l.dims[r - 1]);
     const uint64_t H = r == 1 ? 1 : static_cast<uint64_t>(l.dims[r - 2]);
     const uint64_t B = static_cast<uint64_t>(logical) / (W * H);
     const int64_t tH = l.tiles[0][0], tW = l.tiles[0][1];
-    const int vec = WidestVector(static_cast<uint64_t>(W * s) | static_cast<uint64_t>(tW * s), 16);
-    const uint64_t ng = (H + P - 1) / P;
-    const uint64_t ncv = W * s / vec;
-    int64_t units = 0;
-    standard = H < static_cast<uint64_t>(kDivLimit) && W < static_cast<uint64_t>(kDivLimit) &&
-               tH <= kDivLimit && tW <= kDivLimit && (P == 1 || vec >= 4) &&
-               MulOk(static_cast<int64_t>(B * ng), static_cast<int64_t>(ncv), &units) &&
-               units < kU32Limit && B * ng < static_cast<uint64_t>(kU32Limit) &&
-               B * H < static_cast<uint64_t>(kU32Limit) && tH * tW < kDivLimit &&
-               p.tiled_bytes / (static_cast<int64_t>(P) * vec) < kU32Limit;
-    if (standard) {
-      p.standard = true;
-      p.P = P;
-      p.B = B;
-      p.H = H;
-      p.W = W;
-      p.tH = static_cast<uint64_t>(tH);
-      p.tW = static_cast<uint64_t>(tW);
-      p.nT0 = (H + p.tH - 1) / p.tH;
-      p.nT1 = (W + p.tW - 1) / p.tW;
-      p.vec = vec;
+    const int64_t BH = static_cast<int64_t>(B * H);
+    geom = H < static_cast<uint64_t>(kDivLimit) && W < static_cast<uint64_t>(kDivLimit) &&
+           tH <= kDivLimit && tW <= kDivLimit && BH < kU32Limit && tH * tW < kDivLimit;
+    p.P = P;
+    p.B = B;
+    p.H = H;
+    p.W = W;
+    p.tH = static_cast<uint64_t>(tH);
+    p.tW = static_cast<uint64_t>(tW);
+    p.nT0 = (H + p.tH - 1) / p.tH;
+    p.nT1 = (W + p.tW - 1) / p.tW;
+    // Whether the layout's aligned vectors make it standard; a packed layout
+    // whose rows are no whole number of 4-byte words is standard too, where
+    // the general form could take it.
+    p.vec = WidestVector(W * s | static_cast<uint64_t>(tW * s), 16);
+    p.standard = geom && (P == 1 || p.vec >= 4) && StdUnitsFit(p, p.vec, true);
+    if (geom && !p.standard) {
+      const int v = UnitVector(W, p.tW, s);
+      p.ragged = (P == 1 || v >= 4) && StdUnitsFit(p, v, true);
     }
   }
 
-  // General form (also the fallback of a standard layout whose buffers are
-  // too poorly aligned for its vectors): the final shape's dimensions.
+  // General form: the final shape's dimensions.
   std::vector<WorkDim> fin = ApplyTiles(l);
   bool gen_ok = logical < kU32Limit && fin.size() <= static_cast<size_t>(kTiledMaxGenDims);
   for (int64_t d : l.dims) gen_ok = gen_ok && d <= kDivLimit;
@@ -251,36 +285,13 @@ StatusOr<TiledPlan> PlanTiled(const TiledLayout& l) {
       p.gen[k] = g;
       stride *= fin[k].size;
     }
+    p.standard = p.standard || p.ragged;
   } else if (!p.standard) {
     return UnimplementedError(
         "tiled layout: general layouts need fewer than 2^32 elements, dimensions and tiles "
         "of at most 2^31 and at most 16 tiled dimensions");
   }
   return p;
-}
-
-// Whether the standard form's units at vector width v stay within the
-// kernels' 32-bit unit indices and FastDivU32 divisors: linear order counts
-// B * ceil(H / P) * (W * s / v) units, tiled order tiled_bytes / (P * v).
-static bool StdUnitsFit(const TiledPlan& p, int v, bool tile) {
-  if (v <= 0) return false;
-  const uint64_t s = static_cast<uint64_t>(p.layout.itemsize);
-  const uint64_t ng = (p.H + p.P - 1) / p.P;
-  const uint64_t ncv = p.W * s / static_cast<uint64_t>(v);
-  uint64_t units = 0;
-  if (ncv >= static_cast<uint64_t>(kDivLimit) || ng >= static_cast<uint64_t>(kDivLimit) ||
-      __builtin_mul_overflow(p.B * ng, ncv, &units) ||
-      units >= static_cast<uint64_t>(kU32Limit)) {
-    return false;
-  }
-  if (tile) {
-    const uint64_t ncvt = p.tW * s / static_cast<uint64_t>(v);
-    const uint64_t tunits = static_cast<uint64_t>(p.tiled_bytes) / (p.P * static_cast<uint64_t>(v));
-    if (ncvt >= static_cast<uint64_t>(kDivLimit) || tunits >= static_cast<uint64_t>(kU32Limit)) {
-      return false;
-    }
-  }
-  return true;
 }
 
 Status AppendTiledJobs(const TiledPlan& p, uint64_t tiled, uint64_t linear, int64_t lo,
@@ -299,9 +310,6 @@ Status AppendTiledJobs(const TiledPlan& p, uint64_t tiled, uint64_t linear, int6
   if (((tiled | linear) & static_cast<uint64_t>(s - 1)) != 0) {
     return InvalidArgumentError("tiled copy: buffers not aligned to the element size");
   }
-  // Units need vectors aligned on both buffers; a packed layout whose
-  // buffers allow less than 4 bytes goes element by element.
-  int v = WidestVector(tiled | linear, p.vec);
   // Packed units: one lane per unit with units of one 16-byte tiled vector
   // (v = 16 / P), except that detiling at 16-byte rows goes two lanes per
   // unit for pairs (P = 2) and four for quads (P = 4), exchanging through
@@ -315,28 +323,27 @@ Status AppendTiledJobs(const TiledPlan& p, uint64_t tiled, uint64_t linear, int6
   // (P = 4) at 16-byte rows, detiling: 71.6 % through LDS against 61.8 % for
   // one lane per 16-byte tiled vector; tiling keeps one lane per tiled
   // vector (72.3 % against 67.0 % through LDS).
-  bool two_lanes = false, four_lanes = false;
-  if (p.P == 2 && !tile && v == 16) {
-    two_lanes = true;
-  } else if (p.P == 4 && !tile && v == 16) {
-    four_lanes = true;
-  } else if (p.P > 1) {
-    v = std::min(v, 16 / static_cast<int>(p.P));
-  }
-  // PlanTiled checked the 32-bit unit and divisor limits at the plan's widest
-  // vector; narrower buffers multiply the unit counts, so they are checked
-  // again at the width chosen here (the kernels index units in 32 bits).
-  bool use_std = p.standard && (p.P == 1 || v >= 4);
-  if (use_std && !StdUnitsFit(p, v, tile)) use_std = false;
-  if (!use_std && p.standard && p.gen.empty()) {
+  auto packed = [&](int width) {
+    if (p.P == 1 || (!tile && width == 16)) return width;
+    return std::min(width, 16 / static_cast<int>(p.P));
+  };
+  const int v = p.standard ? packed(UnitVector(p.W, p.tW, static_cast<uint64_t>(s))) : 1;
+  const bool lanes = p.P > 1 && !tile && v == 16;
+  // The kernels index units in 32 bits. A tensor too large for the general
+  // form is taken only where its units fit at the vectors the buffers'
+  // alignment allows too, so that whether a size is accepted does not depend
+  // on which vectors move it.
+  const bool use_std = p.standard && StdUnitsFit(p, v, tile);
+  const int aligned = packed(WidestVector(tiled | linear, p.vec));
+  if (p.standard && p.gen.empty() &&
+      (!use_std || (p.P > 1 && aligned < 4) || !StdUnitsFit(p, aligned, tile))) {
     return UnimplementedError(
         "tiled copy: this layout has more 32-bit-indexed units than one launch can address "
         "at the buffers' alignment");
   }
-  const bool tiled_order = use_std && tile;
-  // Tiled-order units write the padding themselves; otherwise it is cleared
+  // Standard-form units write the padding themselves; otherwise it is cleared
   // first.
-  if (tile && zero_pass && p.padded && !tiled_order) {
+  if (tile && zero_pass && p.padded && !use_std) {
     const int v = WidestVector(tiled, p.zero_vec);
     TiledJob z;
     z.vec = v;
@@ -355,7 +362,7 @@ Status AppendTiledJobs(const TiledPlan& p, uint64_t tiled, uint64_t linear, int6
   if (use_std) {
     const uint64_t row_bytes = p.W * s;
     const uint64_t ng = (p.H + p.P - 1) / p.P;
-    const uint64_t ncv = row_bytes / v;
+    const uint64_t ncv = (row_bytes + v - 1) / v;
     auto group = [&](int64_t x) -> uint64_t {
       if (x >= p.logical_bytes) return p.B * ng;
       const uint64_t row = static_cast<uint64_t>(x) / row_bytes;
@@ -363,9 +370,9 @@ Status AppendTiledJobs(const TiledPlan& p, uint64_t tiled, uint64_t linear, int6
     };
     j.vec = v;
     j.dev.mode = tile ? kTileStd : kDetileStd;
-    j.dev.lanes_per_unit = two_lanes ? 2 : four_lanes ? 4 : 1;
-    j.dev.sliced = two_lanes || four_lanes ? 1u : 0u;
-    if (tiled_order) {
+    j.dev.lanes_per_unit = lanes ? p.P : 1;
+    j.dev.sliced = lanes ? 1u : 0u;
+    if (tile) {
       // Whole tile rows (cuts fall on them): units of tile rows [t_lo, t_hi).
       auto tile_row = [&](int64_t x) -> uint64_t {
         if (x >= p.logical_bytes) return p.B * p.nT0;
@@ -376,7 +383,6 @@ Status AppendTiledJobs(const TiledPlan& p, uint64_t tiled, uint64_t linear, int6
       const uint64_t ncvt = p.tW * s / v;
       const uint64_t per_tile_row = p.nT1 * gpt * ncvt;
       const uint64_t t_lo = tile_row(lo), t_hi = tile_row(hi);
-      j.dev.torder = 1;
       j.dev.lo = t_lo * per_tile_row;
       j.dev.count = (t_hi - t_lo) * per_tile_row;
       j.dev.t_ncv = MakeFastDivU32(static_cast<uint32_t>(ncvt));

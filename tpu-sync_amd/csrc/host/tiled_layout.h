@@ -54,10 +54,12 @@ struct TiledPlan {
   TiledLayout layout;
   bool tiled = false;     // has tiles (else a plain copy)
   bool standard = false;  // standard form (else general)
+  bool ragged = false;    // standard only since its vectors may start anywhere:
+                          // may go general instead (chunks below a tile row)
   bool padded = false;    // tiled elements > logical elements
   int64_t logical_bytes = 0;
   int64_t tiled_bytes = 0;
-  int vec = 16;       // widest vector the layout allows (standard form)
+  int vec = 16;       // widest vector that divides its rows (standard form)
   int zero_vec = 16;  // vector width of the zero pass
   // Standard form: batch matrices [B][H][W], tiles (tH, tW), P rows per unit.
   uint32_t P = 1;

@@ -93,6 +93,13 @@ Status WeightSynchronizer::Init() {
     if (tp == nullptr || !tp->standard) continue;
     const int64_t group =
         static_cast<int64_t>(std::min(tp->tH, tp->H) * tp->W) * tp->layout.itemsize;
+    if (group > chunk && tp->ragged) {
+      // The general form: chunks may be cut between any two elements.
+      auto general = std::make_shared<TiledPlan>(*tp);
+      general->standard = false;
+      cfg_.tiled[k] = general;
+      continue;
+    }
     if (group > chunk) {
       return InvalidArgumentError("tensor " + std::to_string(k) + ": a tile row (" +
                                   std::to_string(group) +

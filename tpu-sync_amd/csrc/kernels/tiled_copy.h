@@ -15,11 +15,12 @@
 //     P consecutive rows element by element, P in {2, 4} with P * itemsize =
 //     4). A unit is P rows x V bytes: V contiguous bytes of each of P linear
 //     rows and P * V contiguous bytes of the tiled buffer, moved by one lane
-//     or, for P = 2 at V = 16, by two lanes that exchange halves. Units are
-//     enumerated in linear order (row groups of the linear image, then column
-//     vectors) or in tiled order (unit u is bytes [u P V, (u + 1) P V) of the
-//     tiled buffer, padding included: rows past H and columns past W read as
-//     zero when tiling and are skipped when detiling).
+//     or, when detiling at V = 16, by P lanes that exchange through LDS. Rows
+//     may start at any address and need not be a whole number of vectors.
+//     Detiling enumerates units in linear order (row groups of the linear
+//     image, then column vectors), tiling in tiled order (unit u is bytes
+//     [u P V, (u + 1) P V) of the tiled buffer, padding included: rows past H
+//     and columns past W read as zero).
 //   * kDetileGen / kTileGen: any other layout, element by element through the
 //     index map of the nested tiling.
 //   * kZero: clears a tiled buffer (V-byte vectors), launched before a
@@ -110,10 +111,9 @@ struct TiledJobDev {
   FastDivU32 t_gpt;  // row groups per tile (GT = tH / P)
   FastDivU32 t_nt1;  // tile columns per matrix (nT1)
   FastDivU32 t_nt0;  // tile rows per matrix (nT0)
-  uint32_t torder;   // 0: linear order, 1: tiled order
   uint32_t lanes_per_unit;  // packed units: 1, or 2 (P = 2) / 4 (P = 4) detiling at 16-byte rows
   uint32_t sliced;  // detiling with 2 or 4 lanes per unit: slots in whole groups go sliced
-  uint32_t pad0;
+  uint32_t pad0[2];
   uint32_t h32;         // H (rows per batch matrix)
   uint32_t w32;         // W (columns)
   uint32_t nt0;         // tile rows per matrix = ceil(H / tH)
@@ -135,12 +135,12 @@ struct TiledLaunchKey {
   uint32_t mode;
   uint32_t vec;       // standard and zero jobs: vector width
   uint32_t P;         // standard jobs
-  uint32_t torder;    // standard jobs
   uint32_t lanes;     // standard packed jobs: lanes per unit
+  uint32_t ragged;    // standard jobs: rows are no whole number of vectors
   uint32_t itemsize;  // general jobs
   bool operator==(const TiledLaunchKey& o) const {
-    return mode == o.mode && vec == o.vec && P == o.P && torder == o.torder &&
-           lanes == o.lanes && itemsize == o.itemsize;
+    return mode == o.mode && vec == o.vec && P == o.P &&
+           lanes == o.lanes && ragged == o.ragged && itemsize == o.itemsize;
   }
 };
 

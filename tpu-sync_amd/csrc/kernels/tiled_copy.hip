@@ -44,12 +44,18 @@ __device__ __forceinline__ uint32_t fdiv(const KVX_CONST FastDivU32* f, uint32_t
   return static_cast<uint32_t>((static_cast<uint64_t>(hi) + n) >> f->s);
 }
 
-// V-byte vector type.
+// V-byte vector at any byte address: the rows of a matrix of odd width start
+// anywhere, and gfx950 serves unaligned accesses about as fast as aligned ones
+// (a wave's accesses are contiguous, so only the lines at its ends are shared).
 template <int V> struct VecT;
-template <> struct VecT<16> { typedef u32x4 T; };
-template <> struct VecT<8> { typedef u32x2 T; };
-template <> struct VecT<4> { typedef uint32_t T; };
-template <> struct VecT<2> { typedef uint16_t T; };
+template <> struct VecT<16> {
+  typedef uint32_t T __attribute__((ext_vector_type(4), aligned(1)));
+};
+template <> struct VecT<8> {
+  typedef uint32_t T __attribute__((ext_vector_type(2), aligned(1)));
+};
+template <> struct VecT<4> { typedef uint32_t T __attribute__((aligned(1))); };
+template <> struct VecT<2> { typedef uint16_t T __attribute__((aligned(1))); };
 template <> struct VecT<1> { typedef uint8_t T; };
 
 template <int V>
@@ -61,7 +67,7 @@ __device__ __forceinline__ void st(uint64_t a, typename VecT<V>::T v) {
   __builtin_nontemporal_store(v, (KVX_GLOBAL typename VecT<V>::T*)a);
 }
 
-// 32-bit words of a V-byte vector (V >= 4).
+// 32-bit words of a V-byte vector (one, zero-extended, below 4 bytes).
 template <int V>
 __device__ __forceinline__ void to_words(typename VecT<V>::T v, uint32_t* w) {
   if constexpr (V == 16) {
@@ -80,9 +86,66 @@ __device__ __forceinline__ typename VecT<V>::T from_words(const uint32_t* w) {
   } else if constexpr (V == 8) {
     v.x = w[0]; v.y = w[1];
   } else {
-    v = w[0];
+    v = static_cast<typename VecT<V>::T>(w[0]);
   }
   return v;
+}
+
+// The n words w moved down by `bytes` (< 4 n), zeros coming in at the top.
+template <int n>
+__device__ __forceinline__ void shift_down(uint32_t* w, uint32_t bytes) {
+  const uint32_t sh = bytes * 8;
+  if constexpr (n == 1) {
+    w[0] >>= sh;
+  } else {
+    uint64_t lo = w[0] | (static_cast<uint64_t>(w[1]) << 32);
+    if constexpr (n == 4) {
+      uint64_t hi = w[2] | (static_cast<uint64_t>(w[3]) << 32);
+      if (sh >= 64) {
+        lo = hi >> (sh - 64);
+        hi = 0;
+      } else if (sh > 0) {
+        lo = (lo >> sh) | (hi << (64 - sh));
+        hi >>= sh;
+      }
+      w[2] = static_cast<uint32_t>(hi);
+      w[3] = static_cast<uint32_t>(hi >> 32);
+    } else {
+      lo >>= sh;
+    }
+    w[0] = static_cast<uint32_t>(lo);
+    w[1] = static_cast<uint32_t>(lo >> 32);
+  }
+}
+
+// Stores the first nb (< V) bytes of a vector of V bytes, held in words w.
+template <int V>
+__device__ __forceinline__ void st_head(uint64_t a, uint32_t* w, uint32_t nb) {
+  if constexpr (V == 16) {
+    if (nb & 8) {
+      const uint32_t v[2] = {w[0], w[1]};
+      st<8>(a, from_words<8>(v));
+      a += 8;
+      w[0] = w[2];
+      w[1] = w[3];
+    }
+  }
+  if constexpr (V >= 8) {
+    if (nb & 4) {
+      st<4>(a, w[0]);
+      a += 4;
+      w[0] = w[1];
+    }
+  }
+  uint32_t x = w[0];
+  if constexpr (V >= 4) {
+    if (nb & 2) {
+      st<2>(a, static_cast<uint16_t>(x));
+      a += 2;
+      x >>= 16;
+    }
+  }
+  if (nb & 1) st<1>(a, static_cast<uint8_t>(x));
 }
 
 // Tiled order of P rows of n words each: element c of row k lands at
@@ -127,89 +190,115 @@ __device__ __forceinline__ void deinterleave(const uint32_t (&in)[P * n], uint32
   }
 }
 
-// Addresses of a standard-form unit: the tiled piece, the linear address of
+// A standard-form unit: the address of its tiled piece, the linear address of
 // its first row (row k is k * W * itemsize further), its first row h within
-// the batch matrix and first column c. In tiled order the unit may lie in
-// padding (h >= H or c >= W): the linear address is then clamped to the last
-// row / last column vector of the matrix (the same tile row, so inside the
-// job's range) for callers that load before they test.
-template <int P, bool TORDER>
-__device__ __forceinline__ void unit_addr(const KVX_CONST TiledJobDev* j, uint32_t u,
-                                          uint32_t E, uint32_t unit_bytes, uint64_t* tiled,
-                                          uint64_t* lin, uint32_t* h, uint32_t* c_out) {
+// the batch matrix and first column c. Tiling enumerates units in tiled order,
+// so a unit may lie in padding (h >= H or c >= W); detiling in linear order.
+// The linear address is clamped to the last row and to the last whole vector
+// of a row (the same tile row, so inside the job's range): with RAGGED rows (no
+// whole number of vectors) a unit whose columns run past W starts `back`
+// columns after that address. Whole rows keep a kernel without that handling
+// (one detile of a [14336, 4096] bf16 weight 52.7 us a call, 53.6 with it).
+struct Unit {
+  uint64_t tiled, lin;
+  uint32_t h, c, back;
+};
+
+template <int P, bool TILE, bool RAGGED>
+__device__ __forceinline__ Unit unit_at(const KVX_CONST TiledJobDev* j, uint32_t u, uint32_t E,
+                                        uint32_t unit_bytes) {
   const uint32_t H = j->h32, W = j->w32, sh = j->log2s;
-  uint32_t b, row, c, T, within;
-  if constexpr (TORDER) {
+  Unit x;
+  uint32_t b, hc;
+  if constexpr (TILE) {
     const uint32_t q = fdiv(&j->t_ncv, u);
     const uint32_t cvt = u - q * j->t_ncv.d;
-    T = fdiv(&j->t_gpt, q);
+    const uint32_t T = fdiv(&j->t_gpt, q);
     const uint32_t gi = q - T * j->t_gpt.d;
     const uint32_t btr = fdiv(&j->t_nt1, T);
     const uint32_t tc = T - btr * j->t_nt1.d;
     b = fdiv(&j->t_nt0, btr);
     const uint32_t tr = btr - b * j->t_nt0.d;
-    row = tr * j->th.d + gi * P;
-    c = tc * j->tw.d + cvt * E;
-    *tiled = j->tiled + static_cast<uint64_t>(u) * unit_bytes;
-    const uint32_t rc = row < H ? row : H - 1;
-    const uint32_t cc = c < W ? c : W - E;
-    *lin = j->linear + ((static_cast<uint64_t>(b * H + rc) * W + cc) << sh);
+    x.h = tr * j->th.d + gi * P;
+    x.c = tc * j->tw.d + cvt * E;
+    x.tiled = j->tiled + static_cast<uint64_t>(u) * unit_bytes;
+    hc = x.h < H ? x.h : H - 1;
   } else {
     const uint32_t q = fdiv(&j->ncv, u);
     const uint32_t cv = u - q * j->ncv.d;
     b = fdiv(&j->ng, q);
     const uint32_t g = q - b * j->ng.d;
-    row = g * P;
-    const uint32_t tr = fdiv(&j->th, row);
-    const uint32_t r0 = row - tr * j->th.d;
-    c = cv * E;
-    const uint32_t tc = fdiv(&j->tw, c);
-    const uint32_t cc = c - tc * j->tw.d;
-    T = (b * j->nt0 + tr) * j->nt1 + tc;
-    within = r0 * j->tw.d + cc * P;
-    *tiled = j->tiled + ((static_cast<uint64_t>(T) * j->tile_elems + within) << sh);
-    *lin = j->linear + ((static_cast<uint64_t>(b * H + row) * W + c) << sh);
+    x.h = g * P;
+    const uint32_t tr = fdiv(&j->th, x.h);
+    const uint32_t r0 = x.h - tr * j->th.d;
+    x.c = cv * E;
+    const uint32_t tc = fdiv(&j->tw, x.c);
+    const uint32_t cc = x.c - tc * j->tw.d;
+    const uint32_t T = (b * j->nt0 + tr) * j->nt1 + tc;
+    const uint32_t within = r0 * j->tw.d + cc * P;
+    x.tiled = j->tiled + ((static_cast<uint64_t>(T) * j->tile_elems + within) << sh);
+    hc = x.h;
   }
-  *h = row;
-  *c_out = c;
+  const uint32_t cl = (!TILE && !RAGGED) || x.c < W - E ? x.c : W - E;
+  x.back = RAGGED ? x.c - cl : 0;
+  x.lin = j->linear + ((static_cast<uint64_t>(b * H + hc) * W + cl) << sh);
+  return x;
+}
+
+// Stores a V-byte row vector (words w) of a unit at its first row's linear
+// address `lin` (a further row's: the caller adds it), only the columns
+// before W.
+template <int V, bool RAGGED>
+__device__ __forceinline__ void st_row(const KVX_CONST TiledJobDev* j, const Unit& x,
+                                       uint64_t lin, uint32_t* w) {
+  if (!RAGGED || x.back == 0) {
+    st<V>(lin, from_words<V>(w));
+  } else {
+    const uint32_t sh = j->log2s;
+    st_head<V>(lin + (static_cast<uint64_t>(x.back) << sh), w, (j->w32 - x.c) << sh);
+  }
 }
 
 // Standard form, P = 1: each unit is one V-byte vector on both sides.
-template <int V, bool TILE, bool TORDER>
+template <int V, bool TILE, bool RAGGED>
 __device__ __forceinline__ void std_p1(const KVX_CONST TiledJobDev* j, uint32_t local) {
   constexpr int U = kVecsPerLane;
+  constexpr int n = V >= 4 ? V / 4 : 1;
   const uint32_t E = V >> j->log2s;
   const uint64_t first = j->lo + static_cast<uint64_t>(local) * (kThreads * U);
   const uint64_t end = j->lo + j->count;
   const uint32_t H = j->h32, W = j->w32;
   typename VecT<V>::T r[U];
-  uint64_t dst[U];
-  bool valid[U];
+  Unit x[U];
 #pragma unroll
   for (int i = 0; i < U; ++i) {
     uint64_t u = first + threadIdx.x + i * kThreads;
     u = u < end ? u : end - 1;
-    uint64_t ta, la;
-    uint32_t h, c;
-    unit_addr<1, TORDER>(j, static_cast<uint32_t>(u), E, V, &ta, &la, &h, &c);
-    valid[i] = !TORDER || (h < H && c < W);
-    r[i] = ld<V>(TILE ? la : ta);
-    dst[i] = TILE ? ta : la;
+    x[i] = unit_at<1, TILE, RAGGED>(j, static_cast<uint32_t>(u), E, V);
+    r[i] = ld<V>(TILE ? x[i].lin : x[i].tiled);
   }
 #pragma unroll
   for (int i = 0; i < U; ++i) {
     if (first + threadIdx.x + i * kThreads >= end) continue;
+    uint32_t w[n];
+    to_words<V>(r[i], w);
     if (TILE) {
-      st<V>(dst[i], valid[i] ? r[i] : typename VecT<V>::T{});
-    } else if (valid[i]) {
-      st<V>(dst[i], r[i]);
+      if (x[i].h >= H || x[i].c >= W) {
+#pragma unroll
+        for (int k = 0; k < n; ++k) w[k] = 0;
+      } else if (RAGGED && x[i].back > 0) {
+        shift_down<n>(w, x[i].back << j->log2s);
+      }
+      st<V>(x[i].tiled, from_words<V>(w));
+    } else {
+      st_row<V, RAGGED>(j, x[i], x[i].lin, w);
     }
   }
 }
 
 // Standard form, P = 2 or 4, one lane per unit: P rows x V bytes, P * V
 // bytes of the tiled buffer.
-template <int V, int P, bool TILE, bool TORDER>
+template <int V, int P, bool TILE, bool RAGGED>
 __device__ __forceinline__ void std_packed(const KVX_CONST TiledJobDev* j, uint32_t local) {
   constexpr int U = 128 / (P * V);
   constexpr int n = V / 4;
@@ -219,41 +308,39 @@ __device__ __forceinline__ void std_packed(const KVX_CONST TiledJobDev* j, uint3
   const uint64_t row_bytes = static_cast<uint64_t>(j->w32) << j->log2s;
   const uint32_t H = j->h32, W = j->w32;
   uint32_t words[U][P * n];
-  uint64_t ta[U], la[U];
-  uint32_t h[U], c[U];
+  Unit x[U];
 #pragma unroll
   for (int i = 0; i < U; ++i) {
     uint64_t u = first + threadIdx.x + i * kThreads;
     u = u < end ? u : end - 1;
-    unit_addr<P, TORDER>(j, static_cast<uint32_t>(u), E, P * V, &ta[i], &la[i], &h[i], &c[i]);
-    if (TILE) {
+    x[i] = unit_at<P, TILE, RAGGED>(j, static_cast<uint32_t>(u), E, P * V);
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
       // Rows past the matrix's end read a valid row and are zeroed below.
-#pragma unroll
-      for (int k = 0; k < P; ++k) {
-        const uint32_t kk = h[i] + k < H ? k : 0;
-        to_words<V>(ld<V>(la[i] + kk * row_bytes), &words[i][k * n]);
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < P; ++k) to_words<V>(ld<V>(ta[i] + k * V), &words[i][k * n]);
+      const uint32_t kk = x[i].h + k < H ? k : 0;
+      to_words<V>(ld<V>(TILE ? x[i].lin + kk * row_bytes : x[i].tiled + k * V),
+                  &words[i][k * n]);
     }
   }
 #pragma unroll
   for (int i = 0; i < U; ++i) {
     if (first + threadIdx.x + i * kThreads >= end) continue;
-    const bool col_ok = c[i] < W;
     if (TILE) {
       uint32_t rows[P][n];
 #pragma unroll
       for (int k = 0; k < P; ++k) {
-        const bool valid = col_ok && h[i] + k < H;
+        const bool valid = x[i].c < W && x[i].h + k < H;
 #pragma unroll
         for (int w = 0; w < n; ++w) rows[k][w] = valid ? words[i][k * n + w] : 0u;
+      }
+      if (RAGGED && x[i].c < W && x[i].back > 0) {
+#pragma unroll
+        for (int k = 0; k < P; ++k) shift_down<n>(rows[k], x[i].back << j->log2s);
       }
       uint32_t out[P * n];
       interleave<P, n>(rows, out);
 #pragma unroll
-      for (int k = 0; k < P; ++k) st<V>(ta[i] + k * V, from_words<V>(&out[k * n]));
+      for (int k = 0; k < P; ++k) st<V>(x[i].tiled + k * V, from_words<V>(&out[k * n]));
     } else {
       uint32_t in[P * n];
 #pragma unroll
@@ -262,7 +349,7 @@ __device__ __forceinline__ void std_packed(const KVX_CONST TiledJobDev* j, uint3
       deinterleave<P, n>(in, rows);
 #pragma unroll
       for (int k = 0; k < P; ++k) {
-        if (col_ok && h[i] + k < H) st<V>(la[i] + k * row_bytes, from_words<V>(rows[k]));
+        if (x[i].h + k < H) st_row<V, RAGGED>(j, x[i], x[i].lin + k * row_bytes, rows[k]);
       }
     }
   }
@@ -284,6 +371,7 @@ __device__ __forceinline__ void std_packed(const KVX_CONST TiledJobDev* j, uint3
 // over groups of 8 workgroups (below): 77.3 -> 79.2 % in one process.
 constexpr uint32_t kPairLdsBytes = kVecsPerLane * 2 * (kThreads / 2) * 4 * 4;
 
+template <bool RAGGED>
 __device__ __forceinline__ void std_pair_detile(const KVX_CONST TiledJobDev* j, uint32_t local) {
   constexpr int P = 2;
   constexpr int U = kVecsPerLane;
@@ -317,10 +405,8 @@ __device__ __forceinline__ void std_pair_detile(const KVX_CONST TiledJobDev* j, 
                                  : first + static_cast<uint64_t>(i) * kSlotUnits;
     const uint64_t u0 = base + ut;
     const uint64_t u = u0 < last_unit ? u0 : last_unit;
-    uint64_t ta, la;
-    uint32_t h, c;
-    unit_addr<P, false>(j, static_cast<uint32_t>(u), E, P * 16, &ta, &la, &h, &c);
-    to_words<16>(ld<16>(ta + 16 * k), v[i]);
+    const Unit x = unit_at<P, false, RAGGED>(j, static_cast<uint32_t>(u), E, P * 16);
+    to_words<16>(ld<16>(x.tiled + 16 * k), v[i]);
   }
 #pragma unroll
   for (int i = 0; i < U; ++i) {
@@ -345,10 +431,8 @@ __device__ __forceinline__ void std_pair_detile(const KVX_CONST TiledJobDev* j, 
                                  : first + static_cast<uint64_t>(i) * kSlotUnits;
     const uint64_t u0 = base + ul;
     const uint64_t u = u0 < last_unit ? u0 : last_unit;
-    uint64_t ta, la;
-    uint32_t h, c;
-    unit_addr<P, false>(j, static_cast<uint32_t>(u), E, P * 16, &ta, &la, &h, &c);
-    if (u0 < end && h + r < H) st<16>(la + r * row_bytes, from_words<16>(v[i]));
+    const Unit x = unit_at<P, false, RAGGED>(j, static_cast<uint32_t>(u), E, P * 16);
+    if (u0 < end && x.h + r < H) st_row<16, RAGGED>(j, x, x.lin + r * row_bytes, v[i]);
   }
 }
 
@@ -374,6 +458,7 @@ __device__ __forceinline__ void std_pair_detile(const KVX_CONST TiledJobDev* j, 
 // sliced over groups of 8 workgroups: 74.1 -> 76.8 % in one process.
 constexpr uint32_t kQuadLdsBytes = kVecsPerLane * 4 * kThreads * 4;
 
+template <bool RAGGED>
 __device__ __forceinline__ void std_quad_detile(const KVX_CONST TiledJobDev* j, uint32_t local) {
   constexpr int P = 4;
   constexpr int U = kVecsPerLane;
@@ -408,10 +493,8 @@ __device__ __forceinline__ void std_quad_detile(const KVX_CONST TiledJobDev* j, 
                                  : first + static_cast<uint64_t>(i) * kSlotUnits;
     const uint64_t u0 = base + ut;
     const uint64_t u = u0 < last_unit ? u0 : last_unit;
-    uint64_t ta, la;
-    uint32_t h, c;
-    unit_addr<P, false>(j, static_cast<uint32_t>(u), E, P * 16, &ta, &la, &h, &c);
-    to_words<16>(ld<16>(ta + 16 * k), v[i]);
+    const Unit x = unit_at<P, false, RAGGED>(j, static_cast<uint32_t>(u), E, P * 16);
+    to_words<16>(ld<16>(x.tiled + 16 * k), v[i]);
   }
 #pragma unroll
   for (int i = 0; i < U; ++i) {
@@ -433,10 +516,8 @@ __device__ __forceinline__ void std_quad_detile(const KVX_CONST TiledJobDev* j, 
                                  : first + static_cast<uint64_t>(i) * kSlotUnits;
     const uint64_t u0 = base + ul;
     const uint64_t u = u0 < last_unit ? u0 : last_unit;
-    uint64_t ta, la;
-    uint32_t h, c;
-    unit_addr<P, false>(j, static_cast<uint32_t>(u), E, P * 16, &ta, &la, &h, &c);
-    if (u0 < end && h + r < H) st<16>(la + r * row_bytes, from_words<16>(v[i]));
+    const Unit x = unit_at<P, false, RAGGED>(j, static_cast<uint32_t>(u), E, P * 16);
+    if (u0 < end && x.h + r < H) st_row<16, RAGGED>(j, x, x.lin + r * row_bytes, v[i]);
   }
 }
 
@@ -516,21 +597,21 @@ __device__ __forceinline__ const KVX_CONST TiledJobDev* job_of(const uint8_t* im
 
 // LANES: lanes per unit; 2 for P = 2 and 4 for P = 4 when detiling at 16-byte
 // rows (through LDS), else 1.
-template <int V, int P, bool TILE, bool TORDER, int LANES>
+template <int V, int P, bool TILE, int LANES, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void tiled_std_kernel(const uint8_t* image,
                                                              uint32_t map_offset) {
   uint32_t local;
   const KVX_CONST TiledJobDev* j = job_of(image, map_offset, &local);
   if constexpr (P == 1) {
-    std_p1<V, TILE, TORDER>(j, local);
+    std_p1<V, TILE, RAGGED>(j, local);
   } else if constexpr (LANES == 2) {
-    static_assert(!TILE && !TORDER, "two lanes per unit: detiling in linear order only");
-    std_pair_detile(j, local);
+    static_assert(!TILE, "two lanes per unit: detiling only");
+    std_pair_detile<RAGGED>(j, local);
   } else if constexpr (LANES == 4) {
-    static_assert(!TILE && !TORDER, "four lanes per unit: detiling in linear order only");
-    std_quad_detile(j, local);
+    static_assert(!TILE, "four lanes per unit: detiling only");
+    std_quad_detile<RAGGED>(j, local);
   } else {
-    std_packed<V, P, TILE, TORDER>(j, local);
+    std_packed<V, P, TILE, RAGGED>(j, local);
   }
 }
 
@@ -560,29 +641,31 @@ __global__ __launch_bounds__(kThreads) void tiled_zero_kernel(const uint8_t* ima
 typedef void (*KernelFn)(const uint8_t*, uint32_t);
 
 template <int V, int P, int LANES>
-KernelFn StdKernel(bool tile, bool torder) {
-  if (tile) {
-    return torder ? tiled_std_kernel<V, P, true, true, LANES>
-                  : tiled_std_kernel<V, P, true, false, LANES>;
+KernelFn StdKernel(bool tile, bool ragged) {
+  if (!tile) {
+    return ragged ? tiled_std_kernel<V, P, false, LANES, true>
+                  : tiled_std_kernel<V, P, false, LANES, false>;
   }
-  return torder ? tiled_std_kernel<V, P, false, true, LANES>
-                : tiled_std_kernel<V, P, false, false, LANES>;
+  if constexpr (LANES == 1) {
+    return ragged ? tiled_std_kernel<V, P, true, 1, true> : tiled_std_kernel<V, P, true, 1, false>;
+  }
+  return nullptr;
 }
 
 template <int V>
-KernelFn StdKernelP(int P, bool tile, bool torder, int lanes) {
-  if (P == 1) return StdKernel<V, 1, 1>(tile, torder);
-  if constexpr (V >= 4) {
-    if constexpr (V == 16) {
-      if (lanes == 2 && P == 2 && !tile && !torder) {
-        return tiled_std_kernel<16, 2, false, false, 2>;
-      }
-      if (lanes == 4 && P == 4 && !tile && !torder) {
-        return tiled_std_kernel<16, 4, false, false, 4>;
-      }
-    }
-    if (P == 2) return StdKernel<V, 2, 1>(tile, torder);
-    if (P == 4) return StdKernel<V, 4, 1>(tile, torder);
+KernelFn StdKernelP(const TiledLaunchKey& k) {
+  const bool tile = k.mode == kTileStd, ragged = k.ragged != 0;
+  if (k.P == 1) return StdKernel<V, 1, 1>(tile, ragged);
+  if constexpr (V == 16) {
+    if (k.lanes == 2 && k.P == 2) return StdKernel<16, 2, 2>(tile, ragged);
+    if (k.lanes == 4 && k.P == 4) return StdKernel<16, 4, 4>(tile, ragged);
+  }
+  // One lane per packed unit moves at most 16 bytes of the tiled buffer.
+  if constexpr (V == 4 || V == 8) {
+    if (k.P == 2) return StdKernel<V, 2, 1>(tile, ragged);
+  }
+  if constexpr (V == 4) {
+    if (k.P == 4) return StdKernel<V, 4, 1>(tile, ragged);
   }
   return nullptr;
 }
@@ -608,14 +691,12 @@ KernelFn PickKernel(const TiledLaunchKey& k) {
       default: return nullptr;
     }
   }
-  const bool tile = k.mode == kTileStd;
-  const int lanes = static_cast<int>(k.lanes);
   switch (k.vec) {
-    case 16: return StdKernelP<16>(k.P, tile, k.torder != 0, lanes);
-    case 8: return StdKernelP<8>(k.P, tile, k.torder != 0, lanes);
-    case 4: return StdKernelP<4>(k.P, tile, k.torder != 0, lanes);
-    case 2: return StdKernelP<2>(k.P, tile, k.torder != 0, lanes);
-    case 1: return StdKernelP<1>(k.P, tile, k.torder != 0, lanes);
+    case 16: return StdKernelP<16>(k);
+    case 8: return StdKernelP<8>(k);
+    case 4: return StdKernelP<4>(k);
+    case 2: return StdKernelP<2>(k);
+    case 1: return StdKernelP<1>(k);
     default: return nullptr;
   }
 }
@@ -629,7 +710,7 @@ TiledLaunchKey LaunchKeyOf(const TiledJobDev& j, int vec_bytes) {
   if (j.mode == kDetileStd || j.mode == kTileStd) {
     k.vec = static_cast<uint32_t>(vec_bytes);
     k.P = j.P;
-    k.torder = j.torder;
+    k.ragged = ((static_cast<uint64_t>(j.w32) << j.log2s) % k.vec) != 0 ? 1 : 0;
     k.lanes = j.P == 2 && vec_bytes == 16 && j.lanes_per_unit == 2   ? 2
               : j.P == 4 && vec_bytes == 16 && j.lanes_per_unit == 4 ? 4
                                                                      : 1;
@@ -659,7 +740,7 @@ hipError_t LaunchTiledCopy(const void* image_dev, uint32_t map_offset, uint32_t 
   // points of HBM peak above no cap. The four-lane kernels' own LDS counts
   // towards the reservation.
   const bool quad = (key.mode == kDetileStd || key.mode == kTileStd) && key.lanes == 4;
-  const bool pair = key.mode == kDetileStd && key.lanes == 2 && key.torder == 0;
+  const bool pair = key.mode == kDetileStd && key.lanes == 2;
   const uint32_t lds = kLdsPerCu / kWorkgroupsPerCu - (quad ? kQuadLdsBytes : 0) -
                        (pair ? kPairLdsBytes : 0);
   hipLaunchKernelGGL(fn, dim3(grid), dim3(kThreads), lds, stream, img, map_offset);
