@@ -414,3 +414,52 @@ def test_weight_sync_odd_widths(kvx, oracle, cuda, chunk):
         _, n, off = ws.host_buffer_info(k, 0)
         assert np.array_equal(u8(tensors[k]), oracle.tile(lay, img[off:off + n].copy())), k
     ws.close()
+
+
+@pytest.mark.parametrize("itemsize,P", [(1, 1), (1, 4), (2, 1), (2, 2), (4, 1), (8, 1)])
+def test_column_major_layouts_match_oracle(kvx, oracle, cuda, itemsize, P):
+    """Tiles over the transposed matrix: heights and widths around a region's
+    edge (128 rows, 256 bytes of a row), odd ones, batches, tiles of other
+    sizes, matrices too small for regions (moved element by element), and
+    buffers off by one element."""
+    rng = np.random.default_rng(37)
+    across = 256 // itemsize
+    shapes = [(128, across), (127, across - 1), (129, across + 1), (300, 2 * across + 3),
+              (64, 5 * across), (257, across // 2 + 1), (1, 40), (40, 1), (3, 5), (130, 7)]
+    for k, (H, W) in enumerate(shapes):
+        for tH, tW, batch in ((8, 128, []), (8, 128, [3]), (16, 64, []), (4, 16, [2])):
+            rank = len(batch) + 2
+            mtm = [rank - 2, rank - 1] + list(range(rank - 3, -1, -1))
+            lay = dict(itemsize=itemsize, dims=batch + [H, W], minor_to_major=mtm,
+                       tiles=[[tH, tW]] + ([[P, 1]] if P > 1 else []))
+            print("tiling case", lay, flush=True)
+            check_layout(kvx, oracle, cuda, lay, rng, lin_off=itemsize * (k % 3),
+                         tiled_off=itemsize * (k % 2))
+
+
+@pytest.mark.parametrize("chunk", [2 << 10, 150 << 10, 0])
+def test_weight_sync_column_major(kvx, oracle, cuda, chunk):
+    """Column-major weights through staging chunks below one tile column (cut
+    between elements), of a few tile columns (within and across matrices of
+    a batch), and whole."""
+    rng = np.random.default_rng(chunk + 7)
+    lays = [dict(itemsize=2, dims=[700, 301], minor_to_major=[0, 1], tiles=[[8, 128], [2, 1]]),
+            dict(itemsize=4, dims=[3, 200, 130], minor_to_major=[1, 2, 0], tiles=[[8, 128]])]
+    layouts = [as_layout(kvx, l) for l in lays]
+    tensors = [torch.from_numpy(rng.integers(0, 256, L.tiled_bytes, dtype=np.uint8)).to(cuda)
+               for L in layouts]
+    dev0 = [u8(t) for t in tensors]
+    ws = kvx.WeightSynchronizer([[t] for t in tensors], layouts=[[l] for l in layouts],
+                                chunk_bytes=chunk)
+    ws.d2h().Await()
+    img = ws.host_image()
+    for k, lay in enumerate(lays):
+        _, n, off = ws.host_buffer_info(k, 0)
+        assert np.array_equal(img[off:off + n], oracle.detile(lay, dev0[k])), k
+        img[off:off + n] = rng.integers(0, 256, n, dtype=np.uint8)
+        tensors[k].fill_(0xA5)
+    ws.h2d().Await()
+    for k, lay in enumerate(lays):
+        _, n, off = ws.host_buffer_info(k, 0)
+        assert np.array_equal(u8(tensors[k]), oracle.tile(lay, img[off:off + n].copy())), k
+    ws.close()

@@ -8,12 +8,14 @@
 // the kernel needs; AppendTiledJobs turns a byte range of the tensor's
 // linear image into jobs; LaunchTiledThroughRing uploads and launches them.
 //
-// Two forms, split where the reference splits (IsStandardRowMajorTiled,
+// Three forms, the first split off where the reference splits (IsStandardRowMajorTiled,
 // tiling_utils.cc:56-82):
 //   * standard: row-major dimension order and one 2-D tile (tH, tW), or that
 //     tile followed by a (P, 1) tile with P in {2, 4}, tH % P == 0 and
 //     P * itemsize == 4 (16-bit elements packed in pairs, 8-bit in fours):
 //     vectorised units of P rows;
+//   * transposed: the same tiles with the two minor dimensions swapped (a weight
+//     kept column-major): regions transposed through LDS;
 //   * general: every other tiled layout, element by element through the
 //     nested-tiling index map. The reference's specialised routine assumes
 //     16-bit elements for P = 2 and 8-bit for P = 4 whatever the element type
@@ -56,21 +58,26 @@ struct TiledPlan {
   bool standard = false;  // standard form (else general)
   bool ragged = false;    // standard only since its vectors may start anywhere:
                           // may go general instead (chunks below a tile row)
+  bool column = false;    // transposed form (neither standard nor general)
   bool padded = false;    // tiled elements > logical elements
   int64_t logical_bytes = 0;
   int64_t tiled_bytes = 0;
   int vec = 16;       // widest vector that divides its rows (standard form)
   int zero_vec = 16;  // vector width of the zero pass
-  // Standard form: batch matrices [B][H][W], tiles (tH, tW), P rows per unit.
+  // Standard and transposed form: batch matrices [B][H][W] of the linear image,
+  // tiles (tH, tW) over them or their transposes, P tiled rows per unit.
   uint32_t P = 1;
   uint64_t B = 1, H = 1, W = 1, tH = 1, tW = 1, nT0 = 1, nT1 = 1;
   // General form: the final tiled shape's dimensions.
   std::vector<TiledGenDim> gen;
   // Largest byte offset <= x (from the start of the linear image) at which
   // the linear image may be cut between two launches: whole tile rows (tH
-  // rows, or the end of a batch matrix) in the standard form, whole elements
-  // in the general form.
+  // rows, or the end of a batch matrix) in the standard form, whole tile
+  // columns (tW rows) in the transposed form, whole elements in the general
+  // form.
   int64_t CutAtOrBelow(int64_t x) const;
+  // Linear rows between two cuts (standard and transposed form).
+  uint64_t CutRows() const { return column ? tW : tH; }
 };
 
 StatusOr<TiledPlan> PlanTiled(const TiledLayout& l);
@@ -79,6 +86,7 @@ StatusOr<TiledPlan> PlanTiled(const TiledLayout& l);
 struct TiledJob {
   TiledJobDev dev{};
   int vec = 0;
+  int64_t bytes = 0;  // linear bytes the job moves (a standard job's last units whole)
   std::vector<TiledGenDim> gen;
 };
 

@@ -90,13 +90,13 @@ Status WeightSynchronizer::Init() {
   // A chunk must hold one tile row of every tiled tensor.
   for (int64_t k = 0; k < n; ++k) {
     const TiledPlan* tp = plan(k);
-    if (tp == nullptr || !tp->standard) continue;
+    if (tp == nullptr || (!tp->standard && !tp->column)) continue;
     const int64_t group =
-        static_cast<int64_t>(std::min(tp->tH, tp->H) * tp->W) * tp->layout.itemsize;
-    if (group > chunk && tp->ragged) {
+        static_cast<int64_t>(std::min(tp->CutRows(), tp->H) * tp->W) * tp->layout.itemsize;
+    if (group > chunk && (tp->ragged || tp->column)) {
       // The general form: chunks may be cut between any two elements.
       auto general = std::make_shared<TiledPlan>(*tp);
-      general->standard = false;
+      general->standard = general->column = false;
       cfg_.tiled[k] = general;
       continue;
     }
@@ -215,11 +215,7 @@ Status WeightSynchronizer::Launch(const std::vector<StridedCopy>& copies,
     if (start != nullptr) KVX_HIP_RETURN_IF_ERROR(hipEventRecord(start, stream));
     KVX_HIP_RETURN_IF_ERROR(hipEventRecord(s.stop, stream));
     for (const StridedCopy& c : copies) s.bytes += c.size * (c.count > 0 ? c.count : 1);
-    for (const TiledJob& j : tiled) {
-      const bool std_form = j.dev.mode == kDetileStd || j.dev.mode == kTileStd;
-      s.bytes += static_cast<int64_t>(j.dev.count) *
-                 (std_form ? static_cast<int64_t>(j.dev.P) * j.vec : j.dev.itemsize);
-    }
+    for (const TiledJob& j : tiled) s.bytes += j.bytes;
     s.pack = pack;
     samples_.push_back(s);
   }

@@ -9,7 +9,7 @@
 //
 // "Detile" copies a tiled buffer into the row-major (linear) byte image of
 // the tensor, "tile" the reverse. One launch runs any number of jobs; a job
-// is a range of one tensor in one of five modes:
+// is a range of one tensor in one of seven modes:
 //   * kDetileStd / kTileStd: the standard form (row-major dimension order and
 //     one 2-D tile (tH, tW), optionally followed by a (P, 1) tile that packs
 //     P consecutive rows element by element, P in {2, 4} with P * itemsize =
@@ -21,6 +21,11 @@
 //     image, then column vectors), tiling in tiled order (unit u is bytes
 //     [u P V, (u + 1) P V) of the tiled buffer, padding included: rows past H
 //     and columns past W read as zero).
+//   * kDetileCol / kTileCol: the same tiles over the transposed matrix (the two
+//     minor dimensions swapped: linear columns are rows of the tiled matrix).
+//     A workgroup moves a region of 128 linear rows x 256 bytes, transposed
+//     through LDS in atoms of P elements (P * itemsize bytes, contiguous on
+//     both sides), so that both sides are read and written in 16-byte vectors.
 //   * kDetileGen / kTileGen: any other layout, element by element through the
 //     index map of the nested tiling.
 //   * kZero: clears a tiled buffer (V-byte vectors), launched before a
@@ -70,7 +75,13 @@ enum TiledMode : uint32_t {
   kZero = 2,
   kDetileGen = 3,
   kTileGen = 4,
+  kDetileCol = 5,
+  kTileCol = 6,
 };
+
+// A region of a transposed job: linear rows x bytes of each.
+constexpr uint32_t kColRows = 128;
+constexpr uint32_t kColBytes = 256;
 
 constexpr int kTiledMaxRank = 8;     // logical dimensions (general path)
 constexpr int kTiledMaxGenDims = 16; // dimensions of the final tiled shape
@@ -96,7 +107,7 @@ struct TiledJobDev {
   uint64_t tiled;   // tiled buffer of the tensor
   uint64_t linear;  // linear image of the tensor (byte 0 = element 0)
   uint64_t lo;      // first unit (std), element (gen) or vector (zero)
-  uint64_t count;   // units / elements / vectors
+  uint64_t count;   // units / elements / vectors / regions (transposed)
   uint32_t mode;    // TiledMode
   uint32_t wg_begin;
   uint32_t P;        // std: rows per unit (1, 2 or 4)
@@ -113,14 +124,19 @@ struct TiledJobDev {
   FastDivU32 t_nt0;  // tile rows per matrix (nT0)
   uint32_t lanes_per_unit;  // packed units: 1, or 2 (P = 2) / 4 (P = 4) detiling at 16-byte rows
   uint32_t sliced;  // detiling with 2 or 4 lanes per unit: slots in whole groups go sliced
-  uint32_t pad0[2];
+  uint32_t b0;     // transposed: first batch matrix
+  uint32_t c_lo;   // transposed: first linear row of a matrix
   uint32_t h32;         // H (rows per batch matrix)
   uint32_t w32;         // W (columns)
   uint32_t nt0;         // tile rows per matrix = ceil(H / tH)
   uint32_t nt1;         // tile columns per matrix = ceil(W / tW)
   uint32_t tile_elems;  // tH * tW
   uint32_t log2s;       // log2(itemsize)
-  uint32_t pad1[2];
+  // Transposed: linear rows [c_lo, c_hi) hold data, [c_hi, c_end) padding;
+  // ncv = regions across them, ng = regions across a row; h32 and w32 stay
+  // the linear matrix's, nt0 = ceil(W / tH), nt1 = ceil(H / tW).
+  uint32_t c_hi;
+  uint32_t c_end;
   // General form.
   uint32_t rank;        // logical dimensions
   uint32_t ngen;        // dimensions of the final tiled shape
@@ -133,7 +149,7 @@ static_assert(sizeof(TiledJobDev) % 16 == 0, "device layout");
 // What selects a kernel: every job of one launch shares it.
 struct TiledLaunchKey {
   uint32_t mode;
-  uint32_t vec;       // standard and zero jobs: vector width
+  uint32_t vec;       // standard and zero jobs: vector width; transposed: atom bytes
   uint32_t P;         // standard jobs
   uint32_t lanes;     // standard packed jobs: lanes per unit
   uint32_t ragged;    // standard jobs: rows are no whole number of vectors
@@ -147,7 +163,8 @@ struct TiledLaunchKey {
 // The key of a job whose launch uses vector width vec_bytes.
 TiledLaunchKey LaunchKeyOf(const TiledJobDev& j, int vec_bytes);
 
-// Units (std), elements (gen) or vectors (zero) one workgroup moves.
+// Units (std), elements (gen), vectors (zero) or regions (transposed) one
+// workgroup moves.
 uint32_t TiledPerWorkgroup(const TiledLaunchKey& k);
 
 // Launches the jobs of a device-resident image: the TiledJobDev array, the
