@@ -269,3 +269,64 @@ def test_fp8_llama3_8b_pool_full_size_round_trip(kvx, cuda):
         got = t.index_select(0, dst_t)
         assert torch.equal(got.view(torch.uint8), saved[k].view(torch.uint8)), k
     mgr.close()
+
+
+# Block bytes around a vector, a lane's share, the whole-block limit (8 KiB)
+# and a workgroup's pass (32 KiB), with side tables of other sizes.
+ANY_SIZES = [(1, 4), (3, 1), (7, 8), (15, 4), (16, 4), (17, 32), (33, 4), (255, 2), (1000, 4),
+             (2048, 4), (2560, 12), (4095, 4), (4097, 32), (8190, 4), (8192, 4), (8193, 20),
+             (10250, 4), (32768, 4), (32769, 4), (40001, 6), (65551, 32)]
+
+
+@pytest.mark.parametrize("block,side", ANY_SIZES, ids=[f"{b}+{s}" for b, s in ANY_SIZES])
+def test_gather_scatter_of_any_block_size(kvx, cuda, block, side):
+    """Payload and side table of any size in one launch, each at its own vector
+    width: a block that is no whole number of vectors ends with one stepped
+    back, and no byte of another block changes. Storages start at odd
+    addresses; layer-major with the side table, block-major without."""
+    rng = np.random.default_rng(block)
+    layers, blocks, n = 3, 40, 29
+    pool_np = rng.integers(0, 256, 2 * layers * blocks * block + 1, dtype=np.uint8)
+    side_np = rng.integers(0, 256, layers * blocks * side + 1, dtype=np.uint8)
+    ids = rng.permutation(blocks)[:n].tolist()
+
+    def storages(buf, count, size):
+        return [buf[1 + k * blocks * size:1 + (k + 1) * blocks * size].reshape(blocks, size)
+                for k in range(count)]
+
+    for tables in (True, False):
+        pool, tab = torch.from_numpy(pool_np.copy()).to(cuda), torch.from_numpy(side_np.copy()).to(cuda)
+        mgr = kvx.KVCacheManager(storages(pool, 2 * layers, block), host_blocks_to_allocate=1,
+                                 scale_tables=storages(tab, layers, side) if tables else None)
+        rows = storages(pool_np, 2 * layers, block)
+        if tables:
+            parts = [r[ids].reshape(-1) for r in rows]
+            parts += [r[ids].reshape(-1) for r in storages(side_np, layers, side)]
+            want = np.concatenate(parts)
+        else:
+            want = np.stack([r[ids] for r in rows], axis=1).reshape(-1)
+        room = torch.full((want.size + 34,), 0xA5, dtype=torch.uint8, device=cuda)
+        staging = room[1:1 + want.size]
+        mgr.gather(ids, staging, block_major=not tables).Await()
+        got = room.cpu().numpy()
+        assert np.array_equal(got[1:1 + want.size], want)
+        assert got[0] == 0xA5 and (got[1 + want.size:] == 0xA5).all()
+        # New bytes back into other blocks; every other byte stays.
+        new = rng.integers(0, 256, want.size, dtype=np.uint8)
+        dst = rng.permutation(blocks)[:n].tolist()
+        staging.copy_(torch.from_numpy(new).to(cuda))
+        mgr.scatter(dst, staging, block_major=not tables).Await()
+        want_pool, want_tab = pool_np.copy(), side_np.copy()
+        if tables:
+            cut = 2 * layers * n * block
+            for r, x in zip(storages(want_pool, 2 * layers, block),
+                            new[:cut].reshape(2 * layers, n, block)):
+                r[dst] = x
+            for r, x in zip(storages(want_tab, layers, side), new[cut:].reshape(layers, n, side)):
+                r[dst] = x
+        else:
+            for w, r in enumerate(storages(want_pool, 2 * layers, block)):
+                r[dst] = new.reshape(n, 2 * layers, block)[:, w]
+        assert np.array_equal(pool.cpu().numpy(), want_pool)
+        assert np.array_equal(tab.cpu().numpy(), want_tab)
+        mgr.close()

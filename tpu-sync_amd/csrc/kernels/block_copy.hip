@@ -6,9 +6,16 @@
 // stores, which is what saturates HBM on a streaming copy. The block id and
 // the storage base are workgroup-uniform, so the compiler reads them with
 // scalar loads into SGPRs: the id table is read once per block, broadcast
-// through SGPRs instead of an LDS round trip and barrier. Small blocks (side
-// tables such as per-head fp8 scales) are packed many to a workgroup so that
-// every lane still moves one vector.
+// through SGPRs instead of an LDS round trip and barrier. Smaller blocks (one
+// KV head of a tensor-parallel rank, side tables such as per-head fp8 scales)
+// are packed many to a workgroup, every lane with up to 8 vectors in flight.
+//
+// Between device buffers every piece takes the widest vectors its blocks hold
+// (16 bytes, or what a smaller block allows) at any address: gfx950 serves
+// unaligned accesses about as fast as aligned ones. A block that is no whole
+// number of vectors ends with one stepped back to its last byte, which
+// rewrites a few bytes with the same values. Launches with host memory on one
+// side take one aligned width for all pieces.
 //
 // Loads and stores are non-temporal: a gathered block is read once and the
 // staging copy is next read by the DMA engine, so neither should displace
@@ -26,12 +33,23 @@ namespace kvx {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kUnroll = 8;  // vectors a lane has in flight
 // Blocks per workgroup on the small-block path: the LDS address table holds
 // 16 bytes per block (4 KiB, which leaves the occupancy of 8 workgroups per
 // CU untouched).
 constexpr uint32_t kSmallMaxBlocks = 256;
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// A vector of V bytes at any byte address.
+template <int V> struct VecT;
+template <> struct VecT<16> {
+  typedef uint32_t T __attribute__((ext_vector_type(4), aligned(1)));
+};
+template <> struct VecT<8> {
+  typedef uint32_t T __attribute__((ext_vector_type(2), aligned(1)));
+};
+template <> struct VecT<4> { typedef uint32_t T __attribute__((aligned(1))); };
+template <> struct VecT<2> { typedef uint16_t T __attribute__((aligned(1))); };
+template <> struct VecT<1> { typedef uint8_t T; };
 
 // Explicit address spaces: data goes through global_load/global_store (not
 // flat), and workgroup-uniform table reads through the constant address
@@ -57,9 +75,14 @@ struct KPiece {
   int64_t stride_i;
   int64_t pool_blocks;
   int64_t other_blocks;
+  uint64_t bytes;     // bytes per block
+  uint64_t magic;     // small blocks: floor(2^32 / elems) + 1
   uint32_t f0;
   uint32_t nblocks;
-  uint32_t elems;     // vectors per block
+  uint32_t vec;       // vector bytes
+  uint32_t elems;     // vectors per block: small blocks with the last, partial
+                      // one; whole blocks without it
+  uint32_t rest;      // bytes past a block's whole vectors
   uint32_t bpw;       // blocks per workgroup
   uint32_t wg_begin;  // first workgroup of the piece
   uint32_t whole;     // 1: every lane works on one block at a time
@@ -74,46 +97,47 @@ struct KParams {
   int32_t npieces;
 };
 
-template <typename V>
-__device__ __forceinline__ V ld_nt(const KVX_GLOBAL V* p) {
-  return __builtin_nontemporal_load(p);
+template <int V>
+__device__ __forceinline__ typename VecT<V>::T ld(uint64_t base, uint64_t off) {
+  return __builtin_nontemporal_load(
+      (const KVX_GLOBAL typename VecT<V>::T*)(gptr<const uint8_t>(base) + off));
 }
 
-template <typename V>
-__device__ __forceinline__ void st_nt(V v, KVX_GLOBAL V* p) {
-  __builtin_nontemporal_store(v, p);
+template <int V>
+__device__ __forceinline__ void st(typename VecT<V>::T v, uint64_t base, uint64_t off) {
+  __builtin_nontemporal_store(v, (KVX_GLOBAL typename VecT<V>::T*)(gptr<uint8_t>(base) + off));
 }
 
-// Whole-block copy by all lanes of the workgroup.
-template <typename V, int kUnroll>
-__device__ __forceinline__ void copy_whole_block(const KVX_GLOBAL V* __restrict__ src,
-                                                 KVX_GLOBAL V* __restrict__ dst,
-                                                 uint32_t elems) {
+// Copy of `elems` vectors by all lanes of the workgroup.
+template <int V>
+__device__ __forceinline__ void copy_whole_block(uint64_t src, uint64_t dst, uint32_t elems) {
+  typedef typename VecT<V>::T T;
   uint32_t k = threadIdx.x;
+  auto at = [](uint32_t i) { return static_cast<uint64_t>(i) * V; };
   for (; k + (kUnroll - 1) * kThreads < elems; k += kUnroll * kThreads) {
-    V r[kUnroll];
+    T r[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) r[u] = ld_nt(src + k + u * kThreads);
+    for (int u = 0; u < kUnroll; ++u) r[u] = ld<V>(src, at(k + u * kThreads));
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) st_nt(r[u], dst + k + u * kThreads);
+    for (int u = 0; u < kUnroll; ++u) st<V>(r[u], dst, at(k + u * kThreads));
   }
   // The tail (all of a 16 KiB block) still keeps 4, then 2 loads in flight.
   if (k + 3 * kThreads < elems) {
-    V r[4];
+    T r[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) r[u] = ld_nt(src + k + u * kThreads);
+    for (int u = 0; u < 4; ++u) r[u] = ld<V>(src, at(k + u * kThreads));
 #pragma unroll
-    for (int u = 0; u < 4; ++u) st_nt(r[u], dst + k + u * kThreads);
+    for (int u = 0; u < 4; ++u) st<V>(r[u], dst, at(k + u * kThreads));
     k += 4 * kThreads;
   }
   if (k + kThreads < elems) {
-    const V r0 = ld_nt(src + k);
-    const V r1 = ld_nt(src + k + kThreads);
-    st_nt(r0, dst + k);
-    st_nt(r1, dst + k + kThreads);
+    const T r0 = ld<V>(src, at(k));
+    const T r1 = ld<V>(src, at(k + kThreads));
+    st<V>(r0, dst, at(k));
+    st<V>(r1, dst, at(k + kThreads));
     k += 2 * kThreads;
   }
-  if (k < elems) st_nt(ld_nt(src + k), dst + k);
+  if (k < elems) st<V>(ld<V>(src, at(k)), dst, at(k));
 }
 
 __device__ __forceinline__ KPiece select_piece(const KParams& P, uint32_t wg) {
@@ -131,14 +155,56 @@ __device__ __forceinline__ bool bad_id(int64_t id, int64_t limit) {
   return static_cast<uint64_t>(id) >= static_cast<uint64_t>(limit);
 }
 
-// Many small blocks per workgroup (side tables such as fp8 scales). The
-// workgroup first resolves its blocks -- id, table entries, bounds check --
-// with one pass of independent, coalesced loads, one block per lane, and
-// stages each block's source and destination address in LDS (0 for a bad
-// id). Then lane e moves vector (e % elems) of block (e / elems) with both
-// addresses read from LDS, so no lane waits on a chain of dependent table
-// loads before its data load. b0: the workgroup's first block of the piece.
-template <typename V, bool kGather>
+// Up to kSteps vectors a lane of the workgroup's small blocks, every load
+// issued before the first store. Lane e moves vector (e % elems) of block
+// (e / elems), its last one stepped back to the block's end; lanes past the
+// end re-read the last vector and store nothing.
+template <int V, int kSteps>
+__device__ __forceinline__ void move_small(const uint64_t* s_src, const uint64_t* s_dst,
+                                           uint32_t total, uint32_t elems, uint64_t magic,
+                                           uint64_t bytes) {
+  typename VecT<V>::T r[kSteps];
+  uint64_t dst[kSteps];
+#pragma unroll
+  for (int u = 0; u < kSteps; ++u) {
+    uint32_t e = threadIdx.x + u * kThreads;
+    const bool in = e < total;
+    e = in ? e : total - 1;
+    const uint32_t b = static_cast<uint32_t>((e * magic) >> 32);
+    const uint32_t sub = e - b * elems;
+    const uint64_t off = sub + 1 < elems ? static_cast<uint64_t>(sub) * V : bytes - V;
+    r[u] = ld<V>(s_src[b], off);
+    const uint64_t d = s_dst[b];
+    dst[u] = in && d != 0 ? d + off : 0;
+  }
+#pragma unroll
+  for (int u = 0; u < kSteps; ++u) {
+    if (dst[u] != 0) st<V>(r[u], dst[u], 0);
+  }
+}
+
+template <int V>
+__device__ __forceinline__ void move_small_blocks(const uint64_t* s_src, const uint64_t* s_dst,
+                                                  uint32_t total, const KPiece& p) {
+  if (total > 4 * kThreads) {
+    move_small<V, 8>(s_src, s_dst, total, p.elems, p.magic, p.bytes);
+  } else if (total > kThreads) {
+    move_small<V, 4>(s_src, s_dst, total, p.elems, p.magic, p.bytes);
+  } else {
+    move_small<V, 1>(s_src, s_dst, total, p.elems, p.magic, p.bytes);
+  }
+}
+
+// Many small blocks per workgroup. The workgroup first resolves its blocks --
+// id, table entries, bounds check -- with one pass of independent, coalesced
+// loads, one block per lane, and stages each block's source and destination
+// address in LDS, so that no lane waits on a chain of dependent table loads
+// before its data loads. A bad id gets no destination and a source that can
+// be read. b0: the workgroup's first block of the piece. Bound by HBM: 768 random
+// 4 KiB blocks of 160 storages gathered in 177 us (5.7 TB/s; 242 with one
+// vector in flight a lane), 2 KiB blocks with a 4-byte scale per (layer, block)
+// scattered in 95 us (114 at the scales' 4-byte vectors for the whole launch).
+template <bool kGather>
 __device__ __forceinline__ void copy_small_blocks(const KPiece& p, const int64_t* ids,
                                                   const int64_t* ids2, int32_t* error,
                                                   uint32_t n, uint32_t b0) {
@@ -146,7 +212,6 @@ __device__ __forceinline__ void copy_small_blocks(const KPiece& p, const int64_t
   __shared__ uint64_t s_dst[kSmallMaxBlocks];
   const uint32_t left = p.nblocks - b0;
   const uint32_t nb = left < p.bpw ? left : p.bpw;
-  const uint64_t block_bytes = static_cast<uint64_t>(p.elems) * sizeof(V);
   for (uint32_t b = threadIdx.x; b < nb; b += kThreads) {
     const uint32_t f = p.f0 + b0 + b;
     const uint32_t w = f / n;
@@ -158,29 +223,30 @@ __device__ __forceinline__ void copy_small_blocks(const KPiece& p, const int64_t
     if (p.others != 0) {
       const int64_t id2 = gptr<const int64_t>(reinterpret_cast<uint64_t>(ids2))[i];
       const uint64_t obase = gptr<const uint64_t>(p.others)[w];
-      bad = bad || bad_id(id2, p.other_blocks);
-      other = obase + static_cast<uint64_t>(id2) * block_bytes;
+      const bool bad2 = bad_id(id2, p.other_blocks);
+      bad = bad || bad2;
+      other = obase + static_cast<uint64_t>(bad2 ? 0 : id2) * p.bytes;
     } else {
       other = p.staging + w * static_cast<uint64_t>(p.stride_w) +
               i * static_cast<uint64_t>(p.stride_i);
     }
-    const uint64_t pool = base + static_cast<uint64_t>(id) * block_bytes;
+    const uint64_t pool = base + static_cast<uint64_t>(id) * p.bytes;
     if (bad && error != nullptr) atomicOr(error, 1);
-    s_src[b] = bad ? 0 : (kGather ? pool : other);
+    s_src[b] = bad || !kGather ? other : pool;
     s_dst[b] = bad ? 0 : (kGather ? other : pool);
   }
   __syncthreads();
   const uint32_t total = nb * p.elems;
-  for (uint32_t e = threadIdx.x; e < total; e += kThreads) {
-    const uint32_t b = e / p.elems;
-    const uint32_t sub = e - b * p.elems;
-    const uint64_t src = s_src[b];
-    if (src == 0) continue;
-    st_nt(ld_nt(gptr<const V>(src) + sub), gptr<V>(s_dst[b]) + sub);
+  switch (p.vec) {
+    case 16: move_small_blocks<16>(s_src, s_dst, total, p); break;
+    case 8: move_small_blocks<8>(s_src, s_dst, total, p); break;
+    case 4: move_small_blocks<4>(s_src, s_dst, total, p); break;
+    case 2: move_small_blocks<2>(s_src, s_dst, total, p); break;
+    default: move_small_blocks<1>(s_src, s_dst, total, p); break;
   }
 }
 
-template <typename V, bool kGather, int kUnroll>
+template <int V, bool kGather>
 __global__ __launch_bounds__(kThreads) void block_copy_kernel(KParams P) {
   const uint32_t wg = blockIdx.x;
   const KPiece p = select_piece(P, wg);
@@ -202,8 +268,7 @@ __global__ __launch_bounds__(kThreads) void block_copy_kernel(KParams P) {
       if (p.others != 0) {
         const int64_t id2 = uniform_load<int64_t>(reinterpret_cast<uint64_t>(P.ids2), i);
         bad = bad || bad_id(id2, p.other_blocks);
-        other = uniform_load<uint64_t>(p.others, w) +
-                static_cast<uint64_t>(id2) * p.elems * sizeof(V);
+        other = uniform_load<uint64_t>(p.others, w) + static_cast<uint64_t>(id2) * p.bytes;
       } else {
         other = p.staging + w * static_cast<uint64_t>(p.stride_w) +
                 i * static_cast<uint64_t>(p.stride_i);
@@ -213,18 +278,18 @@ __global__ __launch_bounds__(kThreads) void block_copy_kernel(KParams P) {
         continue;
       }
       const uint64_t base = uniform_load<uint64_t>(p.storages, w);
-      KVX_GLOBAL V* pool = gptr<V>(base) + static_cast<uint64_t>(id) * p.elems;
-      KVX_GLOBAL V* stg = gptr<V>(other);
-      if (kGather) {
-        copy_whole_block<V, kUnroll>(pool, stg, p.elems);
-      } else {
-        copy_whole_block<V, kUnroll>(stg, pool, p.elems);
+      const uint64_t pool = base + static_cast<uint64_t>(id) * p.bytes;
+      const uint64_t src = kGather ? pool : other;
+      const uint64_t dst = kGather ? other : pool;
+      copy_whole_block<V>(src, dst, p.elems);
+      if (p.rest != 0 && threadIdx.x == 0) {
+        st<V>(ld<V>(src, p.bytes - V), dst, p.bytes - V);
       }
     }
     return;
   }
 
-  copy_small_blocks<V, kGather>(p, P.ids, P.ids2, P.error, n, b0);
+  copy_small_blocks<kGather>(p, P.ids, P.ids2, P.error, n, b0);
 }
 
 // The common launch (one piece of large blocks, no second paged side, one
@@ -246,9 +311,11 @@ struct FastParams {
   int64_t stride_w;
   int64_t stride_i;
   int64_t pool_blocks;
+  uint64_t bytes;      // bytes per block
   uint32_t f0;
   uint32_t n;
-  uint32_t elems;
+  uint32_t elems;      // whole vectors per block
+  uint32_t rest;       // bytes past them
   uint32_t wstorages;  // whole-storage orders: storages in the launch
   uint32_t w0;         // whole-storage orders: first storage (f0 = w0 * n)
   uint32_t pieces;     // workgroups per block (1, or blocks above kUnroll * kThreads vectors)
@@ -260,8 +327,9 @@ enum FastOrder : int { kStorageMajor = 0, kStoragePairs = 1, kAllStorages = 2 };
 // Workgroup g of a fast launch: one whole block, or with pieces > 1 one
 // piece of piece_elems vectors of a block, the pieces of a block on
 // consecutive workgroups (so a large block's writes are in flight together).
-template <typename V, bool kGather, int kUnroll, int kOrder>
+template <bool kGather, int kOrder>
 __device__ __forceinline__ void fast_block(const FastParams& P, uint32_t g) {
+  constexpr int V = 16;
   uint32_t piece = 0;
   if (P.pieces > 1) {
     const uint32_t b = g / P.pieces;
@@ -295,21 +363,22 @@ __device__ __forceinline__ void fast_block(const FastParams& P, uint32_t g) {
   const uint32_t left = P.elems - first;
   const uint32_t span = P.pieces > 1 && left > P.piece_elems ? P.piece_elems : left;
   const uint32_t elems = bad ? 0u : span;
-  KVX_GLOBAL V* pool =
-      gptr<V>(base) + static_cast<uint64_t>(bad ? 0 : id) * P.elems + first;
-  KVX_GLOBAL V* stg = gptr<V>(P.staging + w * static_cast<uint64_t>(P.stride_w) +
-                              i * static_cast<uint64_t>(P.stride_i)) + first;
-  if (kGather) {
-    copy_whole_block<V, kUnroll>(pool, stg, elems);
-  } else {
-    copy_whole_block<V, kUnroll>(stg, pool, elems);
+  const uint64_t pool = base + static_cast<uint64_t>(bad ? 0 : id) * P.bytes;
+  const uint64_t stg = P.staging + w * static_cast<uint64_t>(P.stride_w) +
+                       i * static_cast<uint64_t>(P.stride_i);
+  const uint64_t src = kGather ? pool : stg;
+  const uint64_t dst = kGather ? stg : pool;
+  const uint64_t off = static_cast<uint64_t>(first) * V;
+  copy_whole_block<V>(src + off, dst + off, elems);
+  if (P.rest != 0 && !bad && piece + 1 == P.pieces && threadIdx.x == 0) {
+    st<V>(ld<V>(src, P.bytes - V), dst, P.bytes - V);
   }
   if (bad && threadIdx.x == 0 && P.error != nullptr) atomicOr(P.error, 1);
 }
 
-template <typename V, bool kGather, int kUnroll, int kOrder>
+template <bool kGather, int kOrder>
 __global__ __launch_bounds__(kThreads) void block_copy_fast_kernel(FastParams P) {
-  fast_block<V, kGather, kUnroll, kOrder>(P, blockIdx.x);
+  fast_block<kGather, kOrder>(P, blockIdx.x);
 }
 
 // Sliced form of the fast gather, for blocks of exactly one pass (kUnroll *
@@ -324,8 +393,9 @@ __global__ __launch_bounds__(kThreads) void block_copy_fast_kernel(FastParams P)
 // +2.2 points of HBM bandwidth (e.g. 75.2 against 73.9 %). The same form for
 // the scatter (8 slices, all-storages order) measured -1.5 to +1.7 points
 // and is not used.
-template <typename V, int kUnroll, int kLog2H>
+template <int kLog2H>
 __global__ __launch_bounds__(kThreads) void block_copy_sliced_gather_kernel(FastParams P) {
+  constexpr int V = 16;
   constexpr uint32_t kH = 1u << kLog2H;
   constexpr uint32_t kSlice = kUnroll * kThreads / kH;  // vectors per slice
   // Each unrolled step's kThreads vectors lie in one slice of one block, so
@@ -355,7 +425,7 @@ __global__ __launch_bounds__(kThreads) void block_copy_sliced_gather_kernel(Fast
     const bool bad = in && bad_id(id, P.pool_blocks);
     ok[r] = in && !bad;
     bad_any |= bad;
-    pool_at[r] = base + static_cast<uint64_t>(ok[r] ? id : 0) * P.elems * sizeof(V);
+    pool_at[r] = base + static_cast<uint64_t>(ok[r] ? id : 0) * P.bytes;
     stg_at[r] = stg0 + i * static_cast<uint64_t>(P.stride_i);
   }
   bool all_ok = true;
@@ -364,18 +434,18 @@ __global__ __launch_bounds__(kThreads) void block_copy_sliced_gather_kernel(Fast
   const uint32_t lane0 = cc * kSlice + threadIdx.x;
   if (all_ok) {
     // Every step's load issued before the first store, as in the fast kernel.
-    V v[kUnroll];
+    typename VecT<V>::T v[kUnroll];
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       const uint32_t r = u / kSteps;
       const uint32_t k = lane0 + (u % kSteps) * kThreads;
-      v[u] = ld_nt(gptr<V>(pool_at[r]) + k);
+      v[u] = ld<V>(pool_at[r], k * V);
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       const uint32_t r = u / kSteps;
       const uint32_t k = lane0 + (u % kSteps) * kThreads;
-      st_nt(v[u], gptr<V>(stg_at[r]) + k);
+      st<V>(v[u], stg_at[r], k * V);
     }
     return;
   }
@@ -384,21 +454,20 @@ __global__ __launch_bounds__(kThreads) void block_copy_sliced_gather_kernel(Fast
     if (!ok[r]) continue;
     for (uint32_t t = 0; t < kSteps; ++t) {
       const uint32_t k = lane0 + t * kThreads;
-      st_nt(ld_nt(gptr<V>(pool_at[r]) + k), gptr<V>(stg_at[r]) + k);
+      st<V>(ld<V>(pool_at[r], k * V), stg_at[r], k * V);
     }
   }
   if (bad_any && threadIdx.x == 0 && P.error != nullptr) atomicOr(P.error, 1);
 }
 
 // Slices per block (log2) of a sliced gather, 0 when the launch goes to the
-// fast kernel: 16-byte vectors, blocks of exactly one pass, an even number of
-// whole storages (the pairs order), an uncapped grid that fits.
+// fast kernel: blocks of exactly one pass, an even number of whole storages
+// (the pairs order), an uncapped grid that fits.
 constexpr int kGatherLog2Slices = 2;
-int SlicedGatherLog2(const FastParams& F, CopyDir dir, int order, int vec_bytes, int unroll,
-                     bool capped_grid) {
+int SlicedGatherLog2(const FastParams& F, CopyDir dir, int order, bool capped_grid) {
   if (dir != CopyDir::kGather || order != kStoragePairs) return 0;
-  if (vec_bytes != 16 || capped_grid || F.pieces != 1) return 0;
-  if (F.elems != static_cast<uint32_t>(unroll * kThreads)) return 0;
+  if (capped_grid || F.pieces != 1 || F.rest != 0) return 0;
+  if (F.elems != static_cast<uint32_t>(kUnroll * kThreads)) return 0;
   const uint64_t groups =
       (static_cast<uint64_t>(F.n) + (1u << kGatherLog2Slices) - 1) >> kGatherLog2Slices;
   if ((groups << kGatherLog2Slices) * F.wstorages > INT32_MAX) return 0;
@@ -409,14 +478,14 @@ int SlicedGatherLog2(const FastParams& F, CopyDir dir, int order, int vec_bytes,
 // its scale side table in one launch. The first side_wgs workgroups move the
 // side piece (many blocks each, as in the general kernel), the rest take the
 // payload blocks in the fast kernel's order.
-template <typename V, bool kGather, int kUnroll, int kOrder>
+template <bool kGather, int kOrder>
 __global__ __launch_bounds__(kThreads) void block_copy_fast_side_kernel(FastParams P, KPiece side,
                                                                         uint32_t side_wgs) {
   if (blockIdx.x < side_wgs) {
-    copy_small_blocks<V, kGather>(side, P.ids, nullptr, P.error, P.n, blockIdx.x * side.bpw);
+    copy_small_blocks<kGather>(side, P.ids, nullptr, P.error, P.n, blockIdx.x * side.bpw);
     return;
   }
-  fast_block<V, kGather, kUnroll, kOrder>(P, blockIdx.x - side_wgs);
+  fast_block<kGather, kOrder>(P, blockIdx.x - side_wgs);
 }
 
 // Blocks per workgroup: one for blocks of >= 2 vectors per lane, otherwise
@@ -426,6 +495,14 @@ uint32_t BlocksPerWorkgroup(uint64_t elems) {
   uint64_t bpw = (8 * kThreads) / (elems == 0 ? 1 : elems);
   if (bpw > kSmallMaxBlocks) bpw = kSmallMaxBlocks;
   return static_cast<uint32_t>(bpw < 1 ? 1 : bpw);
+}
+
+// Whether a piece's other side is a second paged buffer (host memory that the
+// kernel reaches over PCIe).
+bool Paged(const CopyLaunch& l) {
+  bool paged = false;
+  for (int k = 0; k < l.npieces; ++k) paged = paged || l.pieces[k].others != 0;
+  return paged;
 }
 
 bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
@@ -440,6 +517,17 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
   P->error = l.error;
   P->n = static_cast<uint32_t>(l.n);
   P->npieces = l.npieces;
+  // Vectors of a piece: the common width if a launch has a second paged side,
+  // else the widest its blocks hold. Blocks of 2 and more vectors per lane go
+  // whole to a workgroup.
+  const bool paged = Paged(l);
+  auto vec_of = [&](uint64_t bytes) -> uint64_t {
+    uint64_t v = static_cast<uint64_t>(vec_bytes);
+    if (!paged) {
+      for (v = 16; v > bytes;) v /= 2;
+    }
+    return v;
+  };
   uint64_t total_blocks = 0;
   for (int k = 0; k < l.npieces; ++k) {
     total_blocks += static_cast<uint64_t>(l.pieces[k].nblocks > 0 ? l.pieces[k].nblocks : 0);
@@ -452,7 +540,7 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
     for (int k = 0; k < l.npieces; ++k) {
       const int64_t bb = l.pieces[k].block_bytes;
       if (bb <= 0) return false;
-      const bool whole = static_cast<uint64_t>(bb) / vec_bytes >= 2 * kThreads;
+      const bool whole = static_cast<uint64_t>(bb) / vec_of(bb) >= 2 * kThreads;
       if (whole == (pass == 1)) order[norder++] = k;
     }
   }
@@ -468,9 +556,14 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
         UINT32_MAX) {
       return false;
     }
-    const uint64_t elems = static_cast<uint64_t>(c.block_bytes) / vec_bytes;
-    if (elems > UINT32_MAX) return false;
+    // The limit on a block is the common width's, so that what a launch
+    // accepts does not depend on the vectors that move it.
+    if (static_cast<uint64_t>(c.block_bytes) / vec_bytes > UINT32_MAX) return false;
+    const uint64_t bytes = static_cast<uint64_t>(c.block_bytes);
+    const uint64_t vec = vec_of(bytes);
+    uint64_t elems = bytes / vec;
     const bool whole = elems >= 2 * kThreads;
+    if (!whole && bytes % vec != 0) ++elems;
     uint64_t bpw = BlocksPerWorkgroup(elems);
     if (whole && l.max_workgroups > 0) {
       // This piece's share of the workgroup cap, at least one.
@@ -491,7 +584,11 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
     kp.pool_blocks = c.pool_blocks;
     kp.f0 = static_cast<uint32_t>(c.f0);
     kp.nblocks = static_cast<uint32_t>(c.nblocks);
+    kp.bytes = bytes;
+    kp.magic = (uint64_t{1} << 32) / elems + 1;
+    kp.vec = static_cast<uint32_t>(vec);
     kp.elems = static_cast<uint32_t>(elems);
+    kp.rest = static_cast<uint32_t>(bytes % vec);
     kp.bpw = static_cast<uint32_t>(bpw);
     kp.whole = whole ? 1u : 0u;
     kp.wg_begin = static_cast<uint32_t>(wg);
@@ -517,7 +614,9 @@ bool BuildFastParams(const KParams& K, CopyDir dir, FastParams* F, int* order) {
   F->pool_blocks = p.pool_blocks;
   F->f0 = p.f0;
   F->n = K.n;
+  F->bytes = p.bytes;
   F->elems = p.elems;
+  F->rest = p.rest;
   const bool whole_storages = p.f0 % K.n == 0 && p.nblocks % K.n == 0;
   const uint32_t W = p.nblocks / K.n;
   *order = kStorageMajor;
@@ -556,9 +655,22 @@ constexpr uint32_t kLdsPerCu = 160u << 10;
 // LDS the general kernel declares (the small-block path's address tables).
 constexpr uint32_t kStaticLds = 2 * kSmallMaxBlocks * sizeof(uint64_t);
 
-template <typename V, int kUnroll>
+template <int V>
+hipError_t LaunchGeneral(const KParams& P, uint32_t grid, CopyDir dir, uint32_t gather_lds,
+                         hipStream_t stream) {
+  if (dir == CopyDir::kGather) {
+    hipLaunchKernelGGL((block_copy_kernel<V, true>), dim3(grid), dim3(kThreads),
+                       gather_lds, stream, P);
+  } else {
+    hipLaunchKernelGGL((block_copy_kernel<V, false>), dim3(grid), dim3(kThreads), 0,
+                       stream, P);
+  }
+  return hipGetLastError();
+}
+
+// whole_vec: vector bytes of the launch's whole-block pieces.
 hipError_t Launch(const KParams& P, uint32_t grid, CopyDir dir, int wg_per_cu,
-                  bool capped_grid, hipStream_t stream) {
+                  bool capped_grid, int whole_vec, hipStream_t stream) {
   FastParams F;
   int order = kStorageMajor;
   // Blocks above one workgroup's pass (kUnroll * kThreads vectors, 32 KiB at
@@ -574,31 +686,29 @@ hipError_t Launch(const KParams& P, uint32_t grid, CopyDir dir, int wg_per_cu,
     *g = *g - blocks + blocks * f->pieces;
   };
   if (BuildFastParams(P, dir, &F, &order)) {
-    if constexpr (sizeof(V) == 16) {
-      const int s = SlicedGatherLog2(F, dir, order, 16, kUnroll, capped_grid);
-      if (s > 0) {
-        const uint32_t sgrid = (((F.n + (1u << s) - 1) >> s) << s) * F.wstorages;
-        // The same cap on workgroups per CU as the fast gather.
-        const uint32_t lds = wg_per_cu > 0 ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) : 0;
-        hipLaunchKernelGGL((block_copy_sliced_gather_kernel<V, kUnroll, kGatherLog2Slices>),
-                           dim3(sgrid), dim3(kThreads), lds, stream, F);
-        return hipGetLastError();
-      }
+    const int s = SlicedGatherLog2(F, dir, order, capped_grid);
+    if (s > 0) {
+      const uint32_t sgrid = (((F.n + (1u << s) - 1) >> s) << s) * F.wstorages;
+      // The same cap on workgroups per CU as the fast gather.
+      const uint32_t lds = wg_per_cu > 0 ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) : 0;
+      hipLaunchKernelGGL((block_copy_sliced_gather_kernel<kGatherLog2Slices>),
+                         dim3(sgrid), dim3(kThreads), lds, stream, F);
+      return hipGetLastError();
     }
     split(&F, grid, &grid);
     // Gathers reserve (unused) LDS to cap their workgroups per CU.
     const uint32_t lds = wg_per_cu > 0 ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) : 0;
     if (dir == CopyDir::kGather && order == kStoragePairs) {
-      hipLaunchKernelGGL((block_copy_fast_kernel<V, true, kUnroll, kStoragePairs>), dim3(grid),
+      hipLaunchKernelGGL((block_copy_fast_kernel<true, kStoragePairs>), dim3(grid),
                          dim3(kThreads), lds, stream, F);
     } else if (dir == CopyDir::kGather) {
-      hipLaunchKernelGGL((block_copy_fast_kernel<V, true, kUnroll, kStorageMajor>), dim3(grid),
+      hipLaunchKernelGGL((block_copy_fast_kernel<true, kStorageMajor>), dim3(grid),
                          dim3(kThreads), lds, stream, F);
     } else if (order == kAllStorages) {
-      hipLaunchKernelGGL((block_copy_fast_kernel<V, false, kUnroll, kAllStorages>), dim3(grid),
+      hipLaunchKernelGGL((block_copy_fast_kernel<false, kAllStorages>), dim3(grid),
                          dim3(kThreads), 0, stream, F);
     } else {
-      hipLaunchKernelGGL((block_copy_fast_kernel<V, false, kUnroll, kStorageMajor>), dim3(grid),
+      hipLaunchKernelGGL((block_copy_fast_kernel<false, kStorageMajor>), dim3(grid),
                          dim3(kThreads), 0, stream, F);
     }
     return hipGetLastError();
@@ -614,28 +724,25 @@ hipError_t Launch(const KParams& P, uint32_t grid, CopyDir dir, int wg_per_cu,
   if (BuildFastSideParams(P, dir, &F, &side, &side_wgs, &order)) {
     split(&F, grid - side_wgs, &grid);
     if (dir == CopyDir::kGather && order == kStoragePairs) {
-      hipLaunchKernelGGL((block_copy_fast_side_kernel<V, true, kUnroll, kStoragePairs>),
+      hipLaunchKernelGGL((block_copy_fast_side_kernel<true, kStoragePairs>),
                          dim3(grid), dim3(kThreads), glds, stream, F, side, side_wgs);
     } else if (dir == CopyDir::kGather) {
-      hipLaunchKernelGGL((block_copy_fast_side_kernel<V, true, kUnroll, kStorageMajor>),
+      hipLaunchKernelGGL((block_copy_fast_side_kernel<true, kStorageMajor>),
                          dim3(grid), dim3(kThreads), glds, stream, F, side, side_wgs);
     } else if (order == kAllStorages) {
-      hipLaunchKernelGGL((block_copy_fast_side_kernel<V, false, kUnroll, kAllStorages>),
+      hipLaunchKernelGGL((block_copy_fast_side_kernel<false, kAllStorages>),
                          dim3(grid), dim3(kThreads), 0, stream, F, side, side_wgs);
     } else {
-      hipLaunchKernelGGL((block_copy_fast_side_kernel<V, false, kUnroll, kStorageMajor>),
+      hipLaunchKernelGGL((block_copy_fast_side_kernel<false, kStorageMajor>),
                          dim3(grid), dim3(kThreads), 0, stream, F, side, side_wgs);
     }
     return hipGetLastError();
   }
-  if (dir == CopyDir::kGather) {
-    hipLaunchKernelGGL((block_copy_kernel<V, true, kUnroll>), dim3(grid),
-                       dim3(kThreads), glds, stream, P);
-  } else {
-    hipLaunchKernelGGL((block_copy_kernel<V, false, kUnroll>), dim3(grid),
-                       dim3(kThreads), 0, stream, P);
+  switch (whole_vec) {
+    case 16: return LaunchGeneral<16>(P, grid, dir, glds, stream);
+    case 4: return LaunchGeneral<4>(P, grid, dir, glds, stream);
+    default: return LaunchGeneral<1>(P, grid, dir, glds, stream);
   }
-  return hipGetLastError();
 }
 
 }  // namespace
@@ -668,16 +775,8 @@ hipError_t LaunchBlockCopy(const CopyLaunch& l, CopyDir dir, int vec_bytes,
     return hipErrorInvalidValue;
   }
   const int cap = l.gather_workgroups_per_cu;
-  switch (vec_bytes) {
-    case 16:
-      return Launch<u32x4, 8>(P, grid, dir, cap, l.max_workgroups > 0, stream);
-    case 4:
-      return Launch<uint32_t, 8>(P, grid, dir, cap, l.max_workgroups > 0, stream);
-    case 1:
-      return Launch<uint8_t, 8>(P, grid, dir, cap, l.max_workgroups > 0, stream);
-    default:
-      return hipErrorInvalidValue;
-  }
+  if (vec_bytes != 16 && vec_bytes != 4 && vec_bytes != 1) return hipErrorInvalidValue;
+  return Launch(P, grid, dir, cap, l.max_workgroups > 0, Paged(l) ? vec_bytes : 16, stream);
 }
 
 }  // namespace kvx
