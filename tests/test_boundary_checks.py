@@ -202,3 +202,18 @@ def test_link_peaks_validate_arguments_before_the_device(kvx):
     assert lib.kvx_measure_link_peaks(1 << 20, 5, None, None) == 3
     with pytest.raises(kvx.KvxError):
         kvx.measure_link_peaks(0, 5)
+
+
+def test_id_lists_convert_as_int_does(kvx):
+    """Lists of ints convert in one pass; everything else as int() and the
+    64-bit wrap of ctypes always did."""
+    np = pytest.importorskip("numpy")
+    cases = [([], []), ([3, -1, 2**63 - 1], [3, -1, 2**63 - 1]), ((4, True), [4, 1]),
+             ([1.5, 2], [1, 2]), (["7"], [7]), ([2**63], [-2**63]), (b"\x05a", [5, 97]),
+             (range(2), [0, 1]), (np.array([8, 9], np.int32), [8, 9]), ([np.int64(6)], [6])]
+    for values, want in cases:
+        arr, n = kvx._capi.i64_array(values)
+        assert n == len(want) and list(arr[:n]) == want, values
+    for bad in ([None], ["x"], [[1]]):
+        with pytest.raises((TypeError, ValueError)):
+            kvx._capi.i64_array(bad)

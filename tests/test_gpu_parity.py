@@ -1084,3 +1084,23 @@ def test_gather_scatter_every_block_of_the_pool(kvx, cuda, layers, cap):
         assert np.array_equal(dev_np(fresh[l][0]), host[l][0]), l
     mgr.close()
     mgr2.close()
+
+
+@pytest.mark.parametrize("blocks", [70, 100000])
+def test_scatter_names_the_same_bad_lists(kvx, cuda, blocks):
+    """Duplicate ids are refused whether they lie close together or far apart,
+    and the first bad id of a list names the error, as with one check per id."""
+    pool = torch.zeros(blocks, 16, dtype=torch.uint8, device=cuda)
+    mgr = kvx.KVCacheManager([pool], host_blocks_to_allocate=1)
+    staging = torch.full((8 * 16,), 7, dtype=torch.uint8, device=cuda)
+    top = blocks - 1
+    for ids in ([0, top, 0], [top, top], [5, 69, 6, 69]):
+        with pytest.raises(kvx.KvxError, match="must be unique"):
+            mgr.scatter(ids, staging)
+    with pytest.raises(kvx.KvxError, match="non-negative"):
+        mgr.scatter([1, -1, blocks], staging)
+    with pytest.raises(kvx.KvxError, match="exceeds"):
+        mgr.gather([1, blocks, -1], staging)
+    assert not pool.any()
+    mgr.scatter([top, 0, 65], staging).Await()
+    assert pool.sum().item() == 3 * 16 * 7
