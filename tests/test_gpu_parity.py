@@ -1104,3 +1104,39 @@ def test_scatter_names_the_same_bad_lists(kvx, cuda, blocks):
     assert not pool.any()
     mgr.scatter([top, 0, 65], staging).Await()
     assert pool.sum().item() == 3 * 16 * 7
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 831, 832, 833, 1500])
+def test_gather_scatter_around_the_inline_id_limits(kvx, cuda, n):
+    """Few ids travel in the kernel's arguments, more in larger arguments, the
+    rest in an uploaded table: each of them with whole blocks, small blocks, a
+    side table, one layer of the pool, and storages whose block sizes
+    alternate (no consecutive bases), on two streams in turn."""
+    rng = np.random.default_rng(n)
+    blocks = 1600
+    streams = [torch.cuda.Stream(cuda), torch.cuda.Stream(cuda)]
+    for k, sizes in enumerate(([32768] * 4, [8192 + 32] * 3, [4096] * 4, [48] * 5,
+                               [16384] * 2 + [4] * 2, [64, 512, 64, 512])):
+        pools_np = [rng.integers(0, 256, (blocks, b), dtype=np.uint8) for b in sizes]
+        pools = [torch.from_numpy(p).to(cuda) for p in pools_np]
+        torch.cuda.synchronize()
+        mgr = kvx.KVCacheManager(pools, host_blocks_to_allocate=1)
+        ids = rng.permutation(blocks)[:n].tolist()
+        order = sorted(range(len(sizes)), key=lambda w: sizes.index(sizes[w]))
+        for layer in (None, len(sizes) - 1):
+            picked = order if layer is None else [layer]
+            want = np.concatenate([pools_np[w][ids].reshape(-1) for w in picked])
+            staging = torch.zeros(want.size, dtype=torch.uint8, device=cuda)
+            torch.cuda.synchronize()
+            s = streams[k % 2]
+            mgr.gather(ids, staging, layer_idx=layer, stream=s).Await()
+            assert np.array_equal(staging.cpu().numpy(), want), (sizes, layer)
+            dst = rng.permutation(blocks)[:n].tolist()
+            mgr.scatter(dst, staging, layer_idx=layer, stream=s).Await()
+            at = 0
+            for w in picked:
+                pools_np[w][dst] = want[at:at + n * sizes[w]].reshape(n, sizes[w])
+                at += n * sizes[w]
+            for w, p in enumerate(pools):
+                assert np.array_equal(p.cpu().numpy(), pools_np[w]), (sizes, layer, w)
+        mgr.close()

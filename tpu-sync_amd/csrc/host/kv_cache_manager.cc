@@ -219,6 +219,9 @@ Status KVCacheManager::Init() {
     EngineOptions eo = cfg_.engine;
     eo.device = cfg_.device;
     KVX_ASSIGN_OR_RETURN(engine_, TransferEngine::Create(eo));
+    std::vector<uint64_t> bases;
+    for (const StorageInfo& si : storages_) bases.push_back(si.dev);
+    KVX_RETURN_IF_ERROR(engine_->SetStorages(bases));
     // hipHostMalloc memory is mapped into the GPU's address space, so the
     // copy kernels may read and write the mirror directly.
     host_kernel_access_ = cfg_.host_alloc == HostAllocKind::kPinned;

@@ -6,6 +6,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <numeric>
+#include <optional>
 #include <thread>
 
 #include "../kernels/block_copy.h"
@@ -229,6 +230,29 @@ Status TransferEngine::Init() {
   return GrowArgRing(opts_.arg_ring_bytes);
 }
 
+Status TransferEngine::SetStorages(const std::vector<uint64_t>& bases) {
+  if (bases.empty()) return OkStatus();
+  DeviceGuard g(opts_.device);
+  void* d = nullptr;
+  KVX_HIP_RETURN_IF_ERROR(hipMalloc(&d, bases.size() * sizeof(uint64_t)));
+  bases_dev_ = reinterpret_cast<uint64_t>(d);
+  KVX_HIP_RETURN_IF_ERROR(
+      hipMemcpy(d, bases.data(), bases.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
+  bases_ = bases;
+  return OkStatus();
+}
+
+uint64_t TransferEngine::ResidentTable(const std::vector<StorageView>& storages,
+                                       const Group& g) const {
+  const size_t W = g.members.size();
+  for (size_t at = 0; at + W <= bases_.size(); ++at) {
+    size_t m = 0;
+    while (m < W && bases_[at + m] == storages[g.members[m]].dev) ++m;
+    if (m == W) return bases_dev_ + at * sizeof(uint64_t);
+  }
+  return 0;
+}
+
 Status TransferEngine::EnsureRing(Ring* r) {
   // Allocated on first use: a manager whose copies all go zero-copy or
   // through the pageable lanes never holds these chunks.
@@ -284,6 +308,7 @@ TransferEngine::~TransferEngine() {
   }
   if (arg_host_ != nullptr) (void)hipHostFree(arg_host_);
   if (arg_dev_ != 0) (void)hipFree(reinterpret_cast<void*>(arg_dev_));
+  if (bases_dev_ != 0) (void)hipFree(reinterpret_cast<void*>(bases_dev_));
   for (hipStream_t s :
        {gather_stream_, d2h_stream_, h2d_stream_, scatter_stream_}) {
     if (s != nullptr) (void)hipStreamDestroy(s);
@@ -1608,33 +1633,58 @@ StatusOr<CopyFuture> TransferEngine::DeviceCopy(
   }
   std::lock_guard<std::mutex> l(mu_);
   DeviceGuard dg(opts_.device);
-  int64_t arg_bytes = AlignUp(n * 8, kArgAlign);
-  std::vector<int64_t> table_off(groups.size());
-  for (size_t gi = 0; gi < groups.size(); ++gi) {
-    table_off[gi] = arg_bytes;
-    arg_bytes += AlignUp(static_cast<int64_t>(groups[gi].members.size()) * 8, kArgAlign);
+  // Up to kMaxInlineIds ids go to the kernel in its arguments and the bases are
+  // on the device already, so that nothing is uploaded before the kernel (an upload is
+  // a copy kernel of 4-5 us and a gap): 512 blocks of 64 storages gathered in
+  // 358 us a call against 367, one block in 13 against 18-22.
+  std::vector<uint32_t> inline_ids;
+  bool inl = n <= kMaxInlineIds;
+  for (size_t gi = 0; inl && gi < groups.size(); ++gi) {
+    groups[gi].table_dev = ResidentTable(storages, groups[gi]);
+    inl = groups[gi].table_dev != 0;
   }
-  KVX_ASSIGN_OR_RETURN(int64_t aoff, ArgAlloc(arg_bytes));
-  ArgSliceGuard keep(
-      [this, aoff, arg_bytes, stream] { return ArgCommit(aoff, aoff + arg_bytes, stream); },
-      stream);
-  std::memcpy(arg_host_ + aoff, ids.data(), n * 8);
-  uint64_t acc = staging;
-  for (size_t gi = 0; gi < groups.size(); ++gi) {
-    uint64_t* t = reinterpret_cast<uint64_t*>(arg_host_ + aoff + table_off[gi]);
-    for (size_t m = 0; m < groups[gi].members.size(); ++m) {
-      t[m] = storages[groups[gi].members[m]].dev;
-      acc |= t[m];
+  if (inl) {
+    inline_ids.reserve(n);
+    for (int64_t id : ids) {
+      inl = inl && id >= 0 && id <= UINT32_MAX;
+      inline_ids.push_back(static_cast<uint32_t>(id));
     }
-    groups[gi].table_dev = arg_dev_ + aoff + table_off[gi];
   }
-  KVX_HIP_RETURN_IF_ERROR(hipMemcpyAsync(reinterpret_cast<void*>(arg_dev_ + aoff),
-                                         arg_host_ + aoff, arg_bytes,
-                                         hipMemcpyHostToDevice, stream));
+  uint64_t acc = staging;
+  for (const StorageView& sv : storages) acc |= sv.dev;
+  int64_t aoff = 0, arg_bytes = 0;
+  std::optional<ArgSliceGuard> keep;
+  if (!inl) {
+    arg_bytes = AlignUp(n * 8, kArgAlign);
+    std::vector<int64_t> table_off(groups.size());
+    for (size_t gi = 0; gi < groups.size(); ++gi) {
+      table_off[gi] = arg_bytes;
+      arg_bytes += AlignUp(static_cast<int64_t>(groups[gi].members.size()) * 8, kArgAlign);
+    }
+    KVX_ASSIGN_OR_RETURN(aoff, ArgAlloc(arg_bytes));
+    keep.emplace(
+        [this, aoff, arg_bytes, stream] { return ArgCommit(aoff, aoff + arg_bytes, stream); },
+        stream);
+    std::memcpy(arg_host_ + aoff, ids.data(), n * 8);
+    for (size_t gi = 0; gi < groups.size(); ++gi) {
+      uint64_t* t = reinterpret_cast<uint64_t*>(arg_host_ + aoff + table_off[gi]);
+      for (size_t m = 0; m < groups[gi].members.size(); ++m) {
+        t[m] = storages[groups[gi].members[m]].dev;
+      }
+      groups[gi].table_dev = arg_dev_ + aoff + table_off[gi];
+    }
+    KVX_HIP_RETURN_IF_ERROR(hipMemcpyAsync(reinterpret_cast<void*>(arg_dev_ + aoff),
+                                           arg_host_ + aoff, arg_bytes,
+                                           hipMemcpyHostToDevice, stream));
+  }
   int64_t off = 0;
   for (size_t g0 = 0; g0 < groups.size(); g0 += kMaxPieces) {
     CopyLaunch cl;
-    cl.ids = reinterpret_cast<const int64_t*>(arg_dev_ + aoff);
+    if (inl) {
+      cl.inline_ids = inline_ids.data();
+    } else {
+      cl.ids = reinterpret_cast<const int64_t*>(arg_dev_ + aoff);
+    }
     cl.n = n;
     for (size_t gi = g0; gi < groups.size() && gi < g0 + kMaxPieces; ++gi) {
       const Group& gr = groups[gi];
@@ -1654,7 +1704,7 @@ StatusOr<CopyFuture> TransferEngine::DeviceCopy(
     const int vec = LaunchVectorBytes(cl, acc);
     KVX_RETURN_IF_ERROR(LaunchCopy(cl, gather, vec, stream));
   }
-  KVX_RETURN_IF_ERROR(keep.Commit());
+  if (keep) KVX_RETURN_IF_ERROR(keep->Commit());
   KVX_ASSIGN_OR_RETURN(hipEvent_t done, NewEvent());
   KVX_HIP_RETURN_IF_ERROR(hipEventRecord(done, stream));
   return CopyFuture::FromEvents({done}, {});

@@ -256,6 +256,10 @@ class TransferEngine {
   // far; waits for them to finish. `reset` drops the samples.
   StatusOr<KernelTimes> ProfiledKernelTimes(bool gather, bool reset);
 
+  // Puts the base addresses of the owner's storages, in (layer, shard) order,
+  // on the device for good. Called once, before any copy.
+  Status SetStorages(const std::vector<uint64_t>& bases);
+
  private:
   struct Group {
     int64_t block_bytes = 0;
@@ -290,6 +294,9 @@ class TransferEngine {
 
   explicit TransferEngine(const EngineOptions& opts);
   Status Init();
+  // Device address of consecutive entries of the resident base table that hold
+  // the group's bases in order; 0 if it has none.
+  uint64_t ResidentTable(const std::vector<StorageView>& storages, const Group& g) const;
   // Reserves `bytes` of the pinned/device argument ring; waits on the host
   // only if the region is still read by an earlier, unfinished copy.
   StatusOr<int64_t> ArgAlloc(int64_t bytes);
@@ -385,6 +392,10 @@ class TransferEngine {
   StreamPlacement placement_;
   Ring out_ring_;
   Ring in_ring_;
+  // Every storage's base address in (layer, shard) order, and its copy on the
+  // device: written once, before the first copy.
+  std::vector<uint64_t> bases_;
+  uint64_t bases_dev_ = 0;
   uint8_t* arg_host_ = nullptr;
   uint64_t arg_dev_ = 0;
   int64_t arg_bytes_ = 0;

@@ -22,6 +22,8 @@
 namespace kvx {
 
 constexpr int kMaxPieces = 4;
+// Ids a launch can carry in its kernel arguments (under 4 KiB with the rest).
+constexpr int kMaxInlineIds = 832;
 constexpr int kDefaultGatherWorkgroupsPerCu = 2;
 
 struct CopyPiece {
@@ -48,6 +50,9 @@ struct CopyLaunch {
   CopyPiece pieces[kMaxPieces];
   int npieces = 0;
   const int64_t* ids = nullptr;   // device array of n block ids
+  // Or, with ids null and no paged other side: n <= kMaxInlineIds ids in host
+  // memory, consumed before the launch returns.
+  const uint32_t* inline_ids = nullptr;
   const int64_t* ids2 = nullptr;  // block ids on the `others` side (if used)
   int64_t n = 0;
   int32_t* error = nullptr;      // optional device word; set to 1 on a bad id

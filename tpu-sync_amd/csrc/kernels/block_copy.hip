@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 
 #include "block_copy.h"
 
@@ -86,6 +87,19 @@ struct KPiece {
   uint32_t bpw;       // blocks per workgroup
   uint32_t wg_begin;  // first workgroup of the piece
   uint32_t whole;     // 1: every lane works on one block at a time
+};
+
+// A kernel's one argument: its parameters and, with kCap > 0, the block ids
+// themselves instead of a device table, so that a call needs no upload before
+// its kernel.
+template <typename P, int kCap>
+struct Args {
+  P p;
+  uint32_t ids[kCap];
+};
+template <typename P>
+struct Args<P, 0> {
+  P p;
 };
 
 struct KParams {
@@ -151,6 +165,34 @@ __device__ __forceinline__ KPiece select_piece(const KParams& P, uint32_t wg) {
   return p;
 }
 
+// Address of a kernel's ids: its table, or where they lie in the kernel
+// arguments (taken from the argument segment itself, so that an indexed read
+// stays a load from there).
+template <typename P, int kCap>
+__device__ __forceinline__ uint64_t ids_address(const int64_t* table) {
+  if constexpr (kCap == 0) {
+    return reinterpret_cast<uint64_t>(table);
+  } else {
+    typedef Args<P, kCap> A;
+    return reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr()) +
+           __builtin_offsetof(A, ids);
+  }
+}
+
+// Id i, the same for the whole workgroup.
+template <int kCap>
+__device__ __forceinline__ int64_t uniform_id(uint64_t ids, uint32_t i) {
+  if constexpr (kCap == 0) return uniform_load<int64_t>(ids, i);
+  return uniform_load<uint32_t>(ids, i);
+}
+
+// Id i of a lane.
+template <int kCap>
+__device__ __forceinline__ int64_t lane_id(uint64_t ids, uint32_t i) {
+  if constexpr (kCap == 0) return gptr<const int64_t>(ids)[i];
+  return gptr<const uint32_t>(ids)[i];
+}
+
 __device__ __forceinline__ bool bad_id(int64_t id, int64_t limit) {
   return static_cast<uint64_t>(id) >= static_cast<uint64_t>(limit);
 }
@@ -204,8 +246,8 @@ __device__ __forceinline__ void move_small_blocks(const uint64_t* s_src, const u
 // 4 KiB blocks of 160 storages gathered in 177 us (5.7 TB/s; 242 with one
 // vector in flight a lane), 2 KiB blocks with a 4-byte scale per (layer, block)
 // scattered in 95 us (114 at the scales' 4-byte vectors for the whole launch).
-template <bool kGather>
-__device__ __forceinline__ void copy_small_blocks(const KPiece& p, const int64_t* ids,
+template <bool kGather, int kCap>
+__device__ __forceinline__ void copy_small_blocks(const KPiece& p, uint64_t ids,
                                                   const int64_t* ids2, int32_t* error,
                                                   uint32_t n, uint32_t b0) {
   __shared__ uint64_t s_src[kSmallMaxBlocks];
@@ -216,7 +258,7 @@ __device__ __forceinline__ void copy_small_blocks(const KPiece& p, const int64_t
     const uint32_t f = p.f0 + b0 + b;
     const uint32_t w = f / n;
     const uint32_t i = f - w * n;
-    const int64_t id = gptr<const int64_t>(reinterpret_cast<uint64_t>(ids))[i];
+    const int64_t id = lane_id<kCap>(ids, i);
     const uint64_t base = gptr<const uint64_t>(p.storages)[w];
     bool bad = bad_id(id, p.pool_blocks);
     uint64_t other;
@@ -246,9 +288,11 @@ __device__ __forceinline__ void copy_small_blocks(const KPiece& p, const int64_t
   }
 }
 
-template <int V, bool kGather>
-__global__ __launch_bounds__(kThreads) void block_copy_kernel(KParams P) {
+template <int V, bool kGather, int kCap>
+__global__ __launch_bounds__(kThreads) void block_copy_kernel(Args<KParams, kCap> args) {
+  const KParams& P = args.p;
   const uint32_t wg = blockIdx.x;
+  const uint64_t ids = ids_address<KParams, kCap>(P.ids);
   const KPiece p = select_piece(P, wg);
   const uint32_t b0 = (wg - p.wg_begin) * p.bpw;
   const uint32_t n = P.n;
@@ -262,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void block_copy_kernel(KParams P) {
       const uint32_t f = p.f0 + b0 + b;
       const uint32_t w = f / n;
       const uint32_t i = f - w * n;
-      const int64_t id = uniform_load<int64_t>(reinterpret_cast<uint64_t>(P.ids), i);
+      const int64_t id = uniform_id<kCap>(ids, i);
       uint64_t other;
       bool bad = bad_id(id, p.pool_blocks);
       if (p.others != 0) {
@@ -289,7 +333,7 @@ __global__ __launch_bounds__(kThreads) void block_copy_kernel(KParams P) {
     return;
   }
 
-  copy_small_blocks<kGather>(p, P.ids, P.ids2, P.error, n, b0);
+  copy_small_blocks<kGather, kCap>(p, ids, P.ids2, P.error, n, b0);
 }
 
 // The common launch (one piece of large blocks, no second paged side, one
@@ -327,8 +371,8 @@ enum FastOrder : int { kStorageMajor = 0, kStoragePairs = 1, kAllStorages = 2 };
 // Workgroup g of a fast launch: one whole block, or with pieces > 1 one
 // piece of piece_elems vectors of a block, the pieces of a block on
 // consecutive workgroups (so a large block's writes are in flight together).
-template <bool kGather, int kOrder>
-__device__ __forceinline__ void fast_block(const FastParams& P, uint32_t g) {
+template <bool kGather, int kOrder, int kCap>
+__device__ __forceinline__ void fast_block(const FastParams& P, uint64_t ids, uint32_t g) {
   constexpr int V = 16;
   uint32_t piece = 0;
   if (P.pieces > 1) {
@@ -357,7 +401,7 @@ __device__ __forceinline__ void fast_block(const FastParams& P, uint32_t g) {
   // work. (Measured against the branching form in one process on the same
   // allocations: equal, within 0.3 %.)
   const uint64_t base = uniform_load<uint64_t>(P.storages, w);
-  const int64_t id = uniform_load<int64_t>(reinterpret_cast<uint64_t>(P.ids), i);
+  const int64_t id = uniform_id<kCap>(ids, i);
   const bool bad = bad_id(id, P.pool_blocks);
   const uint32_t first = piece * P.piece_elems;  // 0 unless the block is split
   const uint32_t left = P.elems - first;
@@ -376,9 +420,9 @@ __device__ __forceinline__ void fast_block(const FastParams& P, uint32_t g) {
   if (bad && threadIdx.x == 0 && P.error != nullptr) atomicOr(P.error, 1);
 }
 
-template <bool kGather, int kOrder>
-__global__ __launch_bounds__(kThreads) void block_copy_fast_kernel(FastParams P) {
-  fast_block<kGather, kOrder>(P, blockIdx.x);
+template <bool kGather, int kOrder, int kCap>
+__global__ __launch_bounds__(kThreads) void block_copy_fast_kernel(Args<FastParams, kCap> args) {
+  fast_block<kGather, kOrder, kCap>(args.p, ids_address<FastParams, kCap>(args.p.ids), blockIdx.x);
 }
 
 // Sliced form of the fast gather, for blocks of exactly one pass (kUnroll *
@@ -393,8 +437,11 @@ __global__ __launch_bounds__(kThreads) void block_copy_fast_kernel(FastParams P)
 // +2.2 points of HBM bandwidth (e.g. 75.2 against 73.9 %). The same form for
 // the scatter (8 slices, all-storages order) measured -1.5 to +1.7 points
 // and is not used.
-template <int kLog2H>
-__global__ __launch_bounds__(kThreads) void block_copy_sliced_gather_kernel(FastParams P) {
+template <int kLog2H, int kCap>
+__global__ __launch_bounds__(kThreads) void block_copy_sliced_gather_kernel(
+    Args<FastParams, kCap> args) {
+  const FastParams& P = args.p;
+  const uint64_t ids = ids_address<FastParams, kCap>(P.ids);
   constexpr int V = 16;
   constexpr uint32_t kH = 1u << kLog2H;
   constexpr uint32_t kSlice = kUnroll * kThreads / kH;  // vectors per slice
@@ -421,7 +468,7 @@ __global__ __launch_bounds__(kThreads) void block_copy_sliced_gather_kernel(Fast
   for (uint32_t r = 0; r < kH; ++r) {
     const uint32_t i = (ig << kLog2H) + r;
     const bool in = i < P.n;
-    const int64_t id = in ? uniform_load<int64_t>(reinterpret_cast<uint64_t>(P.ids), i) : 0;
+    const int64_t id = in ? uniform_id<kCap>(ids, i) : 0;
     const bool bad = in && bad_id(id, P.pool_blocks);
     ok[r] = in && !bad;
     bad_any |= bad;
@@ -478,14 +525,23 @@ int SlicedGatherLog2(const FastParams& F, CopyDir dir, int order, bool capped_gr
 // its scale side table in one launch. The first side_wgs workgroups move the
 // side piece (many blocks each, as in the general kernel), the rest take the
 // payload blocks in the fast kernel's order.
-template <bool kGather, int kOrder>
-__global__ __launch_bounds__(kThreads) void block_copy_fast_side_kernel(FastParams P, KPiece side,
-                                                                        uint32_t side_wgs) {
-  if (blockIdx.x < side_wgs) {
-    copy_small_blocks<kGather>(side, P.ids, nullptr, P.error, P.n, blockIdx.x * side.bpw);
+struct FastSideParams {
+  FastParams fast;
+  KPiece side;
+  uint32_t side_wgs;
+};
+
+template <bool kGather, int kOrder, int kCap>
+__global__ __launch_bounds__(kThreads) void block_copy_fast_side_kernel(
+    Args<FastSideParams, kCap> args) {
+  const FastSideParams& P = args.p;
+  const uint64_t ids = ids_address<FastSideParams, kCap>(P.fast.ids);
+  if (blockIdx.x < P.side_wgs) {
+    copy_small_blocks<kGather, kCap>(P.side, ids, nullptr, P.fast.error, P.fast.n,
+                                     blockIdx.x * P.side.bpw);
     return;
   }
-  fast_block<kGather, kOrder>(P, blockIdx.x - side_wgs);
+  fast_block<kGather, kOrder, kCap>(P.fast, ids, blockIdx.x - P.side_wgs);
 }
 
 // Blocks per workgroup: one for blocks of >= 2 vectors per lane, otherwise
@@ -507,7 +563,8 @@ bool Paged(const CopyLaunch& l) {
 
 bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
                  uint32_t* grid) {
-  if (l.npieces < 1 || l.npieces > kMaxPieces || l.ids == nullptr ||
+  if (l.npieces < 1 || l.npieces > kMaxPieces ||
+      (l.ids == nullptr && (l.inline_ids == nullptr || l.n > kMaxInlineIds || Paged(l))) ||
       l.n <= 0 || l.n > INT32_MAX || vec_bytes <= 0) {
     return false;
   }
@@ -655,94 +712,98 @@ constexpr uint32_t kLdsPerCu = 160u << 10;
 // LDS the general kernel declares (the small-block path's address tables).
 constexpr uint32_t kStaticLds = 2 * kSmallMaxBlocks * sizeof(uint64_t);
 
-template <int V>
-hipError_t LaunchGeneral(const KParams& P, uint32_t grid, CopyDir dir, uint32_t gather_lds,
-                         hipStream_t stream) {
-  if (dir == CopyDir::kGather) {
-    hipLaunchKernelGGL((block_copy_kernel<V, true>), dim3(grid), dim3(kThreads),
-                       gather_lds, stream, P);
-  } else {
-    hipLaunchKernelGGL((block_copy_kernel<V, false>), dim3(grid), dim3(kThreads), 0,
-                       stream, P);
+// Few ids take kernels with smaller arguments: one block of 64 storages
+// gathered in 13.0 us a call, 14.6 with room for kMaxInlineIds (copied twice
+// on the way to the queue).
+constexpr int kFewInlineIds = 64;
+
+// A launch with its ids in a table (kCap = 0) or in its arguments.
+template <int kCap>
+struct Launcher {
+  const uint32_t* inline_ids;
+  uint32_t n;
+  uint32_t grid;
+  uint32_t lds;
+  hipStream_t stream;
+
+  template <typename P>
+  hipError_t Run(void (*kernel)(Args<P, kCap>), const P& p) const {
+    Args<P, kCap> a{};
+    a.p = p;
+    if constexpr (kCap > 0) std::memcpy(a.ids, inline_ids, n * sizeof(uint32_t));
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, a);
+    return hipGetLastError();
   }
-  return hipGetLastError();
-}
+  template <bool kGather, int kOrder>
+  hipError_t Fast(const FastParams& F) const {
+    return Run<FastParams>(block_copy_fast_kernel<kGather, kOrder, kCap>, F);
+  }
+  template <bool kGather, int kOrder>
+  hipError_t FastSide(const FastSideParams& F) const {
+    return Run<FastSideParams>(block_copy_fast_side_kernel<kGather, kOrder, kCap>, F);
+  }
+  template <int V>
+  hipError_t General(const KParams& K, bool gather) const {
+    return gather ? Run<KParams>(block_copy_kernel<V, true, kCap>, K)
+                  : Run<KParams>(block_copy_kernel<V, false, kCap>, K);
+  }
+};
 
 // whole_vec: vector bytes of the launch's whole-block pieces.
-hipError_t Launch(const KParams& P, uint32_t grid, CopyDir dir, int wg_per_cu,
-                  bool capped_grid, int whole_vec, hipStream_t stream) {
-  FastParams F;
+template <int kCap>
+hipError_t Launch(const KParams& P, const uint32_t* inline_ids, uint32_t grid, CopyDir dir,
+                  int wg_per_cu, bool capped_grid, int whole_vec, hipStream_t stream) {
+  const bool gather = dir == CopyDir::kGather;
+  // Gathers reserve (unused) LDS to cap their workgroups per CU.
+  Launcher<kCap> to{inline_ids, P.n, grid, 0, stream};
+  if (gather && wg_per_cu > 0) to.lds = kLdsPerCu / static_cast<uint32_t>(wg_per_cu);
+  FastSideParams FS;
+  FastParams& F = FS.fast;
   int order = kStorageMajor;
   // Blocks above one workgroup's pass (kUnroll * kThreads vectors, 32 KiB at
   // 16-byte vectors) go to consecutive workgroups a pass each, unless the
   // launch's grid is capped (zero-copy copies keep their few workgroups).
-  auto split = [&](FastParams* f, uint32_t blocks, uint32_t* g) {
+  auto split = [&](uint32_t blocks) {
     const uint32_t pass = kUnroll * kThreads;
-    if (capped_grid || f->elems <= pass) return;
-    const uint64_t pieces = (static_cast<uint64_t>(f->elems) + pass - 1) / pass;
-    if (static_cast<uint64_t>(blocks) * pieces + (*g - blocks) > INT32_MAX) return;
-    f->pieces = static_cast<uint32_t>(pieces);
-    f->piece_elems = pass;
-    *g = *g - blocks + blocks * f->pieces;
+    if (capped_grid || F.elems <= pass) return;
+    const uint64_t pieces = (static_cast<uint64_t>(F.elems) + pass - 1) / pass;
+    if (static_cast<uint64_t>(blocks) * pieces + (to.grid - blocks) > INT32_MAX) return;
+    F.pieces = static_cast<uint32_t>(pieces);
+    F.piece_elems = pass;
+    to.grid = to.grid - blocks + blocks * F.pieces;
   };
   if (BuildFastParams(P, dir, &F, &order)) {
     const int s = SlicedGatherLog2(F, dir, order, capped_grid);
     if (s > 0) {
-      const uint32_t sgrid = (((F.n + (1u << s) - 1) >> s) << s) * F.wstorages;
-      // The same cap on workgroups per CU as the fast gather.
-      const uint32_t lds = wg_per_cu > 0 ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) : 0;
-      hipLaunchKernelGGL((block_copy_sliced_gather_kernel<kGatherLog2Slices>),
-                         dim3(sgrid), dim3(kThreads), lds, stream, F);
-      return hipGetLastError();
+      to.grid = (((F.n + (1u << s) - 1) >> s) << s) * F.wstorages;
+      return to.template Run<FastParams>(
+          block_copy_sliced_gather_kernel<kGatherLog2Slices, kCap>, F);
     }
-    split(&F, grid, &grid);
-    // Gathers reserve (unused) LDS to cap their workgroups per CU.
-    const uint32_t lds = wg_per_cu > 0 ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) : 0;
-    if (dir == CopyDir::kGather && order == kStoragePairs) {
-      hipLaunchKernelGGL((block_copy_fast_kernel<true, kStoragePairs>), dim3(grid),
-                         dim3(kThreads), lds, stream, F);
-    } else if (dir == CopyDir::kGather) {
-      hipLaunchKernelGGL((block_copy_fast_kernel<true, kStorageMajor>), dim3(grid),
-                         dim3(kThreads), lds, stream, F);
-    } else if (order == kAllStorages) {
-      hipLaunchKernelGGL((block_copy_fast_kernel<false, kAllStorages>), dim3(grid),
-                         dim3(kThreads), 0, stream, F);
-    } else {
-      hipLaunchKernelGGL((block_copy_fast_kernel<false, kStorageMajor>), dim3(grid),
-                         dim3(kThreads), 0, stream, F);
+    split(grid);
+    if (gather) {
+      return order == kStoragePairs ? to.template Fast<true, kStoragePairs>(F)
+                                    : to.template Fast<true, kStorageMajor>(F);
     }
-    return hipGetLastError();
+    return order == kAllStorages ? to.template Fast<false, kAllStorages>(F)
+                                 : to.template Fast<false, kStorageMajor>(F);
   }
-  // HBM-bound gathers (not the capped grids of zero-copy copies) on the
-  // kernels with the small-block path take the same cap, minus that path's
-  // own 4 KiB of address tables.
-  const uint32_t glds = wg_per_cu > 0 && !capped_grid
-                            ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) - kStaticLds
-                            : 0;
-  KPiece side;
-  uint32_t side_wgs = 0;
-  if (BuildFastSideParams(P, dir, &F, &side, &side_wgs, &order)) {
-    split(&F, grid - side_wgs, &grid);
-    if (dir == CopyDir::kGather && order == kStoragePairs) {
-      hipLaunchKernelGGL((block_copy_fast_side_kernel<true, kStoragePairs>),
-                         dim3(grid), dim3(kThreads), glds, stream, F, side, side_wgs);
-    } else if (dir == CopyDir::kGather) {
-      hipLaunchKernelGGL((block_copy_fast_side_kernel<true, kStorageMajor>),
-                         dim3(grid), dim3(kThreads), glds, stream, F, side, side_wgs);
-    } else if (order == kAllStorages) {
-      hipLaunchKernelGGL((block_copy_fast_side_kernel<false, kAllStorages>),
-                         dim3(grid), dim3(kThreads), 0, stream, F, side, side_wgs);
-    } else {
-      hipLaunchKernelGGL((block_copy_fast_side_kernel<false, kStorageMajor>),
-                         dim3(grid), dim3(kThreads), 0, stream, F, side, side_wgs);
+  // The kernels with the small-block path take the same cap (not the capped
+  // grids of zero-copy copies), minus that path's own 4 KiB of address tables.
+  to.lds = to.lds > 0 && !capped_grid ? to.lds - kStaticLds : 0;
+  if (BuildFastSideParams(P, dir, &F, &FS.side, &FS.side_wgs, &order)) {
+    split(grid - FS.side_wgs);
+    if (gather) {
+      return order == kStoragePairs ? to.template FastSide<true, kStoragePairs>(FS)
+                                    : to.template FastSide<true, kStorageMajor>(FS);
     }
-    return hipGetLastError();
+    return order == kAllStorages ? to.template FastSide<false, kAllStorages>(FS)
+                                 : to.template FastSide<false, kStorageMajor>(FS);
   }
-  switch (whole_vec) {
-    case 16: return LaunchGeneral<16>(P, grid, dir, glds, stream);
-    case 4: return LaunchGeneral<4>(P, grid, dir, glds, stream);
-    default: return LaunchGeneral<1>(P, grid, dir, glds, stream);
+  if constexpr (kCap == 0) {
+    if (whole_vec == 4) return to.template General<4>(P, gather);
+    if (whole_vec == 1) return to.template General<1>(P, gather);
   }
+  return to.template General<16>(P, gather);
 }
 
 }  // namespace
@@ -776,7 +837,14 @@ hipError_t LaunchBlockCopy(const CopyLaunch& l, CopyDir dir, int vec_bytes,
   }
   const int cap = l.gather_workgroups_per_cu;
   if (vec_bytes != 16 && vec_bytes != 4 && vec_bytes != 1) return hipErrorInvalidValue;
-  return Launch(P, grid, dir, cap, l.max_workgroups > 0, Paged(l) ? vec_bytes : 16, stream);
+  const bool capped = l.max_workgroups > 0;
+  if (l.ids == nullptr && l.n <= kFewInlineIds) {
+    return Launch<kFewInlineIds>(P, l.inline_ids, grid, dir, cap, capped, 16, stream);
+  }
+  if (l.ids == nullptr) {
+    return Launch<kMaxInlineIds>(P, l.inline_ids, grid, dir, cap, capped, 16, stream);
+  }
+  return Launch<0>(P, nullptr, grid, dir, cap, capped, Paged(l) ? vec_bytes : 16, stream);
 }
 
 }  // namespace kvx
