@@ -1140,3 +1140,80 @@ def test_gather_scatter_around_the_inline_id_limits(kvx, cuda, n):
             for w, p in enumerate(pools):
                 assert np.array_equal(p.cpu().numpy(), pools_np[w]), (sizes, layer, w)
         mgr.close()
+
+
+# Launches above 160 MiB of whole-KiB blocks go sliced: one whole group of 32
+# ids, with 1 and 31 ids more, several groups; the smallest and largest blocks
+# each way, an odd number of KiB, a side table before the payload.
+SLICED = [(2048, 160, 544, 0), (3072, 130, 481, 0), (4096, 160, 351, 4), (16384, 330, 33, 0),
+          (16384, 160, 95, 32), (33 << 10, 164, 63, 0), (32768, 164, 32, 0),
+          (256 << 10, 22, 40, 0), (1 << 20, 6, 33, 0)]
+
+
+@pytest.mark.parametrize("block,storages,n,side", SLICED, ids=[str(c) for c in SLICED])
+def test_sliced_launches_move_the_same_blocks(kvx, cuda, block, storages, n, side):
+    """Gather and scatter against torch's own indexing, both staging orders
+    (layer-major with a side table), every byte outside the blocks unchanged."""
+    assert block * storages * n >= 160 << 20
+    gen = torch.Generator(device=cuda).manual_seed(block + n)
+    P = n + 9
+
+    def words(count):
+        return torch.randint(-2**31, 2**31 - 1, (count,), dtype=torch.int32, device=cuda,
+                             generator=gen)
+
+    pool = words(storages * P * block // 4).view(storages, P, block // 4)
+    tabs = words(storages * P * side // 4).view(storages, P, side // 4) if side else None
+    mgr = kvx.KVCacheManager([pool[w] for w in range(storages)], host_blocks_to_allocate=1,
+                             scale_tables=[tabs[w] for w in range(storages)] if side else None)
+    ids = torch.randperm(P, device=cuda, generator=gen)[:n]
+    for block_major in ((False,) if side else (False, True)):
+        def image(a, b):
+            x = a[:, ids]
+            x = x.transpose(0, 1).contiguous() if block_major else x
+            return torch.cat([x.reshape(-1)] + ([b[:, ids].reshape(-1)] if side else []))
+
+        staging = torch.zeros(storages * n * (block + side) // 4, dtype=torch.int32, device=cuda)
+        mgr.gather(ids.tolist(), staging, block_major=block_major).Await()
+        assert torch.equal(staging, image(pool, tabs))
+        new = words(staging.numel())
+        want_pool, want_tabs = pool.clone(), tabs.clone() if side else None
+        cut = storages * n * block // 4
+        part = new[:cut].view(n, storages, -1).transpose(0, 1) if block_major else \
+            new[:cut].view(storages, n, -1)
+        want_pool[:, ids] = part
+        if side:
+            want_tabs[:, ids] = new[cut:].view(storages, n, -1)
+        mgr.scatter(ids.tolist(), new, block_major=block_major).Await()
+        assert torch.equal(pool, want_pool)
+        assert not side or torch.equal(tabs, want_tabs)
+    mgr.close()
+
+
+@pytest.mark.parametrize("gather", [True, False])
+def test_sliced_launch_skips_and_flags_bad_ids(kvx, cuda, gather):
+    """Bad ids in a whole group and among a storage's last ids: their blocks
+    and staging stay as they were, every other block moves, the flag is set."""
+    import ctypes
+    S, P, n, words = 96, 70, 61, 32768 // 4
+    pool = torch.arange(S * P * words, dtype=torch.int32, device=cuda).view(S, P, words)
+    staging = torch.full((S, n, words), -5, dtype=torch.int32, device=cuda)
+    table = torch.tensor([pool[w].data_ptr() for w in range(S)], dtype=torch.int64, device=cuda)
+    ids = torch.randperm(P, device=cuda)[:n].to(torch.int64)
+    bad = [3, 31, 40, 60]
+    ids[bad] = torch.tensor([P, -1, 1 << 40, -(1 << 62)], device=cuda)
+    good = [i for i in range(n) if i not in bad]
+    flag = torch.zeros(1, dtype=torch.int32, device=cuda)
+    want_pool, want_staging = pool.clone(), staging.clone()
+    if gather:
+        want_staging[:, good] = pool[:, ids[good]]
+    else:
+        want_pool[:, ids[good]] = staging[:, good]
+    lib, u64 = kvx._capi.load(), ctypes.c_uint64
+    fn = lib.kvx_gather_blocks if gather else lib.kvx_scatter_blocks
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert fn(u64(table.data_ptr()), S, 32768, P, u64(ids.data_ptr()), n,
+              u64(staging.data_ptr()), 0, u64(flag.data_ptr()), stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(pool, want_pool) and torch.equal(staging, want_staging)
+    assert flag.item() == 1

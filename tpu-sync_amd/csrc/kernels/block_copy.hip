@@ -1,9 +1,11 @@
 // Paged-KV block gather/scatter for gfx950 (MI355X).
 //
 // Pure data movement, bound by HBM bandwidth: no MFMA, no LDS on the data
-// itself. Blocks of >= 8 KiB get one 256-lane workgroup each (four wave64s);
-// every lane keeps kUnroll independent 16-byte loads in flight before it
-// stores, which is what saturates HBM on a streaming copy. The block id and
+// itself. Every lane of a 256-lane workgroup (four wave64s) keeps kUnroll
+// independent 16-byte loads in flight before it stores, which is what saturates
+// HBM on a streaming copy. Large launches of blocks that are whole KiB go in
+// slices of many blocks to a workgroup; otherwise blocks of >= 16 KiB get a
+// workgroup each. The block id and
 // the storage base are workgroup-uniform, so the compiler reads them with
 // scalar loads into SGPRs: the id table is read once per block, broadcast
 // through SGPRs instead of an LDS round trip and barrier. Smaller blocks (one
@@ -25,6 +27,7 @@
 // an optional device flag; no lane ever forms an address from one.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 
@@ -204,7 +207,7 @@ __device__ __forceinline__ bool bad_id(int64_t id, int64_t limit) {
 template <int V, int kSteps>
 __device__ __forceinline__ void move_small(const uint64_t* s_src, const uint64_t* s_dst,
                                            uint32_t total, uint32_t elems, uint64_t magic,
-                                           uint64_t bytes) {
+                                           uint32_t bytes) {
   typename VecT<V>::T r[kSteps];
   uint64_t dst[kSteps];
 #pragma unroll
@@ -214,7 +217,7 @@ __device__ __forceinline__ void move_small(const uint64_t* s_src, const uint64_t
     e = in ? e : total - 1;
     const uint32_t b = static_cast<uint32_t>((e * magic) >> 32);
     const uint32_t sub = e - b * elems;
-    const uint64_t off = sub + 1 < elems ? static_cast<uint64_t>(sub) * V : bytes - V;
+    const uint32_t off = sub + 1 < elems ? sub * V : bytes - V;
     r[u] = ld<V>(s_src[b], off);
     const uint64_t d = s_dst[b];
     dst[u] = in && d != 0 ? d + off : 0;
@@ -227,13 +230,14 @@ __device__ __forceinline__ void move_small(const uint64_t* s_src, const uint64_t
 
 template <int V>
 __device__ __forceinline__ void move_small_blocks(const uint64_t* s_src, const uint64_t* s_dst,
-                                                  uint32_t total, const KPiece& p) {
+                                                  uint32_t total, uint32_t elems,
+                                                  uint64_t magic, uint32_t bytes) {
   if (total > 4 * kThreads) {
-    move_small<V, 8>(s_src, s_dst, total, p.elems, p.magic, p.bytes);
+    move_small<V, 8>(s_src, s_dst, total, elems, magic, bytes);
   } else if (total > kThreads) {
-    move_small<V, 4>(s_src, s_dst, total, p.elems, p.magic, p.bytes);
+    move_small<V, 4>(s_src, s_dst, total, elems, magic, bytes);
   } else {
-    move_small<V, 1>(s_src, s_dst, total, p.elems, p.magic, p.bytes);
+    move_small<V, 1>(s_src, s_dst, total, elems, magic, bytes);
   }
 }
 
@@ -242,14 +246,16 @@ __device__ __forceinline__ void move_small_blocks(const uint64_t* s_src, const u
 // loads, one block per lane, and stages each block's source and destination
 // address in LDS, so that no lane waits on a chain of dependent table loads
 // before its data loads. A bad id gets no destination and a source that can
-// be read. b0: the workgroup's first block of the piece. Bound by HBM: 768 random
+// be read. g: the workgroup's number in the piece. Bound by HBM: 768 random
 // 4 KiB blocks of 160 storages gathered in 177 us (5.7 TB/s; 242 with one
 // vector in flight a lane), 2 KiB blocks with a 4-byte scale per (layer, block)
 // scattered in 95 us (114 at the scales' 4-byte vectors for the whole launch).
 template <bool kGather, int kCap>
 __device__ __forceinline__ void copy_small_blocks(const KPiece& p, uint64_t ids,
                                                   const int64_t* ids2, int32_t* error,
-                                                  uint32_t n, uint32_t b0) {
+                                                  uint32_t n, uint32_t g) {
+  const uint32_t b0 = g * p.bpw;
+  const uint32_t bytes = static_cast<uint32_t>(p.bytes);
   __shared__ uint64_t s_src[kSmallMaxBlocks];
   __shared__ uint64_t s_dst[kSmallMaxBlocks];
   const uint32_t left = p.nblocks - b0;
@@ -280,11 +286,11 @@ __device__ __forceinline__ void copy_small_blocks(const KPiece& p, uint64_t ids,
   __syncthreads();
   const uint32_t total = nb * p.elems;
   switch (p.vec) {
-    case 16: move_small_blocks<16>(s_src, s_dst, total, p); break;
-    case 8: move_small_blocks<8>(s_src, s_dst, total, p); break;
-    case 4: move_small_blocks<4>(s_src, s_dst, total, p); break;
-    case 2: move_small_blocks<2>(s_src, s_dst, total, p); break;
-    default: move_small_blocks<1>(s_src, s_dst, total, p); break;
+    case 16: move_small_blocks<16>(s_src, s_dst, total, p.elems, p.magic, bytes); break;
+    case 8: move_small_blocks<8>(s_src, s_dst, total, p.elems, p.magic, bytes); break;
+    case 4: move_small_blocks<4>(s_src, s_dst, total, p.elems, p.magic, bytes); break;
+    case 2: move_small_blocks<2>(s_src, s_dst, total, p.elems, p.magic, bytes); break;
+    default: move_small_blocks<1>(s_src, s_dst, total, p.elems, p.magic, bytes); break;
   }
 }
 
@@ -294,10 +300,10 @@ __global__ __launch_bounds__(kThreads) void block_copy_kernel(Args<KParams, kCap
   const uint32_t wg = blockIdx.x;
   const uint64_t ids = ids_address<KParams, kCap>(P.ids);
   const KPiece p = select_piece(P, wg);
-  const uint32_t b0 = (wg - p.wg_begin) * p.bpw;
   const uint32_t n = P.n;
 
   if (p.whole) {
+    const uint32_t b0 = (wg - p.wg_begin) * p.bpw;
     // All lanes move one block at a time; the workgroup walks a run of
     // consecutive flat blocks (one block unless the grid is capped).
     const uint32_t left = p.nblocks - b0;
@@ -333,7 +339,7 @@ __global__ __launch_bounds__(kThreads) void block_copy_kernel(Args<KParams, kCap
     return;
   }
 
-  copy_small_blocks<kGather, kCap>(p, ids, P.ids2, P.error, n, b0);
+  copy_small_blocks<kGather, kCap>(p, ids, P.ids2, P.error, n, wg - p.wg_begin);
 }
 
 // The common launch (one piece of large blocks, no second paged side, one
@@ -425,100 +431,136 @@ __global__ __launch_bounds__(kThreads) void block_copy_fast_kernel(Args<FastPara
   fast_block<kGather, kOrder, kCap>(args.p, ids_address<FastParams, kCap>(args.p.ids), blockIdx.x);
 }
 
-// Sliced form of the fast gather, for blocks of exactly one pass (kUnroll *
-// kThreads vectors: 32 KiB at 16-byte vectors) over an even number of whole
-// storages: workgroup g moves slice g mod 2^kLog2H of each of 2^kLog2H
-// consecutive ids of one storage, the slices of those blocks on consecutive
-// workgroups, and storages in the fast gather's pairs order with id groups
-// in place of ids. The bytes and where they land are those of the fast
-// kernel; only the set a workgroup moves at once differs. Measured on MI355X
-// (512 random ids over 64 storages of 16384 blocks, 2 GiB per launch, in one
-// process alternating with the fast kernel, four machines): 4 slices +0.9 to
-// +2.2 points of HBM bandwidth (e.g. 75.2 against 73.9 %). The same form for
-// the scatter (8 slices, all-storages order) measured -1.5 to +1.7 points
-// and is not used.
-template <int kLog2H, int kCap>
-__global__ __launch_bounds__(kThreads) void block_copy_sliced_gather_kernel(
-    Args<FastParams, kCap> args) {
-  const FastParams& P = args.p;
-  const uint64_t ids = ids_address<FastParams, kCap>(P.ids);
+// Blocks of a whole number of KiB over whole storages, in slices: a wave moves
+// 1 KiB slices of up to 8 blocks with consecutive ids, a workgroup one slice of
+// 32 blocks of one storage, and consecutive workgroups the other slices of those
+// blocks. A workgroup's bytes are thus short pieces of many blocks, which the
+// random side's DRAM serves better than one block at a time. Bound by HBM, per
+// launch: 512 random 32 KiB blocks of 64 storages gathered in 336 us and
+// scattered in 366 (a whole block to a workgroup: 356, sliced in four, and 390),
+// 768 x 160 of 4 KiB gathered in 163 (packed: 177), 0.54 GB of 8 KiB blocks
+// gathered in 172 and scattered in 181 (a workgroup a block: 197 and 214).
+// The last ids of a storage (fewer than 32) are cut the same way, slices of 1 KiB
+// with the id running fastest, 32 to a workgroup, so that every workgroup is full.
+// The ids and the base are scalar loads, all in flight at once; nothing goes
+// through LDS. A side piece (a scale table) takes the first workgroups.
+constexpr uint32_t kSliceBytes = 1024;                      // 64 lanes x 16 bytes
+constexpr uint32_t kSlices = kUnroll * (kThreads / 64);     // slices per workgroup
+struct SlicedParams {
+  uint64_t storages;
+  uint64_t staging;
+  const int64_t* ids;
+  int32_t* error;
+  int64_t stride_w;
+  int64_t stride_i;
+  int64_t pool_blocks;
+  uint64_t bytes;      // bytes per block
+  uint32_t n;
+  uint32_t w0;         // first storage
+  uint32_t slices;       // slices per block (gridDim.x)
+  uint32_t side_wgs;     // workgroups of the side piece and, after them, of
+  uint32_t last_wgs;     // every storage's last ids, in the first extra_planes
+  uint32_t extra_planes; // values of blockIdx.z
+  uint32_t last_per;     // workgroups of one storage's last ids
+  KPiece side;
+};
+
+template <bool kGather, int kCap>
+__global__ __launch_bounds__(kThreads) void block_copy_sliced_kernel(
+    Args<SlicedParams, kCap> args) {
   constexpr int V = 16;
-  constexpr uint32_t kH = 1u << kLog2H;
-  constexpr uint32_t kSlice = kUnroll * kThreads / kH;  // vectors per slice
-  // Each unrolled step's kThreads vectors lie in one slice of one block, so
-  // a step's block (and its id) is the same for the whole workgroup.
-  static_assert(kSlice % kThreads == 0, "a step must stay in one slice");
-  constexpr uint32_t kSteps = kSlice / kThreads;  // steps per block
-  uint32_t g = blockIdx.x;
-  const uint32_t cc = g & (kH - 1);
-  g >>= kLog2H;
-  const uint32_t groups = (P.n + kH - 1) >> kLog2H;
-  const uint32_t q = g / (2 * groups);
-  const uint32_t r2 = g - q * 2 * groups;
-  const uint32_t ig = r2 >> 1;
-  const uint32_t w = P.w0 + 2 * q + (r2 & 1);
-  const uint64_t base = uniform_load<uint64_t>(P.storages, w);
-  const uint64_t stg0 = P.staging + w * static_cast<uint64_t>(P.stride_w);
-  // The group's ids (the last group of a launch may hold fewer than kH); a
-  // missing or bad id moves nothing, and a bad one sets the error flag.
-  uint64_t pool_at[kH], stg_at[kH];
-  bool ok[kH];
-  bool bad_any = false;
-#pragma unroll
-  for (uint32_t r = 0; r < kH; ++r) {
-    const uint32_t i = (ig << kLog2H) + r;
-    const bool in = i < P.n;
-    const int64_t id = in ? uniform_id<kCap>(ids, i) : 0;
-    const bool bad = in && bad_id(id, P.pool_blocks);
-    ok[r] = in && !bad;
-    bad_any |= bad;
-    pool_at[r] = base + static_cast<uint64_t>(ok[r] ? id : 0) * P.bytes;
-    stg_at[r] = stg0 + i * static_cast<uint64_t>(P.stride_i);
+  const SlicedParams& P = args.p;
+  const uint64_t ids = ids_address<SlicedParams, kCap>(P.ids);
+  uint32_t wl = blockIdx.z - P.extra_planes;  // the storage
+  uint32_t last = 0;                          // workgroup of its last ids
+  const bool whole = blockIdx.z >= P.extra_planes;
+  if (!whole) {
+    uint32_t g = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    if (g < P.side_wgs) {
+      copy_small_blocks<kGather, kCap>(P.side, ids, nullptr, P.error, P.n, g);
+      return;
+    }
+    g -= P.side_wgs;
+    if (g >= P.last_wgs) return;
+    wl = g / P.last_per;
+    last = g - wl * P.last_per;
   }
-  bool all_ok = true;
+  const uint32_t w = P.w0 + wl;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const uint32_t lane = (threadIdx.x % 64) * V;
+  // The group's first id.
+  const uint32_t first = whole ? blockIdx.y * kSlices : P.n / kSlices * kSlices;
+  const uint64_t stg_w = P.staging + w * static_cast<uint64_t>(P.stride_w);
+  typename VecT<V>::T v[kUnroll];
+  uint64_t pool_at[kUnroll], stg_at[kUnroll];
+  bool ok[kUnroll];
+  bool all_ok = true, any_bad = false;
+  if (whole) {
+    const uint32_t i0 = first + wave * kUnroll;
+    const uint32_t off = blockIdx.x * kSliceBytes;
+    const uint64_t base = uniform_load<uint64_t>(P.storages, w) + off;
+    const uint64_t stg = stg_w + i0 * static_cast<uint64_t>(P.stride_i) + off;
 #pragma unroll
-  for (uint32_t r = 0; r < kH; ++r) all_ok = all_ok && ok[r];
-  const uint32_t lane0 = cc * kSlice + threadIdx.x;
+    for (uint32_t u = 0; u < kUnroll; ++u) {
+      const int64_t id = uniform_id<kCap>(ids, i0 + u);
+      ok[u] = !bad_id(id, P.pool_blocks);
+      all_ok = all_ok && ok[u];
+      pool_at[u] = base + static_cast<uint64_t>(ok[u] ? id : 0) * P.bytes;
+      stg_at[u] = stg + u * static_cast<uint64_t>(P.stride_i);
+    }
+    any_bad = !all_ok;
+  } else {
+    // Unit k of the last `many` ids is slice k / many of id k % many.
+    const uint32_t many = P.n - first;
+    const uint32_t units = many * P.slices;
+    const uint32_t k = last * kSlices + wave * kUnroll;
+    if (k >= units) return;
+    const uint64_t base = uniform_load<uint64_t>(P.storages, w);
+    // Places first, then every id load, so that none waits for another; past
+    // the end the last unit repeats.
+    uint32_t id_at[kUnroll], off[kUnroll];
+    uint32_t slice = k / many;
+    uint32_t i = k - slice * many;
+#pragma unroll
+    for (uint32_t u = 0; u < kUnroll; ++u) {
+      id_at[u] = first + i;
+      off[u] = slice * kSliceBytes;
+      const bool more = k + u + 1 < units;
+      const bool wrap = i + 1 == many;
+      i = more ? (wrap ? 0 : i + 1) : i;
+      slice = more && wrap ? slice + 1 : slice;
+    }
+    int64_t id[kUnroll];
+#pragma unroll
+    for (uint32_t u = 0; u < kUnroll; ++u) id[u] = uniform_id<kCap>(ids, id_at[u]);
+#pragma unroll
+    for (uint32_t u = 0; u < kUnroll; ++u) {
+      const bool in = k + u < units;
+      const bool bad = bad_id(id[u], P.pool_blocks);
+      ok[u] = in && !bad;
+      all_ok = all_ok && ok[u];
+      any_bad = any_bad || (in && bad);
+      pool_at[u] = base + static_cast<uint64_t>(bad ? 0 : id[u]) * P.bytes + off[u];
+      stg_at[u] = stg_w + id_at[u] * static_cast<uint64_t>(P.stride_i) + off[u];
+    }
+  }
   if (all_ok) {
-    // Every step's load issued before the first store, as in the fast kernel.
-    typename VecT<V>::T v[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const uint32_t r = u / kSteps;
-      const uint32_t k = lane0 + (u % kSteps) * kThreads;
-      v[u] = ld<V>(pool_at[r], k * V);
-    }
+    for (uint32_t u = 0; u < kUnroll; ++u) v[u] = ld<V>(kGather ? pool_at[u] : stg_at[u], lane);
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const uint32_t r = u / kSteps;
-      const uint32_t k = lane0 + (u % kSteps) * kThreads;
-      st<V>(v[u], stg_at[r], k * V);
-    }
+    for (uint32_t u = 0; u < kUnroll; ++u) st<V>(v[u], kGather ? stg_at[u] : pool_at[u], lane);
     return;
   }
-  // The last group of a launch, or a group with a bad id: block by block.
-  for (uint32_t r = 0; r < kH; ++r) {
-    if (!ok[r]) continue;
-    for (uint32_t t = 0; t < kSteps; ++t) {
-      const uint32_t k = lane0 + t * kThreads;
-      st<V>(ld<V>(pool_at[r], k * V), stg_at[r], k * V);
-    }
+  // Fewer than 8 units, or a bad id.
+#pragma unroll
+  for (uint32_t u = 0; u < kUnroll; ++u) {
+    if (ok[u]) v[u] = ld<V>(kGather ? pool_at[u] : stg_at[u], lane);
   }
-  if (bad_any && threadIdx.x == 0 && P.error != nullptr) atomicOr(P.error, 1);
-}
-
-// Slices per block (log2) of a sliced gather, 0 when the launch goes to the
-// fast kernel: blocks of exactly one pass, an even number of whole storages
-// (the pairs order), an uncapped grid that fits.
-constexpr int kGatherLog2Slices = 2;
-int SlicedGatherLog2(const FastParams& F, CopyDir dir, int order, bool capped_grid) {
-  if (dir != CopyDir::kGather || order != kStoragePairs) return 0;
-  if (capped_grid || F.pieces != 1 || F.rest != 0) return 0;
-  if (F.elems != static_cast<uint32_t>(kUnroll * kThreads)) return 0;
-  const uint64_t groups =
-      (static_cast<uint64_t>(F.n) + (1u << kGatherLog2Slices) - 1) >> kGatherLog2Slices;
-  if ((groups << kGatherLog2Slices) * F.wstorages > INT32_MAX) return 0;
-  return kGatherLog2Slices;
+#pragma unroll
+  for (uint32_t u = 0; u < kUnroll; ++u) {
+    if (ok[u]) st<V>(v[u], kGather ? stg_at[u] : pool_at[u], lane);
+  }
+  if (any_bad && threadIdx.x % 64 == 0 && P.error != nullptr) atomicOr(P.error, 1);
 }
 
 // The fast launch behind one leading small-block piece: the fp8 payload and
@@ -537,20 +579,29 @@ __global__ __launch_bounds__(kThreads) void block_copy_fast_side_kernel(
   const FastSideParams& P = args.p;
   const uint64_t ids = ids_address<FastSideParams, kCap>(P.fast.ids);
   if (blockIdx.x < P.side_wgs) {
-    copy_small_blocks<kGather, kCap>(P.side, ids, nullptr, P.fast.error, P.fast.n,
-                                     blockIdx.x * P.side.bpw);
+    copy_small_blocks<kGather, kCap>(P.side, ids, nullptr, P.fast.error, P.fast.n, blockIdx.x);
     return;
   }
   fast_block<kGather, kOrder, kCap>(P.fast, ids, blockIdx.x - P.side_wgs);
 }
 
-// Blocks per workgroup: one for blocks of >= 2 vectors per lane, otherwise
-// enough blocks to give each lane up to 8 vectors, at most kSmallMaxBlocks.
+// Two workgroups on each of the 256 CUs.
+constexpr uint64_t kFillWorkgroups = 512;
+
+// Packed blocks per workgroup: enough to give each lane up to 8 vectors, at most
+// kSmallMaxBlocks.
 uint32_t BlocksPerWorkgroup(uint64_t elems) {
-  if (elems >= 2 * kThreads) return 1;
   uint64_t bpw = (8 * kThreads) / (elems == 0 ? 1 : elems);
   if (bpw > kSmallMaxBlocks) bpw = kSmallMaxBlocks;
   return static_cast<uint32_t>(bpw < 1 ? 1 : bpw);
+}
+
+// Whether a block of `elems` vectors goes whole to a workgroup (else packed).
+// Between device buffers that is one of 4 and more vectors a lane (16 KiB):
+// packed, 10 KB blocks of 64 storages gather 190 against 236 us and scatter 208
+// against 225 (0.54 GB a launch).
+bool WholeBlock(uint64_t elems, bool paged) {
+  return elems >= (paged ? 2 : 4) * kThreads;
 }
 
 // Whether a piece's other side is a second paged buffer (host memory that the
@@ -589,17 +640,16 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
   for (int k = 0; k < l.npieces; ++k) {
     total_blocks += static_cast<uint64_t>(l.pieces[k].nblocks > 0 ? l.pieces[k].nblocks : 0);
   }
-  // Small-block pieces (side tables) take the first workgroups, so their
+  // Pieces of smaller blocks (side tables) take the first workgroups, so their
   // few workgroups run alongside the large blocks instead of after them.
   int order[kMaxPieces];
-  int norder = 0;
-  for (int pass = 0; pass < 2; ++pass) {
-    for (int k = 0; k < l.npieces; ++k) {
-      const int64_t bb = l.pieces[k].block_bytes;
-      if (bb <= 0) return false;
-      const bool whole = static_cast<uint64_t>(bb) / vec_of(bb) >= 2 * kThreads;
-      if (whole == (pass == 1)) order[norder++] = k;
+  for (int k = 0; k < l.npieces; ++k) {
+    if (l.pieces[k].block_bytes <= 0) return false;
+    int at = k;
+    for (; at > 0 && l.pieces[order[at - 1]].block_bytes > l.pieces[k].block_bytes; --at) {
+      order[at] = order[at - 1];
     }
+    order[at] = k;
   }
   uint64_t wg = 0;
   for (int slot = 0; slot < l.npieces; ++slot) {
@@ -619,9 +669,15 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
     const uint64_t bytes = static_cast<uint64_t>(c.block_bytes);
     const uint64_t vec = vec_of(bytes);
     uint64_t elems = bytes / vec;
-    const bool whole = elems >= 2 * kThreads;
+    const bool whole = WholeBlock(elems, paged);
     if (!whole && bytes % vec != 0) ++elems;
-    uint64_t bpw = BlocksPerWorkgroup(elems);
+    uint64_t bpw = whole ? 1 : BlocksPerWorkgroup(elems);
+    // A launch that does not fill the chip has fewer vectors a lane instead (16
+    // x 160 blocks of 4 KiB gathered in 6.5 against 7.3 us).
+    while (!whole && !paged && bpw > 1 && bpw * elems > kThreads &&
+           static_cast<uint64_t>(c.nblocks) < bpw * kFillWorkgroups) {
+      bpw /= 2;
+    }
     if (whole && l.max_workgroups > 0) {
       // This piece's share of the workgroup cap, at least one.
       uint64_t share = static_cast<uint64_t>(l.max_workgroups) *
@@ -630,7 +686,7 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
       const uint64_t need = (static_cast<uint64_t>(c.nblocks) + share - 1) / share;
       if (need > bpw) bpw = need;
     }
-    if (bpw > UINT32_MAX || (!whole && bpw * elems > UINT32_MAX)) return false;
+    if (bpw > UINT32_MAX) return false;
     KPiece& kp = P->p[slot];
     kp.storages = c.storages;
     kp.staging = c.staging;
@@ -706,8 +762,71 @@ bool BuildFastSideParams(const KParams& K, CopyDir dir, FastParams* F, KPiece* s
   return true;
 }
 
+// Slices of a block when a launch goes sliced, else 0: blocks of 2 KiB and more
+// that are whole KiB, over whole storages, at least one group of 32 ids. Launches
+// whose two sides fit the 256 MB last-level cache have no DRAM order to gain
+// from and keep the other kernels (64 x 64 blocks of 32 KiB scattered in 46.6 us
+// against 48.4 sliced, 256 x 160 of 4 KiB, at the line, in 65.0 against 62.6);
+// gathers of 512 KiB blocks measured 185 us whole and 192 sliced (0.54 GB), 256
+// KiB ones 184 and 177, scatters up to 1 MiB 193 and 184.
+constexpr uint64_t kSlicedMinBytes = 160 << 20;
+uint32_t SlicesOf(const KPiece& p, uint32_t n, CopyDir dir) {
+  if (p.others != 0 || p.bytes % kSliceBytes != 0 || p.bytes < 2 * kSliceBytes) return 0;
+  if (p.bytes > (dir == CopyDir::kGather ? 256u << 10 : 1u << 20)) return 0;
+  if (n < kSlices || p.f0 % n != 0 || p.nblocks % n != 0) return 0;
+  if (p.bytes * p.nblocks < kSlicedMinBytes) return 0;
+  return static_cast<uint32_t>(p.bytes / kSliceBytes);
+}
+
+// The sliced launch of one piece, or of one behind a side piece of smaller
+// blocks; *grid receives its workgroups.
+bool BuildSlicedParams(const KParams& K, CopyDir dir, SlicedParams* S, dim3* grid) {
+  if (K.npieces > 2) return false;
+  const KPiece& p = K.p[K.npieces - 1];
+  const uint32_t slices = SlicesOf(p, K.n, dir);
+  if (slices == 0) return false;
+  if (K.npieces == 2 && (K.p[0].whole || K.p[0].others != 0)) return false;
+  *S = SlicedParams{};
+  S->storages = p.storages;
+  S->staging = p.staging;
+  S->ids = K.ids;
+  S->error = K.error;
+  S->stride_w = p.stride_w;
+  S->stride_i = p.stride_i;
+  S->pool_blocks = p.pool_blocks;
+  S->bytes = p.bytes;
+  S->n = K.n;
+  S->w0 = p.f0 / K.n;
+  S->slices = slices;
+  // Slices, id groups, storages: the grid's dimensions, so that a workgroup
+  // divides nothing to find its place (two divisions cost a gather 4 %: 0.54 GB
+  // of 32 KiB blocks in 176.5 against 169.6 us). The side piece and the last ids
+  // of the storages fill planes of their own before them.
+  const uint64_t W = p.nblocks / K.n;
+  const uint64_t groups = K.n / kSlices;
+  const uint64_t per_plane = slices * groups;
+  S->last_per = (K.n % kSlices * slices + kSlices - 1) / kSlices;
+  const uint64_t last_wgs = W * S->last_per;
+  if (K.npieces == 2) {
+    S->side = K.p[0];
+    S->side_wgs = K.p[1].wg_begin;
+  }
+  const uint64_t extra = (S->side_wgs + last_wgs + per_plane - 1) / per_plane;
+  const uint64_t planes = extra + W;
+  S->last_wgs = static_cast<uint32_t>(last_wgs);
+  S->extra_planes = static_cast<uint32_t>(extra);
+  if (groups > 65535 || planes > 65535 || per_plane * planes > INT32_MAX) return false;
+  *grid = dim3(slices, static_cast<uint32_t>(groups), static_cast<uint32_t>(planes));
+  return true;
+}
+
 // LDS of one CU on gfx950.
 constexpr uint32_t kLdsPerCu = 160u << 10;
+
+// Launches of the packed and sliced kernels with fewer workgroups than this are
+// not capped: they would run in a few unequal rounds (20 MB of 2 KiB blocks
+// scattered in 9.7 us capped, 8.6 not).
+constexpr uint32_t kCapGrid = 2048;
 
 // LDS the general kernel declares (the small-block path's address tables).
 constexpr uint32_t kStaticLds = 2 * kSmallMaxBlocks * sizeof(uint64_t);
@@ -722,7 +841,7 @@ template <int kCap>
 struct Launcher {
   const uint32_t* inline_ids;
   uint32_t n;
-  uint32_t grid;
+  dim3 grid;
   uint32_t lds;
   hipStream_t stream;
 
@@ -731,7 +850,7 @@ struct Launcher {
     Args<P, kCap> a{};
     a.p = p;
     if constexpr (kCap > 0) std::memcpy(a.ids, inline_ids, n * sizeof(uint32_t));
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, a);
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), lds, stream, a);
     return hipGetLastError();
   }
   template <bool kGather, int kOrder>
@@ -755,7 +874,7 @@ hipError_t Launch(const KParams& P, const uint32_t* inline_ids, uint32_t grid, C
                   int wg_per_cu, bool capped_grid, int whole_vec, hipStream_t stream) {
   const bool gather = dir == CopyDir::kGather;
   // Gathers reserve (unused) LDS to cap their workgroups per CU.
-  Launcher<kCap> to{inline_ids, P.n, grid, 0, stream};
+  Launcher<kCap> to{inline_ids, P.n, dim3(grid), 0, stream};
   if (gather && wg_per_cu > 0) to.lds = kLdsPerCu / static_cast<uint32_t>(wg_per_cu);
   FastSideParams FS;
   FastParams& F = FS.fast;
@@ -767,18 +886,20 @@ hipError_t Launch(const KParams& P, const uint32_t* inline_ids, uint32_t grid, C
     const uint32_t pass = kUnroll * kThreads;
     if (capped_grid || F.elems <= pass) return;
     const uint64_t pieces = (static_cast<uint64_t>(F.elems) + pass - 1) / pass;
-    if (static_cast<uint64_t>(blocks) * pieces + (to.grid - blocks) > INT32_MAX) return;
+    if (static_cast<uint64_t>(blocks) * pieces + (to.grid.x - blocks) > INT32_MAX) return;
     F.pieces = static_cast<uint32_t>(pieces);
     F.piece_elems = pass;
-    to.grid = to.grid - blocks + blocks * F.pieces;
+    to.grid.x = to.grid.x - blocks + blocks * F.pieces;
   };
+  SlicedParams S;
+  if (!capped_grid && BuildSlicedParams(P, dir, &S, &to.grid)) {
+    to.lds = wg_per_cu > 0 && to.grid.x * to.grid.y * to.grid.z >= kCapGrid
+                 ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) - kStaticLds
+                 : 0;
+    return gather ? to.template Run<SlicedParams>(block_copy_sliced_kernel<true, kCap>, S)
+                  : to.template Run<SlicedParams>(block_copy_sliced_kernel<false, kCap>, S);
+  }
   if (BuildFastParams(P, dir, &F, &order)) {
-    const int s = SlicedGatherLog2(F, dir, order, capped_grid);
-    if (s > 0) {
-      to.grid = (((F.n + (1u << s) - 1) >> s) << s) * F.wstorages;
-      return to.template Run<FastParams>(
-          block_copy_sliced_gather_kernel<kGatherLog2Slices, kCap>, F);
-    }
     split(grid);
     if (gather) {
       return order == kStoragePairs ? to.template Fast<true, kStoragePairs>(F)
@@ -787,9 +908,13 @@ hipError_t Launch(const KParams& P, const uint32_t* inline_ids, uint32_t grid, C
     return order == kAllStorages ? to.template Fast<false, kAllStorages>(F)
                                  : to.template Fast<false, kStorageMajor>(F);
   }
-  // The kernels with the small-block path take the same cap (not the capped
-  // grids of zero-copy copies), minus that path's own 4 KiB of address tables.
-  to.lds = to.lds > 0 && !capped_grid ? to.lds - kStaticLds : 0;
+  // The kernels with the packed path take the same cap in both directions (not
+  // the capped grids of zero-copy copies), minus that path's own 4 KiB of address
+  // tables: 3 and 4 KiB blocks scattered in 152 and 198 us capped, 160 and 208
+  // not.
+  to.lds = wg_per_cu > 0 && !capped_grid && grid >= kCapGrid
+               ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) - kStaticLds
+               : 0;
   if (BuildFastSideParams(P, dir, &F, &FS.side, &FS.side_wgs, &order)) {
     split(grid - FS.side_wgs);
     if (gather) {
