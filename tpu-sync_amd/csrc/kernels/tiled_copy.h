@@ -169,9 +169,10 @@ uint32_t TiledPerWorkgroup(const TiledLaunchKey& k);
 
 // Launches the jobs of a device-resident image: the TiledJobDev array, the
 // general-path dimension arrays, then a workgroup -> job map of `grid`
-// uint32 at byte offset `map_offset`. Every job of the image has `key`.
-hipError_t LaunchTiledCopy(const void* image_dev, uint32_t map_offset, uint32_t grid,
-                           const TiledLaunchKey& key, hipStream_t stream);
+// uint32 at byte offset `map_offset`. Every job of the image has `key`. Or, with
+// `job` (not general), that one job, carried in the kernel's arguments.
+hipError_t LaunchTiledCopy(const void* image_dev, uint32_t map_offset, const TiledJobDev* job,
+                           uint32_t grid, const TiledLaunchKey& key, hipStream_t stream);
 
 }  // namespace kvx
 

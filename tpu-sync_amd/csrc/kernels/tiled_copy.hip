@@ -224,7 +224,7 @@ __device__ __forceinline__ void deinterleave(const uint32_t (&in)[P * n], uint32
 // of a row (the same tile row, so inside the job's range): with RAGGED rows (no
 // whole number of vectors) a unit whose columns run past W starts `back`
 // columns after that address. Whole rows keep a kernel without that handling
-// (one detile of a [14336, 4096] bf16 weight 52.7 us a call, 53.6 with it).
+// (one detile of a [14336, 4096] bf16 weight 0.9 us faster than with it).
 struct Unit {
   uint64_t tiled, lin;
   uint32_t h, c, back;
@@ -558,7 +558,7 @@ __device__ __forceinline__ void std_quad_detile(const KVX_CONST TiledJobDev* j, 
 // stay whole. Every global access of a wave is 256-byte rows on the linear
 // side and, at the tile widths in use (128), 512-byte or longer pieces on the
 // tiled side; regions along a linear row are consecutive.
-// Bound by HBM: a bf16 [4096, 14336] weight detiles in 55.6 us a call (floor 35
+// Bound by HBM: a bf16 [4096, 14336] weight detiles in 46.4 us a call (floor 35
 // at 6.7 TB/s), element by element in 901.
 template <int A, bool TILE>
 __device__ __forceinline__ void col_region(const KVX_CONST TiledJobDev* j, uint32_t region) {
@@ -764,12 +764,27 @@ __device__ __forceinline__ uint32_t xcd_item(uint32_t g, uint32_t n) {
   return (g % kXcds) * per + g / kXcds;
 }
 
-__device__ __forceinline__ const KVX_CONST TiledJobDev* job_of(const uint8_t* image,
-                                                               uint32_t map_offset,
+// A kernel's one argument: a device image of jobs with its workgroup -> job
+// map, or (image null) the launch's only job itself, which then needs no upload
+// before the kernel.
+struct TiledArgs {
+  const uint8_t* image;
+  uint64_t map_offset;
+  TiledJobDev job;
+};
+
+// The workgroup's job, and its number in the job.
+__device__ __forceinline__ const KVX_CONST TiledJobDev* job_of(const TiledArgs& args,
                                                                uint32_t* local) {
   const uint32_t wg = xcd_item(blockIdx.x, gridDim.x);
-  const uint32_t ji = ((const KVX_CONST uint32_t*)(image + map_offset))[wg];
-  const KVX_CONST TiledJobDev* j = (const KVX_CONST TiledJobDev*)image + ji;
+  if (args.image == nullptr) {
+    *local = wg;
+    return (const KVX_CONST TiledJobDev*)((const KVX_CONST uint8_t*)
+                                              __builtin_amdgcn_kernarg_segment_ptr() +
+                                          __builtin_offsetof(TiledArgs, job));
+  }
+  const uint32_t ji = ((const KVX_CONST uint32_t*)(args.image + args.map_offset))[wg];
+  const KVX_CONST TiledJobDev* j = (const KVX_CONST TiledJobDev*)args.image + ji;
   *local = wg - j->wg_begin;
   return j;
 }
@@ -777,10 +792,9 @@ __device__ __forceinline__ const KVX_CONST TiledJobDev* job_of(const uint8_t* im
 // LANES: lanes per unit; 2 for P = 2 and 4 for P = 4 when detiling at 16-byte
 // rows (through LDS), else 1.
 template <int V, int P, bool TILE, int LANES, bool RAGGED>
-__global__ __launch_bounds__(kThreads) void tiled_std_kernel(const uint8_t* image,
-                                                             uint32_t map_offset) {
+__global__ __launch_bounds__(kThreads) void tiled_std_kernel(TiledArgs args) {
   uint32_t local;
-  const KVX_CONST TiledJobDev* j = job_of(image, map_offset, &local);
+  const KVX_CONST TiledJobDev* j = job_of(args, &local);
   if constexpr (P == 1) {
     std_p1<V, TILE, RAGGED>(j, local);
   } else if constexpr (LANES == 2) {
@@ -795,26 +809,23 @@ __global__ __launch_bounds__(kThreads) void tiled_std_kernel(const uint8_t* imag
 }
 
 template <int A, bool TILE>
-__global__ __launch_bounds__(kThreads) void tiled_col_kernel(const uint8_t* image,
-                                                             uint32_t map_offset) {
+__global__ __launch_bounds__(kThreads) void tiled_col_kernel(TiledArgs args) {
   uint32_t local;
-  const KVX_CONST TiledJobDev* j = job_of(image, map_offset, &local);
+  const KVX_CONST TiledJobDev* j = job_of(args, &local);
   col_region<A, TILE>(j, local);
 }
 
 template <typename T, bool TILE>
-__global__ __launch_bounds__(kThreads) void tiled_gen_kernel(const uint8_t* image,
-                                                             uint32_t map_offset) {
+__global__ __launch_bounds__(kThreads) void tiled_gen_kernel(TiledArgs args) {
   uint32_t local;
-  const KVX_CONST TiledJobDev* j = job_of(image, map_offset, &local);
-  gen_job<T, TILE>(j, (const KVX_CONST TiledGenDim*)(image + j->gen_offset), local);
+  const KVX_CONST TiledJobDev* j = job_of(args, &local);
+  gen_job<T, TILE>(j, (const KVX_CONST TiledGenDim*)(args.image + j->gen_offset), local);
 }
 
 template <int V>
-__global__ __launch_bounds__(kThreads) void tiled_zero_kernel(const uint8_t* image,
-                                                              uint32_t map_offset) {
+__global__ __launch_bounds__(kThreads) void tiled_zero_kernel(TiledArgs args) {
   uint32_t local;
-  const KVX_CONST TiledJobDev* j = job_of(image, map_offset, &local);
+  const KVX_CONST TiledJobDev* j = job_of(args, &local);
   const uint64_t first = j->lo + static_cast<uint64_t>(local) * (kThreads * kVecsPerLane);
   const uint64_t end = j->lo + j->count;
   typename VecT<V>::T z{};
@@ -825,7 +836,7 @@ __global__ __launch_bounds__(kThreads) void tiled_zero_kernel(const uint8_t* ima
   }
 }
 
-typedef void (*KernelFn)(const uint8_t*, uint32_t);
+typedef void (*KernelFn)(TiledArgs);
 
 template <int V, int P, int LANES>
 KernelFn StdKernel(bool tile, bool ragged) {
@@ -931,12 +942,19 @@ uint32_t TiledPerWorkgroup(const TiledLaunchKey& k) {
   return kThreads * kVecsPerLane;
 }
 
-hipError_t LaunchTiledCopy(const void* image_dev, uint32_t map_offset, uint32_t grid,
-                           const TiledLaunchKey& key, hipStream_t stream) {
+hipError_t LaunchTiledCopy(const void* image_dev, uint32_t map_offset, const TiledJobDev* job,
+                           uint32_t grid, const TiledLaunchKey& key, hipStream_t stream) {
   if (grid == 0) return hipSuccess;
   const KernelFn fn = PickKernel(key);
   if (fn == nullptr) return hipErrorInvalidValue;
-  const uint8_t* img = static_cast<const uint8_t*>(image_dev);
+  TiledArgs args{};
+  if (job != nullptr) {
+    if (key.mode == kDetileGen || key.mode == kTileGen) return hipErrorInvalidValue;
+    args.job = *job;
+  } else {
+    args.image = static_cast<const uint8_t*>(image_dev);
+    args.map_offset = map_offset;
+  }
   // The bf16 Llama-3-8B set and a set of f32 matrices measured 1.3-3.4
   // points of HBM peak above no cap. The four-lane kernels' own LDS counts
   // towards the reservation.
@@ -945,7 +963,7 @@ hipError_t LaunchTiledCopy(const void* image_dev, uint32_t map_offset, uint32_t 
   const bool col = key.mode == kDetileCol || key.mode == kTileCol;
   const uint32_t lds = kLdsPerCu / kWorkgroupsPerCu - (quad ? kQuadLdsBytes : 0) -
                        (pair ? kPairLdsBytes : 0) - (col ? kColRows * kColBytes : 0);
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(kThreads), lds, stream, img, map_offset);
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(kThreads), lds, stream, args);
   return hipGetLastError();
 }
 
