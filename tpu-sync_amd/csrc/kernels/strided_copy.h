@@ -41,8 +41,10 @@ struct StridedEntryDev {
   uint32_t tile_begin;     // first workgroup of the entry
   uint32_t rows_per_tile;  // > 0: whole rows per workgroup
   uint32_t tiles_per_row;  // > 0: a row spans this many workgroups
-  uint16_t vec;            // vector bytes: 16, 8, 4, 2 or 1
-  uint16_t tail;           // bytes by which a row's last vector is stepped back
+  // One word, read with the rest by scalar loads: vector bytes (16, 8, 4, 2 or
+  // 1), bytes by which a row's last vector is stepped back (<< 8), whether
+  // tiles in whole groups go sliced (<< 16).
+  uint32_t format;
 };
 static_assert(sizeof(StridedEntryDev) == 64, "device table layout");
 

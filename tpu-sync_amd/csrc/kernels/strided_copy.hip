@@ -19,7 +19,7 @@
 // that is not a whole number of vectors ends with one that is stepped back to
 // the row's last byte, rewriting a few bytes with the same values. Measured
 // against one width for the whole launch that divides every address, size and
-// stride: four bf16 [14336, 4096] split 3 ways (2730-byte rows) 511 -> 195 us,
+// stride: four bf16 [14336, 4096] split 3 ways (2730-byte rows) 511 -> 176 us,
 // 0.87 GB of 8-bit weights with a 4-byte scale each packed in 500 -> 287 us
 // (a whole call; floors 140 and 260 us at this kernel's 6.7 TB/s).
 //
@@ -85,9 +85,9 @@ __device__ __forceinline__ void st(uint64_t a, typename VecT<V>::T v) {
 
 // Byte offset of vector v of a row of `vecs` vectors, the last one stepped
 // back by `tail` bytes.
-template <int V>
+template <int V, bool TAIL>
 __device__ __forceinline__ uint64_t vec_offset(uint64_t v, uint32_t vecs, uint32_t tail) {
-  return v * V - (v == vecs - 1 ? tail : 0);
+  return v * V - (TAIL && v == vecs - 1 ? tail : 0);
 }
 
 struct KArgs {
@@ -106,7 +106,7 @@ constexpr uint32_t kSliceVecs = 64;
 constexpr uint32_t kSliceTiles = kTileVecs / kSliceVecs;
 static_assert(kSliceTiles == kUnroll * (kThreads / 64), "one slice per wave and step");
 
-template <int V>
+template <int V, bool TAIL>
 __device__ __forceinline__ void copy_sliced(uint64_t src, uint64_t dst, uint32_t vecs,
                                             uint32_t tail, uint32_t ct) {
   const uint32_t j = ct & (kSliceTiles - 1);
@@ -122,12 +122,12 @@ __device__ __forceinline__ void copy_sliced(uint64_t src, uint64_t dst, uint32_t
     const uint32_t c = u * (kThreads / 64) + wave;  // tile of the group
     vi[u] = first + static_cast<uint64_t>(c) * kTileVecs + lane;
     const uint64_t vl = vi[u] < vecs ? vi[u] : vecs - 1;
-    r[u] = ld<V>(src + vec_offset<V>(vl, vecs, tail));
+    r[u] = ld<V>(src + vec_offset<V, TAIL>(vl, vecs, tail));
   }
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
     if (vi[u] < vecs) {
-      st<V>(dst + vec_offset<V>(vi[u], vecs, tail), r[u]);
+      st<V>(dst + vec_offset<V, TAIL>(vi[u], vecs, tail), r[u]);
     }
   }
 }
@@ -135,7 +135,7 @@ __device__ __forceinline__ void copy_sliced(uint64_t src, uint64_t dst, uint32_t
 // Slice j of each tile of the group of kSliceTiles tiles from tile tb of an
 // entry of short rows (rows_per_tile rows per tile; only the entry's last
 // tile may hold fewer).
-template <int V>
+template <int V, bool TAIL>
 __device__ __forceinline__ void copy_sliced_rows(const KVX_CONST StridedEntryDev& ent,
                                                  uint32_t tb, uint32_t j) {
   const uint32_t wave = threadIdx.x / 64;
@@ -158,7 +158,7 @@ __device__ __forceinline__ void copy_sliced_rows(const KVX_CONST StridedEntryDev
     const uint32_t kk = valid[u] ? k : total - 1;
     const uint32_t row = static_cast<uint32_t>((kk * magic) >> 32);
     const uint64_t r_abs = row0 + row;
-    const uint64_t col = vec_offset<V>(kk - row * vecs, vecs, ent.tail);
+    const uint64_t col = vec_offset<V, TAIL>(kk - row * vecs, vecs, (ent.format >> 8) & 0xff);
     r[u] = ld<V>(ent.src + r_abs * ent.src_stride + col);
     doff[u] = r_abs * ent.dst_stride + col;
   }
@@ -170,7 +170,7 @@ __device__ __forceinline__ void copy_sliced_rows(const KVX_CONST StridedEntryDev
 
 // Moves tile `wg` of entry `ent` (some of its rows, or one slice of a long
 // row) in vectors of V bytes.
-template <int V>
+template <int V, bool TAIL>
 __device__ __forceinline__ void copy_tile_v(const KArgs& a, const KVX_CONST StridedEntryDev* ent,
                                             uint32_t wg) {
   const uint64_t src = ent->src;
@@ -178,26 +178,27 @@ __device__ __forceinline__ void copy_tile_v(const KArgs& a, const KVX_CONST Stri
   const uint64_t sstride = ent->src_stride;
   const uint64_t dstride = ent->dst_stride;
   const uint32_t vecs = ent->vecs;
-  const uint32_t tail = ent->tail;
+  const uint32_t tail = (ent->format >> 8) & 0xff;
+  const bool sliced = a.sliced && (ent->format >> 16) != 0;
   const uint32_t t = wg - ent->tile_begin;
-  if (V == 16 && a.sliced && ent->rows_per_tile == 0) {
+  if (V == 16 && sliced && ent->rows_per_tile == 0) {
     const uint32_t tpr = ent->tiles_per_row;
     const uint32_t row = t / tpr;
     const uint32_t ct = t - row * tpr;
     // Tiles in whole groups go sliced; a row's last tiles (fewer than a
     // group) stay contiguous.
     if (ct < (tpr & ~(kSliceTiles - 1))) {
-      copy_sliced<V>(src + row * sstride, dst + row * dstride, vecs, tail, ct);
+      copy_sliced<V, TAIL>(src + row * sstride, dst + row * dstride, vecs, tail, ct);
       return;
     }
-  } else if (V == 16 && a.sliced) {
+  } else if (V == 16 && sliced) {
     const uint32_t rpt = ent->rows_per_tile;
     const uint32_t ntiles = (ent->count + rpt - 1) / rpt;
     const uint32_t tb = t & ~(kSliceTiles - 1);
     // Runs of short rows: tiles in whole groups of the entry go sliced, the
     // entry's last tiles (fewer than a group) contiguous.
     if (tb + kSliceTiles <= ntiles) {
-      copy_sliced_rows<V>(*ent, tb, t - tb);
+      copy_sliced_rows<V, TAIL>(*ent, tb, t - tb);
       return;
     }
   }
@@ -233,7 +234,7 @@ __device__ __forceinline__ void copy_tile_v(const KArgs& a, const KVX_CONST Stri
     const uint32_t row = nrows == 1 ? 0u : static_cast<uint32_t>((k * magic) >> 32);
     const uint32_t v = k - row * nv;
     const uint64_t r_abs = row0 + row;
-    const uint64_t col = vec_offset<V>(v0 + v, vecs, tail);
+    const uint64_t col = vec_offset<V, TAIL>(v0 + v, vecs, tail);
     r[u] = ld<V>(src + r_abs * sstride + col);
     doff[u] = r_abs * dstride + col;
   }
@@ -249,12 +250,17 @@ __device__ __forceinline__ void copy_tile_v(const KArgs& a, const KVX_CONST Stri
 __device__ __forceinline__ void copy_tile(const KArgs& a, uint32_t wg) {
   const uint32_t e = ((const KVX_CONST uint32_t*)a.tile_entry)[wg];
   const KVX_CONST StridedEntryDev* ent = (const KVX_CONST StridedEntryDev*)a.table + e;
-  switch (ent->vec) {
-    case 16: copy_tile_v<16>(a, ent, wg); break;
-    case 8: copy_tile_v<8>(a, ent, wg); break;
-    case 4: copy_tile_v<4>(a, ent, wg); break;
-    case 2: copy_tile_v<2>(a, ent, wg); break;
-    default: copy_tile_v<1>(a, ent, wg); break;
+  const uint32_t format = ent->format & 0xffff;
+  if (format == 16) {  // no row steps back
+    copy_tile_v<16, false>(a, ent, wg);
+    return;
+  }
+  switch (format & 0xff) {
+    case 16: copy_tile_v<16, true>(a, ent, wg); break;
+    case 8: copy_tile_v<8, true>(a, ent, wg); break;
+    case 4: copy_tile_v<4, true>(a, ent, wg); break;
+    case 2: copy_tile_v<2, true>(a, ent, wg); break;
+    default: copy_tile_v<1, true>(a, ent, wg); break;
   }
 }
 
@@ -334,8 +340,17 @@ bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes, bo
       d.vecs = static_cast<uint32_t>(vecs);
       d.div_magic = (uint64_t{1} << 32) / vecs + 1;
       d.tile_begin = static_cast<uint32_t>(tiles);
-      d.vec = static_cast<uint16_t>(vec);
-      d.tail = static_cast<uint16_t>(vecs * vec - static_cast<uint64_t>(c.size));
+      const uint64_t tail = vecs * vec - static_cast<uint64_t>(c.size);
+      // The wave-sized pieces of rows off 16 bytes share lines with their
+      // neighbours, which other workgroups (other XCDs' caches) hold when tiles
+      // go sliced. Short rows then stay contiguous if either side is off (bf16
+      // [14336, 4096] x 4 split 3 ways: 193 sliced, 176 us contiguous), long
+      // rows if both are (1 GiB: 418 and 394 us; with one side off 377 and 383).
+      const uint64_t off_src = (d.src | (count > 1 ? d.src_stride : 0)) & 15;
+      const uint64_t off_dst = (d.dst | (count > 1 ? d.dst_stride : 0)) & 15;
+      const bool sliced =
+          long_row ? off_src == 0 || off_dst == 0 : off_src == 0 && off_dst == 0;
+      d.format = static_cast<uint32_t>(vec | (tail << 8) | (sliced ? 1u << 16 : 0u));
       uint64_t t;
       if (!long_row) {
         d.rows_per_tile = static_cast<uint32_t>(kTileVecs / vecs);
