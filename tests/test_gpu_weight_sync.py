@@ -344,3 +344,34 @@ def test_strided_copy_any_alignment_matches_oracle(kvx, cuda, use_plan):
                for a, b, sz, c, ss, ds in ora]
     kvx.copy_strided(kvx.StridedPlan(entries) if use_plan else entries, device=0).Await()
     assert np.array_equal(u8(dst), want)
+
+
+def test_pack_and_unpack_into_any_staging_buffer(kvx, cuda):
+    """Pack and Unpack run resident tables against whatever buffer a call
+    names: two buffers in turn, one off a vector's alignment, odd sizes and a
+    4-byte tensor beside long ones, on two streams."""
+    rng = np.random.default_rng(29)
+    sizes = [1, 4, 100001, 32768, 3 << 20, 17, 65536 + 8]
+    src = [rng.integers(0, 256, n, dtype=np.uint8) for n in sizes]
+    params = [torch.from_numpy(x).to(cuda) for x in src]
+    ws = kvx.WeightSynchronizer([[p] for p in params])
+    offs = [ws.host_buffer_info(k, 0)[2] for k in range(len(sizes))]
+    rooms = [torch.full((ws.total_bytes + 64,), 0xEE, dtype=torch.uint8, device=cuda)
+             for _ in range(2)]
+    for k, at in ((0, 0), (1, 5), (0, 16)):
+        stream = torch.cuda.Stream(cuda)
+        torch.cuda.synchronize()
+        staging = rooms[k][at:at + ws.total_bytes]
+        ws.pack(staging, stream=stream).Await()
+        got = staging.cpu().numpy()
+        for x, o in zip(src, offs):
+            assert np.array_equal(got[o:o + x.size], x)
+        new = [rng.integers(0, 256, n, dtype=np.uint8) for n in sizes]
+        for x, o in zip(new, offs):
+            staging[o:o + x.size] = torch.from_numpy(x).to(cuda)
+        torch.cuda.synchronize()
+        ws.unpack(staging, stream=stream).Await()
+        for p, x in zip(params, new):
+            assert np.array_equal(p.cpu().numpy(), x)
+        src = new
+    ws.close()

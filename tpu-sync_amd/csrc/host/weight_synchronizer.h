@@ -63,6 +63,18 @@ struct WeightSyncConfig {
   bool numa_local = true;
 };
 
+// Strided entries as a device image (entry table + tile map), built and
+// uploaded once; the owner frees it when no launch reads it any more.
+struct StridedImage {
+  void* dev = nullptr;
+  uint32_t n = 0;
+  uint32_t grid = 0;
+  uint32_t long_tiles = 0;  // the first tiles of the grid, long rows (sliced)
+  // The device must be current.
+  Status Build(const std::vector<StridedCopy>& copies);
+  hipError_t Launch(hipStream_t stream, uint64_t src_add = 0, uint64_t dst_add = 0) const;
+};
+
 class WeightSynchronizer {
  public:
   static StatusOr<std::unique_ptr<WeightSynchronizer>> Create(WeightSyncConfig cfg);
@@ -111,8 +123,11 @@ class WeightSynchronizer {
   Status RangeEntries(int64_t lo, int64_t hi, uint64_t image, bool pack,
                       std::vector<StridedCopy>* out, std::vector<TiledJob>* zero,
                       std::vector<TiledJob>* tiled) const;
+  // staging != 0: `copies` are those of the whole set with its image there, and
+  // run from the resident table.
   Status Launch(const std::vector<StridedCopy>& copies, const std::vector<TiledJob>& zero,
-                const std::vector<TiledJob>& tiled, bool pack, hipStream_t stream);
+                const std::vector<TiledJob>& tiled, bool pack, hipStream_t stream,
+                uint64_t staging = 0);
   // Tiled layout of tensor k, or null for row-major bytes.
   const TiledPlan* plan(int64_t k) const {
     if (cfg_.tiled.empty() || cfg_.tiled[k] == nullptr || !cfg_.tiled[k]->tiled) return nullptr;
@@ -142,6 +157,7 @@ class WeightSynchronizer {
   std::vector<hipStream_t> slot_stream_;  // the stream of that use (null: none)
   size_t next_ = 0;
   ArgRing args_;
+  StridedImage whole_[2];  // every row-major tensor: pack, unpack
   std::vector<Sample> samples_;
 };
 
@@ -172,7 +188,7 @@ class StridedCopyPlan {
   StridedCopyPlan& operator=(const StridedCopyPlan&) = delete;
 
   StatusOr<CopyFuture> Run(hipStream_t stream);
-  uint32_t workgroups() const { return grid_; }
+  uint32_t workgroups() const { return image_.grid; }
   // With profiling on, each later run records a pair of timing events right
   // around its launch (and nothing else between them) on its stream.
   void SetProfiling(bool on);
@@ -183,13 +199,10 @@ class StridedCopyPlan {
  private:
   StridedCopyPlan() = default;
   int device_ = 0;
-  uint32_t n_ = 0;
-  uint32_t grid_ = 0;
-  uint32_t long_tiles_ = 0;  // the first tiles of the grid, long rows (sliced)
   int64_t bytes_ = 0;  // bytes one run moves
-  void* image_ = nullptr;
+  StridedImage image_;
   std::mutex mu_;
-  std::vector<hipEvent_t> runs_;  // one per run that may still read the image
+  std::vector<CopyFuture> runs_;  // the runs that may still read the image
   bool profile_ = false;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> samples_;  // (start, stop) per profiled run
 };

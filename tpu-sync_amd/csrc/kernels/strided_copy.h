@@ -71,10 +71,13 @@ int StridedVectorBytes(const std::vector<StridedCopy>& copies);
 // then walks tiles with a stride of the grid), for copies bound by PCIe
 // rather than HBM; otherwise the launch reserves LDS so that at most 2 of
 // its workgroups share a CU, and at 16-byte vectors moves the long-row tiles
-// sliced (0: every tile contiguous).
+// sliced (0: every tile contiguous). src_add and dst_add are added to every
+// entry's addresses (a table whose one side lies in a buffer that each call
+// names).
 hipError_t LaunchStridedCopy(const StridedEntryDev* table_dev, uint32_t n,
                              uint32_t tiles, hipStream_t stream,
-                             uint32_t max_workgroups = 0, uint32_t long_tiles = 0);
+                             uint32_t max_workgroups = 0, uint32_t long_tiles = 0,
+                             uint64_t src_add = 0, uint64_t dst_add = 0);
 
 }  // namespace kvx
 

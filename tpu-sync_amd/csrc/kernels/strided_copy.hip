@@ -19,8 +19,8 @@
 // that is not a whole number of vectors ends with one that is stepped back to
 // the row's last byte, rewriting a few bytes with the same values. Measured
 // against one width for the whole launch that divides every address, size and
-// stride: four bf16 [14336, 4096] split 3 ways (2730-byte rows) 511 -> 176 us,
-// 0.87 GB of 8-bit weights with a 4-byte scale each packed in 500 -> 287 us
+// stride: four bf16 [14336, 4096] split 3 ways (2730-byte rows) 511 -> 170 us,
+// 0.87 GB of 8-bit weights with a 4-byte scale each packed in 500 -> 268 us
 // (a whole call; floors 140 and 260 us at this kernel's 6.7 TB/s).
 //
 // At 16-byte vectors with one workgroup per tile, tiles go sliced: in a
@@ -91,6 +91,8 @@ __device__ __forceinline__ uint64_t vec_offset(uint64_t v, uint32_t vecs, uint32
 }
 
 struct KArgs {
+  uint64_t src_add;  // added to every entry's addresses
+  uint64_t dst_add;
   const StridedEntryDev* table;
   const uint32_t* tile_entry;  // tile -> entry index
   uint32_t tiles;
@@ -137,7 +139,8 @@ __device__ __forceinline__ void copy_sliced(uint64_t src, uint64_t dst, uint32_t
 // tile may hold fewer).
 template <int V, bool TAIL>
 __device__ __forceinline__ void copy_sliced_rows(const KVX_CONST StridedEntryDev& ent,
-                                                 uint32_t tb, uint32_t j) {
+                                                 uint64_t src, uint64_t dst, uint32_t tb,
+                                                 uint32_t j) {
   const uint32_t wave = threadIdx.x / 64;
   const uint32_t lane = threadIdx.x % 64;
   const uint32_t rpt = ent.rows_per_tile;
@@ -159,12 +162,12 @@ __device__ __forceinline__ void copy_sliced_rows(const KVX_CONST StridedEntryDev
     const uint32_t row = static_cast<uint32_t>((kk * magic) >> 32);
     const uint64_t r_abs = row0 + row;
     const uint64_t col = vec_offset<V, TAIL>(kk - row * vecs, vecs, (ent.format >> 8) & 0xff);
-    r[u] = ld<V>(ent.src + r_abs * ent.src_stride + col);
+    r[u] = ld<V>(src + r_abs * ent.src_stride + col);
     doff[u] = r_abs * ent.dst_stride + col;
   }
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
-    if (valid[u]) st<V>(ent.dst + doff[u], r[u]);
+    if (valid[u]) st<V>(dst + doff[u], r[u]);
   }
 }
 
@@ -173,8 +176,8 @@ __device__ __forceinline__ void copy_sliced_rows(const KVX_CONST StridedEntryDev
 template <int V, bool TAIL>
 __device__ __forceinline__ void copy_tile_v(const KArgs& a, const KVX_CONST StridedEntryDev* ent,
                                             uint32_t wg) {
-  const uint64_t src = ent->src;
-  const uint64_t dst = ent->dst;
+  const uint64_t src = ent->src + a.src_add;
+  const uint64_t dst = ent->dst + a.dst_add;
   const uint64_t sstride = ent->src_stride;
   const uint64_t dstride = ent->dst_stride;
   const uint32_t vecs = ent->vecs;
@@ -198,7 +201,7 @@ __device__ __forceinline__ void copy_tile_v(const KArgs& a, const KVX_CONST Stri
     // Runs of short rows: tiles in whole groups of the entry go sliced, the
     // entry's last tiles (fewer than a group) contiguous.
     if (tb + kSliceTiles <= ntiles) {
-      copy_sliced_rows<V, TAIL>(*ent, tb, t - tb);
+      copy_sliced_rows<V, TAIL>(*ent, src, dst, tb, t - tb);
       return;
     }
   }
@@ -372,9 +375,12 @@ bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes, bo
 
 hipError_t LaunchStridedCopy(const StridedEntryDev* table_dev, uint32_t n,
                              uint32_t tiles, hipStream_t stream,
-                             uint32_t max_workgroups, uint32_t long_tiles) {
+                             uint32_t max_workgroups, uint32_t long_tiles, uint64_t src_add,
+                             uint64_t dst_add) {
   if (tiles == 0) return hipSuccess;
   KArgs a;
+  a.src_add = src_add;
+  a.dst_add = dst_add;
   a.table = table_dev;
   // The tile -> entry map follows the table in the same device allocation.
   a.tile_entry = reinterpret_cast<const uint32_t*>(table_dev + n);
