@@ -427,7 +427,8 @@ def test_column_major_layouts_match_oracle(kvx, oracle, cuda, itemsize, P):
     shapes = [(128, across), (127, across - 1), (129, across + 1), (300, 2 * across + 3),
               (64, 5 * across), (257, across // 2 + 1), (1, 40), (40, 1), (3, 5), (130, 7)]
     for k, (H, W) in enumerate(shapes):
-        for tH, tW, batch in ((8, 128, []), (8, 128, [3]), (16, 64, []), (4, 16, [2])):
+        for tH, tW, batch in ((8, 128, []), (8, 128, [3]), (16, 64, []), (4, 16, [2]),
+                              (8, 512, [])):
             rank = len(batch) + 2
             mtm = [rank - 2, rank - 1] + list(range(rank - 3, -1, -1))
             lay = dict(itemsize=itemsize, dims=batch + [H, W], minor_to_major=mtm,

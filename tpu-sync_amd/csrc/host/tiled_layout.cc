@@ -180,7 +180,8 @@ static uint64_t ColumnRegionsAlong(const TiledPlan& p) {
 }
 static uint64_t ColumnRegionsAcross(uint64_t rows) { return (rows + kColRows - 1) / kColRows; }
 
-// Whether the transposed form takes the layout: tiled vectors of 16 bytes stay
+// Whether the transposed form takes the layout: rows hold a vector (the kernel
+// steps their last one back to the row's end), tiled vectors of 16 bytes stay
 // in one row group of one tile, and the matrices fill at least a sixteenth of
 // their regions, where the two forms meet: bf16 batches of [32, 32], a
 // sixteenth full, detile / tile in 23.5 / 38.1 us against 52.1 / 63.5 element
@@ -188,7 +189,7 @@ static uint64_t ColumnRegionsAcross(uint64_t rows) { return (rows + kColRows - 1
 // [16, 16] in 41.3 / 67.4 against 34.1 / 45.5.
 static bool ColumnFits(const TiledPlan& p) {
   const uint64_t s = static_cast<uint64_t>(p.layout.itemsize);
-  if (p.tW * p.P * s % 16 != 0) return false;
+  if (p.tW * p.P * s % 16 != 0 || p.W * s < 16) return false;
   const uint64_t along = ColumnRegionsAlong(p);
   const uint64_t across = ColumnRegionsAcross(p.nT1 * p.tW);
   uint64_t regions = 0;

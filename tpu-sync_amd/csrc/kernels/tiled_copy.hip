@@ -148,32 +148,6 @@ __device__ __forceinline__ void st_head(uint64_t a, uint32_t* w, uint32_t nb) {
   if (nb & 1) st<1>(a, static_cast<uint8_t>(x));
 }
 
-// Loads nb (< 16) bytes into the words w (zero on entry).
-__device__ __forceinline__ void ld_head(uint64_t a, uint32_t* w, uint32_t nb) {
-  uint32_t at = 0;
-  if (nb & 8) {
-    to_words<8>(ld<8>(a), w);
-    at = 8;
-  }
-  uint32_t lo = 0, hi = 0;  // the up to 7 bytes after them
-  if (nb & 4) {
-    lo = ld<4>(a + at);
-    const uint64_t b = a + at + 4;
-    if (nb & 2) hi = ld<2>(b);
-    if (nb & 1) hi |= static_cast<uint32_t>(ld<1>(b + (nb & 2))) << (8 * (nb & 2));
-  } else {
-    if (nb & 2) lo = ld<2>(a + at);
-    if (nb & 1) lo |= static_cast<uint32_t>(ld<1>(a + at + (nb & 2))) << (8 * (nb & 2));
-  }
-  if (nb & 8) {
-    w[2] = lo;
-    w[3] = hi;
-  } else {
-    w[0] = lo;
-    w[1] = hi;
-  }
-}
-
 // Tiled order of P rows of n words each: element c of row k lands at
 // position c * P + k. P = 2: 16-bit elements; P = 4: 8-bit elements.
 template <int P, int n>
@@ -599,9 +573,9 @@ __device__ __forceinline__ void col_region(const KVX_CONST TiledJobDev* j, uint3
     const uint32_t within = (r - tr * j->th.d) * j->tw.d + ((c - tc * j->tw.d) << log2p);
     return j->tiled + ((T * j->tile_elems + within) << sh);
   };
-  // Linear address of row h of the region.
-  auto row_at = [&](uint32_t h) -> uint64_t {
-    return j->linear + (b * j->h32 + c0 + h) * row_bytes;
+  // Address of a linear row of the region's matrix.
+  auto row_at = [&](uint32_t row) -> uint64_t {
+    return j->linear + (b * j->h32 + row) * row_bytes;
   };
   uint32_t v[U][4];
   if constexpr (!TILE) {
@@ -640,35 +614,33 @@ __device__ __forceinline__ void col_region(const KVX_CONST TiledJobDev* j, uint3
       const u32x4 y = *chunk_at(h, c);
       uint32_t w[4] = {y.x, y.y, y.z, y.w};
       if (x + 16 <= row_bytes) {
-        st<16>(row_at(h) + x, from_words<16>(w));
+        st<16>(row_at(c0 + h) + x, from_words<16>(w));
       } else {
-        st_head<16>(row_at(h) + x, w, static_cast<uint32_t>(row_bytes - x));
+        st_head<16>(row_at(c0 + h) + x, w, static_cast<uint32_t>(row_bytes - x));
       }
     }
   } else {
+    // Every load goes out without a branch: past the data a lane re-reads the
+    // last row or the row's last vector (zeroed below), and a row's last, partial
+    // vector is stepped back to the row's end (shifted below). With a branch
+    // around each load a bf16 [4096, 14336] weight tiled in 94 us, 50 so.
 #pragma unroll
     for (int i = 0; i < U; ++i) {
       const uint32_t k = threadIdx.x + i * kThreads;
       const uint32_t h = k / kChunks;
       const uint64_t x = x0 + (k % kChunks) * 16;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) v[i][w] = 0;
-      if (c0 + h < c_hi && x < row_bytes) {
-        if (row_bytes >= 16) {
-          // A row's last vector is stepped back to its end, then shifted.
-          const uint64_t xl = x + 16 <= row_bytes ? x : row_bytes - 16;
-          to_words<16>(ld<16>(row_at(h) + xl), v[i]);
-        } else {
-          ld_head(row_at(h), v[i], static_cast<uint32_t>(row_bytes));
-        }
-      }
+      const uint64_t xl = x + 16 <= row_bytes ? x : row_bytes - 16;
+      to_words<16>(ld<16>(row_at(c0 + h < c_hi ? c0 + h : c_hi - 1) + xl), v[i]);
     }
 #pragma unroll
     for (int i = 0; i < U; ++i) {
       const uint32_t k = threadIdx.x + i * kThreads;
       const uint32_t h = k / kChunks, c = k % kChunks;
       const uint64_t x = x0 + c * 16;
-      if (row_bytes >= 16 && x < row_bytes && x + 16 > row_bytes) {
+      if (c0 + h >= c_hi || x >= row_bytes) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) v[i][w] = 0;
+      } else if (x + 16 > row_bytes) {
         shift_down<4>(v[i], static_cast<uint32_t>(x + 16 - row_bytes));
       }
       *chunk_at(h, c) = u32x4{v[i][0], v[i][1], v[i][2], v[i][3]};
