@@ -733,10 +733,8 @@ static int RawCopy(bool gather, uint64_t storage_table, int64_t num_storages,
   p.nblocks = num_storages * n;
   p.block_bytes = block_bytes;
   p.pool_blocks = pool_blocks;
-  // The storage bases are device data the host cannot inspect; the vector
-  // width follows block_bytes and staging. gfx950 global memory accepts
-  // unaligned vector accesses, so a base that is not 16-byte aligned is slower
-  // but still copied exactly.
+  // The storage bases are device data the host cannot inspect: the kernels take
+  // them at any alignment.
   const int vec = kvx::LaunchVectorBytes(l, 0);
   hipError_t e = kvx::LaunchBlockCopy(
       l, gather ? kvx::CopyDir::kGather : kvx::CopyDir::kScatter, vec,

@@ -231,13 +231,19 @@ Status TransferEngine::Init() {
 }
 
 Status TransferEngine::SetStorages(const std::vector<uint64_t>& bases) {
-  if (bases.empty()) return OkStatus();
+  const size_t bytes = bases.size() * sizeof(uint64_t);
+  // (More storages than the argument ring holds go through it call by call.)
+  if (bases.empty() || bytes > static_cast<size_t>(arg_bytes_)) return OkStatus();
   DeviceGuard g(opts_.device);
   void* d = nullptr;
-  KVX_HIP_RETURN_IF_ERROR(hipMalloc(&d, bases.size() * sizeof(uint64_t)));
+  KVX_HIP_RETURN_IF_ERROR(hipMalloc(&d, bytes));
   bases_dev_ = reinterpret_cast<uint64_t>(d);
+  // On an own stream, from the ring's pinned memory: the caller's work in flight
+  // (a pool being filled) is not waited for.
+  std::memcpy(arg_host_, bases.data(), bytes);
   KVX_HIP_RETURN_IF_ERROR(
-      hipMemcpy(d, bases.data(), bases.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
+      hipMemcpyAsync(d, arg_host_, bytes, hipMemcpyHostToDevice, gather_stream_));
+  KVX_HIP_RETURN_IF_ERROR(hipStreamSynchronize(gather_stream_));
   bases_ = bases;
   return OkStatus();
 }

@@ -26,7 +26,7 @@ StatusOr<hipEvent_t> NewEvent() {
 // the caller's staging buffer.
 constexpr uint64_t kImageBase = 4096;
 
-Status StridedImage::Build(const std::vector<StridedCopy>& copies) {
+Status StridedImage::Build(const std::vector<StridedCopy>& copies, hipStream_t stream) {
   std::vector<StridedEntryDev> table;
   if (!copies.empty() &&
       !BuildStridedTable(copies, StridedVectorBytes(copies), /*any_align=*/true, &table, &grid,
@@ -38,7 +38,9 @@ Status StridedImage::Build(const std::vector<StridedCopy>& copies) {
   std::vector<uint8_t> image(static_cast<size_t>(StridedImageBytes(table.size(), grid)));
   WriteStridedImage(table, grid, image.data());
   KVX_HIP_RETURN_IF_ERROR(hipMalloc(&dev, image.size()));
-  KVX_HIP_RETURN_IF_ERROR(hipMemcpy(dev, image.data(), image.size(), hipMemcpyHostToDevice));
+  KVX_HIP_RETURN_IF_ERROR(
+      hipMemcpyAsync(dev, image.data(), image.size(), hipMemcpyHostToDevice, stream));
+  KVX_HIP_RETURN_IF_ERROR(hipStreamSynchronize(stream));
   return OkStatus();
 }
 
@@ -149,7 +151,7 @@ Status WeightSynchronizer::Init() {
     std::vector<TiledJob> zero, tiled;
     // Tensors that no launch can take fail a Pack, not the creation.
     if (!RangeEntries(0, total_, kImageBase, pack, &entries, &zero, &tiled).ok()) continue;
-    Status st = whole_[pack ? 0 : 1].Build(entries);
+    Status st = whole_[pack ? 0 : 1].Build(entries, ks_);
     if (!st.ok() && st.code() != Code::kInvalidArgument) return st;
   }
   return args_.Init(1 << 20);
@@ -526,7 +528,7 @@ StatusOr<std::unique_ptr<StridedCopyPlan>> StridedCopyPlan::Create(
   }
   DeviceGuard g(device);
   if (!copies.empty() && !g.ok()) return InvalidArgumentError("cannot select HIP device");
-  KVX_RETURN_IF_ERROR(p->image_.Build(copies));
+  KVX_RETURN_IF_ERROR(p->image_.Build(copies, nullptr));
   return p;
 }
 

@@ -70,8 +70,8 @@ struct StridedImage {
   uint32_t n = 0;
   uint32_t grid = 0;
   uint32_t long_tiles = 0;  // the first tiles of the grid, long rows (sliced)
-  // The device must be current.
-  Status Build(const std::vector<StridedCopy>& copies);
+  // The device must be current; the upload runs on `stream` and is waited for.
+  Status Build(const std::vector<StridedCopy>& copies, hipStream_t stream);
   hipError_t Launch(hipStream_t stream, uint64_t src_add = 0, uint64_t dst_add = 0) const;
 };
 

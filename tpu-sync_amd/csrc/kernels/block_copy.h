@@ -78,7 +78,9 @@ struct CopyLaunch {
 enum class CopyDir : int { kGather = 0, kScatter = 1 };
 
 // Largest vector width (16, 4 or 1 bytes) that every address of the launch
-// is aligned to. `extra_align` folds in addresses the caller knows about.
+// is aligned to: the width of a launch whose other side is paged host memory
+// (the others take 16-byte vectors at any address), and what the limits of every
+// launch are counted in. `extra_align` folds in addresses the caller knows about.
 int LaunchVectorBytes(const CopyLaunch& l, uint64_t extra_align);
 
 // Enqueues the copy on `stream`. Returns hipErrorInvalidValue when the launch

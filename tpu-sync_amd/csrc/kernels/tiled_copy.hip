@@ -4,8 +4,8 @@
 // 545-1036) before or after a raw DMA of the tiled bytes.
 //
 // Pure data movement, bound by HBM bandwidth. Every (vector width, rows per
-// unit, direction, unit order) combination is a kernel of its own, so the
-// hot loop carries no mode branches; the host groups a launch's jobs by that
+// unit, direction, whole or ragged rows) combination is a kernel of its own, so
+// the hot loop carries no mode branches; the host groups a launch's jobs by that
 // key. Standard-form jobs move units of P rows x V bytes; a lane issues all
 // loads of its units (128 bytes in flight) before its stores, so a workgroup
 // keeps 32 KiB in flight like the other copy kernels. Consecutive lanes take
