@@ -19,7 +19,7 @@
 // that is not a whole number of vectors ends with one that is stepped back to
 // the row's last byte, rewriting a few bytes with the same values. Measured
 // against one width for the whole launch that divides every address, size and
-// stride: four bf16 [14336, 4096] split 3 ways (2730-byte rows) 511 -> 170 us,
+// stride: four bf16 [14336, 4096] split 3 ways (2730-byte rows) 511 -> 170-176 us,
 // 0.87 GB of 8-bit weights with a 4-byte scale each packed in 500 -> 268 us
 // (a whole call; floors 140 and 260 us at this kernel's 6.7 TB/s).
 //
