@@ -136,13 +136,18 @@ typedef struct kvx_manager_config {
   int32_t host_copy_threads;    /* pageable host mirrors (malloc, shm): host
                                    threads of the pinned bounce lanes; 0 = 8,
                                    -1 = per-run pageable hipMemcpyAsync */
-  int32_t gather_workgroups_per_cu; /* device gathers (not zero-copy ones), and
-                                   larger scatters of blocks that are whole
-                                   KiB or under 16 KiB, reserve LDS so at most
-                                   this many share a CU (faster random reads
+  int32_t gather_workgroups_per_cu; /* device copies (not zero-copy ones)
+                                   reserve LDS so at most this many of their
+                                   workgroups share a CU (faster random reads
                                    and writes; keeps LDS-heavy kernels of other
-                                   streams off those CUs meanwhile); 0 = 2,
-                                   -1 = no limit */
+                                   streams off those CUs meanwhile): every
+                                   gather of one block size from 16 KiB up; of
+                                   2048 workgroups and more, other gathers, and
+                                   scatters of blocks under 16 KiB, of several
+                                   block sizes none above 16 KiB, or of
+                                   160 MiB and more (of one block size only if
+                                   it is whole KiB up to 1 MiB and there are 32
+                                   ids); 0 = 2, -1 = no limit */
 } kvx_manager_config;
 
 /* D2h/H2d dispatch (kv_cache_manager_base.cc:452-512, 2575-2630): ENV (0)

@@ -61,9 +61,12 @@ struct CopyLaunch {
   // consecutive blocks, which leaves CUs free for other work (a PCIe-bound
   // zero-copy kernel needs only a few hundred workgroups in flight).
   int64_t max_workgroups = 0;
-  // Gathers (other than capped zero-copy grids), and scatters of the packed and
-  // sliced kernels, reserve LDS so that at most this many of their workgroups
-  // share a CU (0: no limit). Fewer random accesses in flight per CU let the
+  // Copies between device buffers reserve LDS so that at most this many of
+  // their workgroups share a CU (0: no limit): gathers of one block size that do
+  // not go packed or sliced always; packed and sliced copies, and those of
+  // several block sizes, from 2048 workgroups on, of their scatters only those
+  // that are sliced, whose blocks are at most 16 KiB or that move 160 MiB and
+  // more. Fewer random accesses in flight per CU let the
   // DRAM serve them more efficiently: 2 measured 74.5 -> 76.0 % of HBM peak for
   // a gather of 512 x 64 blocks of 32 KiB (1 and 3 the same, 4 and 6 no gain),
   // 67.2 -> 69.9 % for fp8 payload (16 KiB) + scales, and for scatters of packed
@@ -88,8 +91,15 @@ int LaunchVectorBytes(const CopyLaunch& l, uint64_t extra_align);
 hipError_t LaunchBlockCopy(const CopyLaunch& l, CopyDir dir, int vec_bytes,
                            hipStream_t stream);
 
-// Workgroups a launch uses (for tests and profiling).
-int64_t BlockCopyWorkgroups(const CopyLaunch& l, int vec_bytes);
+// The kernel a launch runs, its workgroups and the LDS it reserves: what
+// LaunchBlockCopy would choose, without a launch (for tests and reports). False
+// where LaunchBlockCopy would refuse the launch's sizes.
+struct BlockCopyRoute {
+  const char* kernel = nullptr;
+  uint64_t workgroups = 0;
+  uint32_t lds_bytes = 0;
+};
+bool BlockCopyRouteOf(const CopyLaunch& l, CopyDir dir, int vec_bytes, BlockCopyRoute* route);
 
 }  // namespace kvx
 

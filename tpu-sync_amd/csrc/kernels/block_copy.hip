@@ -626,8 +626,7 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
   P->n = static_cast<uint32_t>(l.n);
   P->npieces = l.npieces;
   // Vectors of a piece: the common width if a launch has a second paged side,
-  // else the widest its blocks hold. Blocks of 2 and more vectors per lane go
-  // whole to a workgroup.
+  // else the widest its blocks hold.
   const bool paged = Paged(l);
   auto vec_of = [&](uint64_t bytes) -> uint64_t {
     uint64_t v = static_cast<uint64_t>(vec_bytes);
@@ -828,8 +827,78 @@ constexpr uint32_t kLdsPerCu = 160u << 10;
 // scattered in 9.7 us capped, 8.6 not).
 constexpr uint32_t kCapGrid = 2048;
 
-// LDS the general kernel declares (the small-block path's address tables).
+// LDS the kernels with the small-block path declare (its address tables).
 constexpr uint32_t kStaticLds = 2 * kSmallMaxBlocks * sizeof(uint64_t);
+
+// Whether a scatter with packed or several pieces takes the cap on workgroups
+// per CU: where its blocks are at most 16 KiB (the packed ones and those of 4
+// vectors a lane), or its two sides do not fit the last-level cache. Capped and
+// not, in one process: 2 KiB blocks with 4-byte scales 48.7 and 52.4 us (134
+// MB), 16 KiB with 32-byte ones 48.4 and 49.7 (134 MB), 20000 bytes with 4-byte
+// ones 126.0 and 130.5 (314 MB), 8 and 32 KiB storages 113.8 and 115.5 (315
+// MB). Larger blocks whose launch stays in the cache gain nothing and some lose
+// (17 KiB blocks with scales 28.5 and 27.7 us, 20000 bytes 30.7 and 29.4, both
+// 67 MB; 24 KiB 56.0 and 53.9, 135 MB): they leave the CUs' LDS free.
+bool CapScatter(const KParams& P) {
+  uint64_t total = 0, largest = 0;
+  for (int k = 0; k < P.npieces; ++k) {
+    total += P.p[k].bytes * P.p[k].nblocks;
+    largest = std::max(largest, P.p[k].bytes);
+  }
+  return largest <= 4 * kThreads * 16 || total >= kSlicedMinBytes;
+}
+
+// What a launch runs: its kernel, that kernel's parameters (the general kernel
+// takes the KParams as they are), its grid and the LDS it reserves.
+struct Choice {
+  enum Kernel { kGeneral, kFast, kFastSide, kSliced } kernel = kGeneral;
+  int order = kStorageMajor;
+  dim3 grid;
+  uint32_t lds = 0;
+  FastSideParams FS;
+  SlicedParams S;
+};
+
+Choice Choose(const KParams& P, uint32_t grid, CopyDir dir, int wg_per_cu, bool capped_grid) {
+  const bool gather = dir == CopyDir::kGather;
+  Choice c;
+  c.grid = dim3(grid);
+  FastParams& F = c.FS.fast;
+  // Blocks above one workgroup's pass (kUnroll * kThreads vectors, 32 KiB at
+  // 16-byte vectors) go to consecutive workgroups a pass each, unless the
+  // launch's grid is capped (zero-copy copies keep their few workgroups).
+  auto split = [&](uint32_t blocks) {
+    const uint32_t pass = kUnroll * kThreads;
+    if (capped_grid || F.elems <= pass) return;
+    const uint64_t pieces = (static_cast<uint64_t>(F.elems) + pass - 1) / pass;
+    if (static_cast<uint64_t>(blocks) * pieces + (grid - blocks) > INT32_MAX) return;
+    F.pieces = static_cast<uint32_t>(pieces);
+    F.piece_elems = pass;
+    c.grid.x = grid - blocks + blocks * F.pieces;
+  };
+  // The reservation that leaves room for wg_per_cu workgroups on a CU.
+  const uint32_t room = wg_per_cu > 0 ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) : 0;
+  const uint32_t side_room = room > kStaticLds ? room - kStaticLds : 0;
+  if (!capped_grid && BuildSlicedParams(P, dir, &c.S, &c.grid)) {
+    c.kernel = Choice::kSliced;
+    if (c.grid.x * c.grid.y * c.grid.z >= kCapGrid) c.lds = side_room;
+    return c;
+  }
+  if (BuildFastParams(P, dir, &F, &c.order)) {
+    c.kernel = Choice::kFast;
+    split(grid);
+    if (gather) c.lds = room;
+    return c;
+  }
+  // The kernels with the packed path: not the capped grids of zero-copy copies.
+  const bool cap = !capped_grid && grid >= kCapGrid && (gather || CapScatter(P));
+  if (cap) c.lds = side_room;
+  if (BuildFastSideParams(P, dir, &F, &c.FS.side, &c.FS.side_wgs, &c.order)) {
+    c.kernel = Choice::kFastSide;
+    split(grid - c.FS.side_wgs);
+  }
+  return c;
+}
 
 // Few ids take kernels with smaller arguments: one block of 64 storages
 // gathered in 13.0 us a call, 14.6 with room for kMaxInlineIds (copied twice
@@ -873,56 +942,28 @@ template <int kCap>
 hipError_t Launch(const KParams& P, const uint32_t* inline_ids, uint32_t grid, CopyDir dir,
                   int wg_per_cu, bool capped_grid, int whole_vec, hipStream_t stream) {
   const bool gather = dir == CopyDir::kGather;
-  // Gathers reserve (unused) LDS to cap their workgroups per CU.
-  Launcher<kCap> to{inline_ids, P.n, dim3(grid), 0, stream};
-  if (gather && wg_per_cu > 0) to.lds = kLdsPerCu / static_cast<uint32_t>(wg_per_cu);
-  FastSideParams FS;
-  FastParams& F = FS.fast;
-  int order = kStorageMajor;
-  // Blocks above one workgroup's pass (kUnroll * kThreads vectors, 32 KiB at
-  // 16-byte vectors) go to consecutive workgroups a pass each, unless the
-  // launch's grid is capped (zero-copy copies keep their few workgroups).
-  auto split = [&](uint32_t blocks) {
-    const uint32_t pass = kUnroll * kThreads;
-    if (capped_grid || F.elems <= pass) return;
-    const uint64_t pieces = (static_cast<uint64_t>(F.elems) + pass - 1) / pass;
-    if (static_cast<uint64_t>(blocks) * pieces + (to.grid.x - blocks) > INT32_MAX) return;
-    F.pieces = static_cast<uint32_t>(pieces);
-    F.piece_elems = pass;
-    to.grid.x = to.grid.x - blocks + blocks * F.pieces;
-  };
-  SlicedParams S;
-  if (!capped_grid && BuildSlicedParams(P, dir, &S, &to.grid)) {
-    to.lds = wg_per_cu > 0 && to.grid.x * to.grid.y * to.grid.z >= kCapGrid
-                 ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) - kStaticLds
-                 : 0;
-    return gather ? to.template Run<SlicedParams>(block_copy_sliced_kernel<true, kCap>, S)
-                  : to.template Run<SlicedParams>(block_copy_sliced_kernel<false, kCap>, S);
+  const Choice c = Choose(P, grid, dir, wg_per_cu, capped_grid);
+  const Launcher<kCap> to{inline_ids, P.n, c.grid, c.lds, stream};
+  const FastParams& F = c.FS.fast;
+  if (c.kernel == Choice::kSliced) {
+    return gather ? to.template Run<SlicedParams>(block_copy_sliced_kernel<true, kCap>, c.S)
+                  : to.template Run<SlicedParams>(block_copy_sliced_kernel<false, kCap>, c.S);
   }
-  if (BuildFastParams(P, dir, &F, &order)) {
-    split(grid);
+  if (c.kernel == Choice::kFast) {
     if (gather) {
-      return order == kStoragePairs ? to.template Fast<true, kStoragePairs>(F)
-                                    : to.template Fast<true, kStorageMajor>(F);
+      return c.order == kStoragePairs ? to.template Fast<true, kStoragePairs>(F)
+                                      : to.template Fast<true, kStorageMajor>(F);
     }
-    return order == kAllStorages ? to.template Fast<false, kAllStorages>(F)
-                                 : to.template Fast<false, kStorageMajor>(F);
+    return c.order == kAllStorages ? to.template Fast<false, kAllStorages>(F)
+                                   : to.template Fast<false, kStorageMajor>(F);
   }
-  // The kernels with the packed path take the same cap in both directions (not
-  // the capped grids of zero-copy copies), minus that path's own 4 KiB of address
-  // tables: 3 and 4 KiB blocks scattered in 152 and 198 us capped, 160 and 208
-  // not.
-  to.lds = wg_per_cu > 0 && !capped_grid && grid >= kCapGrid
-               ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) - kStaticLds
-               : 0;
-  if (BuildFastSideParams(P, dir, &F, &FS.side, &FS.side_wgs, &order)) {
-    split(grid - FS.side_wgs);
+  if (c.kernel == Choice::kFastSide) {
     if (gather) {
-      return order == kStoragePairs ? to.template FastSide<true, kStoragePairs>(FS)
-                                    : to.template FastSide<true, kStorageMajor>(FS);
+      return c.order == kStoragePairs ? to.template FastSide<true, kStoragePairs>(c.FS)
+                                      : to.template FastSide<true, kStorageMajor>(c.FS);
     }
-    return order == kAllStorages ? to.template FastSide<false, kAllStorages>(FS)
-                                 : to.template FastSide<false, kStorageMajor>(FS);
+    return c.order == kAllStorages ? to.template FastSide<false, kAllStorages>(c.FS)
+                                   : to.template FastSide<false, kStorageMajor>(c.FS);
   }
   if constexpr (kCap == 0) {
     if (whole_vec == 4) return to.template General<4>(P, gather);
@@ -945,11 +986,17 @@ int LaunchVectorBytes(const CopyLaunch& l, uint64_t extra_align) {
   return 1;
 }
 
-int64_t BlockCopyWorkgroups(const CopyLaunch& l, int vec_bytes) {
+bool BlockCopyRouteOf(const CopyLaunch& l, CopyDir dir, int vec_bytes, BlockCopyRoute* route) {
   KParams P;
   uint32_t grid = 0;
-  if (!BuildParams(l, vec_bytes, &P, &grid)) return -1;
-  return grid;
+  if (!BuildParams(l, vec_bytes, &P, &grid)) return false;
+  const Choice c = Choose(P, grid, dir, l.gather_workgroups_per_cu, l.max_workgroups > 0);
+  static const char* const kNames[] = {"block_copy_kernel", "block_copy_fast_kernel",
+                                       "block_copy_fast_side_kernel", "block_copy_sliced_kernel"};
+  route->kernel = kNames[c.kernel];
+  route->workgroups = static_cast<uint64_t>(c.grid.x) * c.grid.y * c.grid.z;
+  route->lds_bytes = c.lds;
+  return true;
 }
 
 hipError_t LaunchBlockCopy(const CopyLaunch& l, CopyDir dir, int vec_bytes,

@@ -224,11 +224,14 @@ class KVCacheManager:
       host_copy_threads: a pageable host mirror ("malloc", "shm") moves
         through pinned bounce buffers that this many host threads fill and
         drain (0: 8; -1: per-run pageable copies by the HIP runtime).
-      gather_workgroups_per_cu: device gathers (not zero-copy ones), and larger
-        scatters of blocks that are whole KiB or under 16 KiB, reserve LDS so
-        that at most this many share a CU, which serves their random side
-        faster but keeps LDS-heavy kernels of other streams off those CUs while
-        they run (0: 2; -1: no limit).
+      gather_workgroups_per_cu: device copies (not zero-copy ones) reserve LDS
+        so that at most this many of their workgroups share a CU, which serves
+        their random side faster but keeps LDS-heavy kernels of other streams
+        off those CUs while they run (0: 2; -1: no limit): every gather of one
+        block size from 16 KiB up; of 2048 workgroups and more, other gathers,
+        and scatters of blocks under 16 KiB, of several block sizes none above
+        16 KiB, or of 160 MiB and more (of one block size only if it is whole
+        KiB up to 1 MiB and there are 32 ids).
       The remaining reference arguments (ports, worker id, timeout,
       parallelism, unsafe_skip_buffer_lock) configure its networking, which
       this single-GPU build does not have; they are accepted and ignored.
