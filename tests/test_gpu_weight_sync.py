@@ -375,3 +375,28 @@ def test_pack_and_unpack_into_any_staging_buffer(kvx, cuda):
             assert np.array_equal(p.cpu().numpy(), x)
         src = new
     ws.close()
+
+
+def test_pack_limit_is_the_staging_buffers(kvx, cuda):
+    """A row holds at most 2^32 - 1 vectors of the width that divides every
+    address and size of the call: a tensor of 4 GiB packs into (and unpacks
+    from) an even address, and is refused at an odd one with nothing written."""
+    n = 1 << 32
+    param = torch.empty(n, dtype=torch.uint8, device=cuda)
+    param.view(torch.int64).random_()
+    ws = kvx.WeightSynchronizer([[param]])
+    assert ws.total_bytes == n
+    room = torch.full((n + 16,), 0xEE, dtype=torch.uint8, device=cuda)
+    for copy in (ws.pack, ws.unpack):
+        with pytest.raises(kvx.KvxError, match="limits") as e:
+            copy(room[1:1 + n])
+        assert e.value.code == 3
+    torch.cuda.synchronize()
+    assert bool((room.view(torch.int64) == room.view(torch.int64)[0]).all())
+    ws.pack(room[2:2 + n]).Await()
+    assert torch.equal(room[2:2 + n], param)
+    assert room[:2].tolist() + room[2 + n:].tolist() == [0xEE] * 16
+    param.zero_()
+    ws.unpack(room[2:2 + n]).Await()
+    assert torch.equal(room[2:2 + n], param)
+    ws.close()

@@ -437,6 +437,11 @@ StatusOr<CopyFuture> WeightSynchronizer::WholeCopy(bool pack, uint64_t staging, 
   std::vector<StridedCopy> entries;
   std::vector<TiledJob> zero, tiled;
   KVX_RETURN_IF_ERROR(RangeEntries(0, total_, staging, pack, &entries, &zero, &tiled));
+  // The limits are those of the caller's address, wherever the resident table
+  // places the image.
+  if (!StridedRowsFit(entries, StridedVectorBytes(entries))) {
+    return InvalidArgumentError("strided copy entry out of the kernel's limits");
+  }
   KVX_RETURN_IF_ERROR(Launch(entries, zero, tiled, pack, stream, staging));
   KVX_ASSIGN_OR_RETURN(hipEvent_t done, NewEvent());
   KVX_HIP_RETURN_IF_ERROR(hipEventRecord(done, stream));

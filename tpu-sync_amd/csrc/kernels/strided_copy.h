@@ -48,6 +48,11 @@ struct StridedEntryDev {
 };
 static_assert(sizeof(StridedEntryDev) == 64, "device table layout");
 
+// Whether every entry is within the kernel's limits. A row's limit is 2^32 - 1
+// vectors of the common width `vec_bytes` (StridedVectorBytes), so that what a
+// launch accepts does not depend on the vectors that move it.
+bool StridedRowsFit(const std::vector<StridedCopy>& copies, int vec_bytes);
+
 // Builds the device table for `copies`; returns false if an entry violates
 // the kernel's limits. any_align: both sides are device memory, and each entry
 // takes the widest vectors its rows hold, at any address (a row's last vector

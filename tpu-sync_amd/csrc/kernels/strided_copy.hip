@@ -308,10 +308,22 @@ int StridedVectorBytes(const std::vector<StridedCopy>& copies) {
   return 1;
 }
 
+bool StridedRowsFit(const std::vector<StridedCopy>& copies, int vec_bytes) {
+  for (const StridedCopy& c : copies) {
+    if (c.size <= 0 || c.size % vec_bytes != 0 || c.src == 0 || c.dst == 0 ||
+        c.src_stride < 0 || c.dst_stride < 0 || c.count > UINT32_MAX ||
+        static_cast<uint64_t>(c.size) / vec_bytes > UINT32_MAX) {
+      return false;
+    }
+  }
+  return true;
+}
+
 bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes, bool any_align,
                        std::vector<StridedEntryDev>* table, uint32_t* grid,
                        uint32_t* long_tiles) {
   table->clear();
+  if (!StridedRowsFit(copies, vec_bytes)) return false;
   uint64_t tiles = 0;
   uint64_t long_end = 0;
   // Entries of long rows (more than one tile) first, then the others; each
@@ -319,13 +331,6 @@ bool BuildStridedTable(const std::vector<StridedCopy>& copies, int vec_bytes, bo
   for (int pass = 0; pass < 2; ++pass) {
     for (const StridedCopy& c : copies) {
       const int64_t count = c.count > 0 ? c.count : 1;
-      if (c.size <= 0 || c.size % vec_bytes != 0 || c.src == 0 || c.dst == 0 ||
-          c.src_stride < 0 || c.dst_stride < 0 || count > UINT32_MAX) {
-        return false;
-      }
-      // The limit on a row is the common width's, so that what a launch
-      // accepts does not depend on where it runs.
-      if (static_cast<uint64_t>(c.size) / vec_bytes > UINT32_MAX) return false;
       uint64_t vec = static_cast<uint64_t>(vec_bytes);
       if (any_align) {
         vec = 16;
