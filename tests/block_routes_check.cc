@@ -72,6 +72,14 @@ int main() {
   Expect("80 x 64 x 32 KiB gather, 160 MiB", Make(80, {{64, 32768}}), G, sliced, two_side);
   Expect("79 x 64 x 32 KiB gather", Make(79, {{64, 32768}}), G, fast, two);
   Expect("79 x 64 x 32 KiB scatter", Make(79, {{64, 32768}}), S, fast, 0);
+  // A chunk of whole storages, the first of them not storage 0; and one that
+  // starts inside a storage.
+  CopyLaunch chunk = Make(63, {{84, 32768}});
+  chunk.pieces[0].f0 = 84 * 63;
+  Expect("storages 84 to 167 of 63 ids, gather", chunk, G, sliced, two_side);
+  Expect("storages 84 to 167 of 63 ids, scatter", chunk, S, sliced, two_side);
+  chunk.pieces[0].f0 += 1;
+  Expect("the same one id further, gather", chunk, G, fast, two);
   Expect("512 x 64 x 20000 scatter", Make(512, {{64, 20000}}), S, fast, 0);
   Expect("64 x 64 x 16 KiB scatter", Make(64, {{64, 16384}}), S, fast, 0);
   Expect("1 x 64 x 32 KiB gather", Make(1, {{64, 32768}}), G, fast, two);

@@ -271,21 +271,9 @@ def test_fp8_llama3_8b_pool_full_size_round_trip(kvx, cuda):
     mgr.close()
 
 
-# Block bytes around a vector, a lane's share, the whole-block limit (8 KiB)
-# and a workgroup's pass (32 KiB), with side tables of other sizes.
-ANY_SIZES = [(1, 4), (3, 1), (7, 8), (15, 4), (16, 4), (17, 32), (33, 4), (255, 2), (1000, 4),
-             (2048, 4), (2560, 12), (4095, 4), (4097, 32), (8190, 4), (8192, 4), (8193, 20),
-             (10250, 4), (32768, 4), (32769, 4), (40001, 6), (65551, 32)]
-
-
-@pytest.mark.parametrize("block,side", ANY_SIZES, ids=[f"{b}+{s}" for b, s in ANY_SIZES])
-def test_gather_scatter_of_any_block_size(kvx, cuda, block, side):
-    """Payload and side table of any size in one launch, each at its own vector
-    width: a block that is no whole number of vectors ends with one stepped
-    back, and no byte of another block changes. Storages start at odd
-    addresses; layer-major with the side table, block-major without."""
-    rng = np.random.default_rng(block)
-    layers, blocks, n = 3, 40, 29
+def any_size_round_trip(kvx, cuda, rng, block, side, layers, blocks, n):
+    """Gather and scatter of n blocks of 2 * layers storages, with `layers` side
+    tables (layer-major) and without (block-major), all at odd addresses."""
     pool_np = rng.integers(0, 256, 2 * layers * blocks * block + 1, dtype=np.uint8)
     side_np = rng.integers(0, 256, layers * blocks * side + 1, dtype=np.uint8)
     ids = rng.permutation(blocks)[:n].tolist()
@@ -330,3 +318,31 @@ def test_gather_scatter_of_any_block_size(kvx, cuda, block, side):
         assert np.array_equal(pool.cpu().numpy(), want_pool)
         assert np.array_equal(tab.cpu().numpy(), want_tab)
         mgr.close()
+
+
+# Block bytes around a vector, a lane's share, the whole-block limit (16 KiB)
+# and a workgroup's pass (32 KiB), with side tables of other sizes.
+ANY_SIZES = [(1, 4), (3, 1), (7, 8), (15, 4), (16, 4), (17, 32), (33, 4), (255, 2), (1000, 4),
+             (2048, 4), (2560, 12), (4095, 4), (4097, 32), (8190, 4), (8192, 4), (8193, 20),
+             (10250, 4), (16367, 4), (16368, 4), (16383, 4), (16384, 4), (16385, 4), (16400, 4),
+             (32768, 4), (32769, 4), (40001, 6), (65551, 32)]
+
+
+@pytest.mark.parametrize("block,side", ANY_SIZES, ids=[f"{b}+{s}" for b, s in ANY_SIZES])
+def test_gather_scatter_of_any_block_size(kvx, cuda, block, side):
+    """Payload and side table of any size in one launch, each at its own vector
+    width: a block that is no whole number of vectors ends with one stepped
+    back, and no byte of another block changes. Storages start at odd
+    addresses; layer-major with the side table, block-major without."""
+    rng = np.random.default_rng(block)
+    any_size_round_trip(kvx, cuda, rng, block, side, layers=3, blocks=40, n=29)
+
+
+@pytest.mark.parametrize("block", [64, 1000, 8200, 16367, 16368, 16383])
+def test_gather_scatter_of_full_packed_workgroups(kvx, cuda, block):
+    """Packed launches of 512 workgroups and more, whose workgroups take all the
+    blocks they can (up to 2048 vectors), the last one fewer."""
+    rng = np.random.default_rng(block)
+    per = min(256, 2048 // -(-block // 16))
+    n = (512 * per + per // 2) // 16 + 3
+    any_size_round_trip(kvx, cuda, rng, block, 4, layers=8, blocks=n + 11, n=n)

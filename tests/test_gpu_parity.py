@@ -432,12 +432,11 @@ def test_raw_kernel_bad_id_flag(kvx, cuda):
 @pytest.mark.parametrize("bb", [32768, 16384])
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 7, 8, 33, 510])
 @pytest.mark.parametrize("W,order", [(2, 0), (4, 1), (6, 0)])
-def test_sliced_gather_matches_oracle(kvx, oracle, cuda, n, W, order, bb):
-    """32 KiB blocks at 16-byte vectors over an even number of whole
-    storages take the sliced gather (a quarter of each of 4 consecutive ids
-    per workgroup; 16 KiB blocks, the fast kernel, alongside): any n, so the
-    last group holds 1-4 ids, duplicate ids, layer-major (0) and block-major
-    (1) staging, byte for byte against the oracle's extract."""
+def test_fast_gather_matches_oracle(kvx, oracle, cuda, n, W, order, bb):
+    """Blocks of 16 and 32 KiB over an even number of whole storages, far below
+    the 160 MiB of a sliced launch, take the fast kernel in storage pairs: any
+    n, duplicate ids, layer-major (0) and block-major (1) staging, byte for
+    byte against the oracle's extract."""
     rng = np.random.default_rng(1000 + 10 * n + W + bb)
     P = 600
     host = [rng.integers(0, 256, (P, bb), dtype=np.uint8) for _ in range(W)]
@@ -459,11 +458,10 @@ def test_sliced_gather_matches_oracle(kvx, oracle, cuda, n, W, order, bb):
 
 
 @pytest.mark.parametrize("bb", [32768, 16384])
-def test_sliced_gather_bad_ids_in_a_group_and_in_the_last(kvx, cuda, bb):
-    """The sliced gather (32 KiB blocks; 16 KiB blocks, the fast kernel,
-    alongside) with bad ids: two in the first group of 4, one in the second,
-    one in the last (short) group. Good blocks land, bad ones leave their
-    staging untouched, and the error flag is set."""
+def test_fast_gather_skips_and_flags_bad_ids(kvx, cuda, bb):
+    """The fast gather with bad ids at both ends of the list and between good
+    ones: good blocks land, bad ones leave their staging untouched, and the
+    error flag is set."""
     rng = np.random.default_rng(31)
     W, P = 2, 20
     id_list = [3, 20, 5, -1, 8, 9, 99, 0, 7, -2]
@@ -1187,6 +1185,80 @@ def test_sliced_launches_move_the_same_blocks(kvx, cuda, block, storages, n, sid
         mgr.scatter(ids.tolist(), new, block_major=block_major).Await()
         assert torch.equal(pool, want_pool)
         assert not side or torch.equal(tabs, want_tabs)
+    mgr.close()
+
+
+@pytest.mark.parametrize("block,storages,n,side", [(2048, 160, 545, 0), (32768, 164, 33, 0),
+                                                   (16384, 160, 95, 6)])
+def test_sliced_launches_at_any_address(kvx, cuda, block, storages, n, side):
+    """Sliced launches whose storages, tables and staging all start at odd
+    addresses, a gather with repeated ids among them: every byte outside the
+    blocks, before and after the buffers too, stays."""
+    assert block * storages * n >= 160 << 20
+    gen = torch.Generator(device=cuda).manual_seed(block + n)
+    P = n + 9
+
+    def odd(count, size, gap):
+        """`count` tables of P rows of `size` bytes, `gap` bytes before each and
+        after the last, in one buffer."""
+        pitch = P * size + gap
+        buf = torch.randint(0, 256, (count * pitch + gap,), dtype=torch.uint8, device=cuda,
+                            generator=gen)
+        return buf, [buf[gap + w * pitch:gap + w * pitch + P * size].view(P, size)
+                     for w in range(count)]
+
+    pool, caches = odd(storages, block, 5)
+    tab, tables = odd(storages, side, 3) if side else (None, [])
+    mgr = kvx.KVCacheManager(caches, host_blocks_to_allocate=1, scale_tables=tables or None)
+    cut, total = storages * n * block, storages * n * (block + side)
+    room = torch.full((total + 32,), 0x5A, dtype=torch.uint8, device=cuda)
+    staging = room[7:7 + total]
+    ids = torch.randint(0, P, (n,), device=cuda, generator=gen)
+    ids[1], ids[n - 1] = ids[0], ids[n - 2]
+    mgr.gather(ids.tolist(), staging).Await()
+    for w in range(storages):
+        assert torch.equal(staging[:cut].view(storages, n, block)[w], caches[w][ids]), w
+        assert not side or torch.equal(staging[cut:].view(storages, n, side)[w], tables[w][ids]), w
+    assert bool((room[:7] == 0x5A).all()) and bool((room[7 + total:] == 0x5A).all())
+    new = torch.randint(0, 256, (total + 1,), dtype=torch.uint8, device=cuda, generator=gen)[1:]
+    dst = torch.randperm(P, device=cuda, generator=gen)[:n]
+    want_pool, want_tab = pool.clone(), tab.clone() if side else None
+    for whole, size, start, part in ((want_pool, block, 5, new[:cut]),
+                                     (want_tab, side, 3, new[cut:])):
+        for w in range(storages if size else 0):
+            at = start + w * (P * size + start)
+            whole[at:at + P * size].view(P, size)[dst] = part.view(storages, n, size)[w]
+    mgr.scatter(dst.tolist(), new).Await()
+    assert torch.equal(pool, want_pool)
+    assert not side or torch.equal(tab, want_tab)
+    mgr.close()
+
+
+def test_staged_chunks_of_whole_storages_go_sliced(kvx, cuda):
+    """A staged offload and reload in chunks of 84 whole storages each (165 MiB,
+    so sliced launches, the second from storage 84 on) and a last chunk of 5."""
+    S, P, n, block = 173, 72, 63, 32768
+    gen = torch.Generator(device=cuda).manual_seed(3)
+    pool = torch.randint(-2**31, 2**31 - 1, (S, P, block // 4), dtype=torch.int32, device=cuda,
+                         generator=gen)
+    chunk = 84 * n * block
+    assert chunk >= 160 << 20
+    mgr = kvx.KVCacheManager([pool[w] for w in range(S)], host_blocks_to_allocate=n,
+                             transfer_mode="staged", staging_chunk_bytes=chunk,
+                             staging_chunks=2, direct_min_bytes=n * block + 1)
+    src = torch.randperm(P, device=cuda, generator=gen)[:n]
+    before = pool.clone()
+    mgr.d2h(src.tolist(), list(range(n))).Await()
+    for w in range(S):
+        got = torch.from_numpy(mgr.host_view(w)[:n * block]).to(cuda).view(torch.int32)
+        assert torch.equal(got.view(n, -1), pool[w][src]), w
+    dst = torch.randperm(P, device=cuda, generator=gen)[:n]
+    mgr.h2d(list(range(n)), dst.tolist()).Await()
+    want = before.clone()
+    want[:, dst] = before[:, src]
+    assert torch.equal(pool, want)
+    stats = mgr.engine_stats()
+    assert stats["staged_copies"] == 2 and stats["kernel_launches"] == 6
     mgr.close()
 
 
