@@ -196,9 +196,9 @@ def test_fast_division_matches_integer_division(tmp_path):
 def test_tiled_job_builder_alignment_and_limits(tmp_path):
     """The job builder of libkvx on the CPU (tests/tiled_jobs_check.cc):
     buffers below the element size's alignment are refused for every form,
-    and the 32-bit unit limits are re-checked at the vector width the
-    buffers allow (an 8 GiB int8 tensor at 1- or 2-byte alignment is refused
-    instead of wrapping its unit indices)."""
+    the 32-bit unit limits hold at every width (an 8 GiB int8 tensor at 1- or
+    2-byte alignment stays refused), and odd widths and column-major matrices
+    take the form, vectors and number of units they should."""
     cxx = shutil.which("g++") or shutil.which("c++")
     libdir = os.path.join(ROOT, "tpu-sync_amd")
     if cxx is None or not os.path.exists(os.path.join(libdir, "libkvx.so")):

@@ -418,9 +418,10 @@ Status AppendTiledJobs(const TiledPlan& p, uint64_t tiled, uint64_t linear, int6
   const int v = p.standard ? packed(UnitVector(p.W, p.tW, static_cast<uint64_t>(s))) : 1;
   const bool lanes = p.P > 1 && !tile && v == 16;
   // The kernels index units in 32 bits. A tensor too large for the general
-  // form is taken only where its units fit at the vectors the buffers'
-  // alignment allows too, so that whether a size is accepted does not depend
-  // on which vectors move it.
+  // form is taken only where its units would fit at aligned vectors of its
+  // buffers as well, so that whether a call is accepted does not depend on
+  // which vectors move it. What passes here without a standard form has a
+  // general one (PlanTiled).
   const bool use_std = p.standard && StdUnitsFit(p, v, tile);
   const int aligned = packed(WidestVector(tiled | linear, p.vec));
   if (p.standard && p.gen.empty() &&
@@ -498,12 +499,6 @@ Status AppendTiledJobs(const TiledPlan& p, uint64_t tiled, uint64_t linear, int6
     j.dev.tile_elems = static_cast<uint32_t>(p.tH * p.tW);
     j.dev.log2s = static_cast<uint32_t>(__builtin_ctz(static_cast<unsigned>(s)));
   } else {
-    if (p.gen.empty()) {
-      return UnimplementedError("tiled copy: buffers not aligned for this layout's vectors");
-    }
-    if (((tiled | linear) & static_cast<uint64_t>(s - 1)) != 0) {
-      return InvalidArgumentError("tiled copy: buffers not aligned to the element size");
-    }
     j.vec = 0;
     j.dev.mode = tile ? kTileGen : kDetileGen;
     j.dev.lo = static_cast<uint64_t>(lo / s);
