@@ -141,13 +141,13 @@ typedef struct kvx_manager_config {
                                    workgroups share a CU (faster random reads
                                    and writes; keeps LDS-heavy kernels of other
                                    streams off those CUs meanwhile): every
-                                   gather of one block size from 16 KiB up; of
-                                   2048 workgroups and more, other gathers, and
-                                   scatters of blocks under 16 KiB, of several
-                                   block sizes none above 16 KiB, or of
-                                   160 MiB and more (of one block size only if
-                                   it is whole KiB up to 1 MiB and there are 32
-                                   ids); 0 = 2, -1 = no limit */
+                                   gather of one block size from 16 KiB up;
+                                   other gathers of 2048 workgroups and more;
+                                   scatters of as many, if their blocks go
+                                   packed (under 8 KiB) or, from 160 MiB on, in
+                                   slices (whole KiB; half as many of them where
+                                   the ids lie far apart); 0 = 2,
+                                   -1 = no limit */
 } kvx_manager_config;
 
 /* D2h/H2d dispatch (kv_cache_manager_base.cc:452-512, 2575-2630): ENV (0)

@@ -320,8 +320,9 @@ def any_size_round_trip(kvx, cuda, rng, block, side, layers, blocks, n):
         mgr.close()
 
 
-# Block bytes around a vector, a lane's share, the whole-block limit (16 KiB)
-# and a workgroup's pass (32 KiB), with side tables of other sizes.
+# Block bytes around a vector, a lane's share, the whole-block limits (8 KiB
+# scattered, 16 KiB gathered) and a workgroup's pass (32 KiB), with side tables of
+# other sizes.
 ANY_SIZES = [(1, 4), (3, 1), (7, 8), (15, 4), (16, 4), (17, 32), (33, 4), (255, 2), (1000, 4),
              (2048, 4), (2560, 12), (4095, 4), (4097, 32), (8190, 4), (8192, 4), (8193, 20),
              (10250, 4), (16367, 4), (16368, 4), (16383, 4), (16384, 4), (16385, 4), (16400, 4),
@@ -341,7 +342,8 @@ def test_gather_scatter_of_any_block_size(kvx, cuda, block, side):
 @pytest.mark.parametrize("block", [64, 1000, 8200, 16367, 16368, 16383])
 def test_gather_scatter_of_full_packed_workgroups(kvx, cuda, block):
     """Packed launches of 512 workgroups and more, whose workgroups take all the
-    blocks they can (up to 2048 vectors), the last one fewer."""
+    blocks they can (up to 2048 vectors), the last one fewer: both directions below
+    8 KiB, gathers above (scatters go whole)."""
     rng = np.random.default_rng(block)
     per = min(256, 2048 // -(-block // 16))
     n = (512 * per + per // 2) // 16 + 3

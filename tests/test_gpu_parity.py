@@ -1146,15 +1146,24 @@ def test_gather_scatter_around_the_inline_id_limits(kvx, cuda, n):
 SLICED = [(2048, 160, 544, 0), (3072, 130, 481, 0), (4096, 160, 351, 4), (16384, 330, 33, 0),
           (16384, 160, 95, 32), (33 << 10, 164, 63, 0), (32768, 164, 32, 0),
           (256 << 10, 22, 40, 0), (1 << 20, 6, 33, 0)]
+# Scatters of ids spread over a pool: pieces of 2, 4 and 8 KiB with 0 to 15 ids past
+# the last group, a side table, one storage; packed blocks across the storages, in
+# the cache too; blocks that stay whole.
+SPREAD = [(2048, 160, 530, 0), (4096, 160, 271, 8), (4096, 1, 41000, 0), (8192, 64, 327, 0),
+          (16384, 64, 165, 32), (32768, 64, 83, 0), (32768, 5, 1026, 0), (4096, 40, 200, 8),
+          (4100, 7, 333, 12), (5000, 160, 230, 4), (7168, 160, 150, 0), (7168, 160, 150, 4),
+          (12288, 64, 230, 16), (24576, 64, 112, 0)]
+SPANS = [c + (0,) for c in SLICED] + [c + (4,) for c in SPREAD]
 
 
-@pytest.mark.parametrize("block,storages,n,side", SLICED, ids=[str(c) for c in SLICED])
-def test_sliced_launches_move_the_same_blocks(kvx, cuda, block, storages, n, side):
+@pytest.mark.parametrize("block,storages,n,side,spread", SPANS, ids=[str(c) for c in SPANS])
+def test_large_launches_move_the_same_blocks(kvx, cuda, block, storages, n, side, spread):
     """Gather and scatter against torch's own indexing, both staging orders
-    (layer-major with a side table), every byte outside the blocks unchanged."""
-    assert block * storages * n >= 160 << 20
+    (layer-major with a side table), every byte outside the blocks unchanged;
+    ids that fill the pool, and (spread) a quarter of it."""
+    assert spread or block * storages * n >= 160 << 20
     gen = torch.Generator(device=cuda).manual_seed(block + n)
-    P = n + 9
+    P = spread * n if spread else n + 9
 
     def words(count):
         return torch.randint(-2**31, 2**31 - 1, (count,), dtype=torch.int32, device=cuda,
@@ -1234,10 +1243,12 @@ def test_sliced_launches_at_any_address(kvx, cuda, block, storages, n, side):
     mgr.close()
 
 
-def test_staged_chunks_of_whole_storages_go_sliced(kvx, cuda):
+@pytest.mark.parametrize("P", [72, 190])
+def test_staged_chunks_of_whole_storages_go_sliced(kvx, cuda, P):
     """A staged offload and reload in chunks of 84 whole storages each (165 MiB,
-    so sliced launches, the second from storage 84 on) and a last chunk of 5."""
-    S, P, n, block = 173, 72, 63, 32768
+    so sliced launches, the second from storage 84 on) and a last chunk of 5;
+    reloaded ids that lie close together and (190) spread."""
+    S, n, block = 173, 63, 32768
     gen = torch.Generator(device=cuda).manual_seed(3)
     pool = torch.randint(-2**31, 2**31 - 1, (S, P, block // 4), dtype=torch.int32, device=cuda,
                          generator=gen)
@@ -1252,7 +1263,8 @@ def test_staged_chunks_of_whole_storages_go_sliced(kvx, cuda):
     for w in range(S):
         got = torch.from_numpy(mgr.host_view(w)[:n * block]).to(cuda).view(torch.int32)
         assert torch.equal(got.view(n, -1), pool[w][src]), w
-    dst = torch.randperm(P, device=cuda, generator=gen)[:n]
+    dst = torch.randperm(P - 2, device=cuda, generator=gen)[:n] + 1
+    dst[5], dst[40] = 0, P - 1
     mgr.h2d(list(range(n)), dst.tolist()).Await()
     want = before.clone()
     want[:, dst] = before[:, src]
@@ -1262,12 +1274,15 @@ def test_staged_chunks_of_whole_storages_go_sliced(kvx, cuda):
     mgr.close()
 
 
+@pytest.mark.parametrize("P", [72, 400])
 @pytest.mark.parametrize("gather", [True, False])
-def test_sliced_launch_skips_and_flags_bad_ids(kvx, cuda, gather):
-    """Bad ids in a whole group and among a storage's last ids: their blocks
-    and staging stay as they were, every other block moves, the flag is set."""
+def test_sliced_launch_skips_and_flags_bad_ids(kvx, cuda, gather, P):
+    """Bad ids in whole groups and among a storage's last ids: their blocks
+    and staging stay as they were, every other block moves, the flag is set;
+    slices storage by storage and (a scatter into the larger pool) in every
+    storage at once."""
     import ctypes
-    S, P, n, words = 96, 70, 61, 32768 // 4
+    S, n, words = 96, 63, 32768 // 4
     pool = torch.arange(S * P * words, dtype=torch.int32, device=cuda).view(S, P, words)
     staging = torch.full((S, n, words), -5, dtype=torch.int32, device=cuda)
     table = torch.tensor([pool[w].data_ptr() for w in range(S)], dtype=torch.int64, device=cuda)

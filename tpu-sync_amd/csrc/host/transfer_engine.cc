@@ -32,6 +32,14 @@ int64_t LaneChunkCap(int64_t cap, size_t index, int64_t left) {
   return std::max<int64_t>(c, 1);
 }
 
+// CopyLaunch::id_span of non-negative ids.
+int64_t IdSpan(const std::vector<int64_t>& ids) {
+  if (ids.empty()) return 0;
+  const auto ends = std::minmax_element(ids.begin(), ids.end());
+  const int64_t last = *ends.second - *ends.first;
+  return last < INT64_MAX ? last + 1 : last;
+}
+
 // A run of compact indices whose host ids are consecutive.
 struct HostRun {
   int64_t i0;
@@ -1322,11 +1330,13 @@ Status TransferEngine::StagedOnLane(const LaneView& lane, Direction dir,
     }
   };
 
+  const int64_t span = IdSpan(cdev);
   auto launch = [&](const std::vector<PiecePlan>& ps, uint64_t buf) -> Status {
     for (size_t p0 = 0; p0 < ps.size(); p0 += kMaxPieces) {
       CopyLaunch cl;
       cl.ids = ids_dev;
       cl.n = n;
+      cl.id_span = span;
       uint64_t acc = align_acc | buf;
       for (size_t k = p0; k < ps.size() && k < p0 + kMaxPieces; ++k) {
         const PiecePlan& p = ps[k];
@@ -1683,6 +1693,7 @@ StatusOr<CopyFuture> TransferEngine::DeviceCopy(
                                            arg_host_ + aoff, arg_bytes,
                                            hipMemcpyHostToDevice, stream));
   }
+  const int64_t span = gather ? 0 : IdSpan(ids);
   int64_t off = 0;
   for (size_t g0 = 0; g0 < groups.size(); g0 += kMaxPieces) {
     CopyLaunch cl;
@@ -1692,6 +1703,7 @@ StatusOr<CopyFuture> TransferEngine::DeviceCopy(
       cl.ids = reinterpret_cast<const int64_t*>(arg_dev_ + aoff);
     }
     cl.n = n;
+    cl.id_span = span;
     for (size_t gi = g0; gi < groups.size() && gi < g0 + kMaxPieces; ++gi) {
       const Group& gr = groups[gi];
       const int64_t W = static_cast<int64_t>(gr.members.size());

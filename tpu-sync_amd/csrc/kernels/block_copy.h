@@ -55,6 +55,10 @@ struct CopyLaunch {
   const uint32_t* inline_ids = nullptr;
   const int64_t* ids2 = nullptr;  // block ids on the `others` side (if used)
   int64_t n = 0;
+  // Largest id - smallest id + 1 where the host knows the ids, else 0. Scatters
+  // of ids that lie close together take another order (it never changes what a
+  // launch accepts or writes).
+  int64_t id_span = 0;
   int32_t* error = nullptr;      // optional device word; set to 1 on a bad id
   // 0: one workgroup per large block (best for HBM-bound copies). Otherwise
   // at most about this many workgroups: each then moves a run of
@@ -62,11 +66,10 @@ struct CopyLaunch {
   // zero-copy kernel needs only a few hundred workgroups in flight).
   int64_t max_workgroups = 0;
   // Copies between device buffers reserve LDS so that at most this many of
-  // their workgroups share a CU (0: no limit): gathers of one block size that do
-  // not go packed or sliced always; packed and sliced copies, and those of
-  // several block sizes, from 2048 workgroups on, of their scatters only those
-  // that are sliced, whose blocks are at most 16 KiB or that move 160 MiB and
-  // more. Fewer random accesses in flight per CU let the
+  // their workgroups share a CU (0: no limit): gathers of one block size that go
+  // neither packed nor sliced always; other gathers, and scatters that go packed
+  // or sliced, from 2048 workgroups on (half as many of those scatters that keep
+  // every storage in flight). Fewer random accesses in flight per CU let the
   // DRAM serve them more efficiently: 2 measured 74.5 -> 76.0 % of HBM peak for
   // a gather of 512 x 64 blocks of 32 KiB (1 and 3 the same, 4 and 6 no gain),
   // 67.2 -> 69.9 % for fp8 payload (16 KiB) + scales, and for scatters of packed
@@ -96,6 +99,7 @@ hipError_t LaunchBlockCopy(const CopyLaunch& l, CopyDir dir, int vec_bytes,
 // where LaunchBlockCopy would refuse the launch's sizes.
 struct BlockCopyRoute {
   const char* kernel = nullptr;
+  uint32_t piece_kib = 0;  // the sliced kernel's pieces (else 0)
   uint64_t workgroups = 0;
   uint32_t lds_bytes = 0;
 };

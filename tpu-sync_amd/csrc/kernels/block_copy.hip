@@ -4,8 +4,8 @@
 // itself. Every lane of a 256-lane workgroup (four wave64s) keeps kUnroll
 // independent 16-byte loads in flight before it stores, which is what saturates
 // HBM on a streaming copy. Large launches of blocks that are whole KiB go in
-// slices of many blocks to a workgroup; otherwise blocks of >= 16 KiB get a
-// workgroup each. The block id and
+// slices of several blocks to a workgroup; otherwise blocks of 8 KiB (gathered:
+// 16 KiB) and more get a workgroup each. The block id and
 // the storage base are workgroup-uniform, so the compiler reads them with
 // scalar loads into SGPRs: the id table is read once per block, broadcast
 // through SGPRs instead of an LDS round trip and barrier. Smaller blocks (one
@@ -90,6 +90,8 @@ struct KPiece {
   uint32_t bpw;       // blocks per workgroup
   uint32_t wg_begin;  // first workgroup of the piece
   uint32_t whole;     // 1: every lane works on one block at a time
+  uint32_t across;    // small blocks: > 0: of this many storages, from w0 on, the
+  uint32_t w0;        // same id of each, then the next id (0: storage by storage)
 };
 
 // A kernel's one argument: its parameters and, with kCap > 0, the block ids
@@ -261,9 +263,12 @@ __device__ __forceinline__ void copy_small_blocks(const KPiece& p, uint64_t ids,
   const uint32_t left = p.nblocks - b0;
   const uint32_t nb = left < p.bpw ? left : p.bpw;
   for (uint32_t b = threadIdx.x; b < nb; b += kThreads) {
-    const uint32_t f = p.f0 + b0 + b;
-    const uint32_t w = f / n;
-    const uint32_t i = f - w * n;
+    const uint32_t f = (p.across != 0 ? 0 : p.f0) + b0 + b;
+    const uint32_t d = p.across != 0 ? p.across : n;
+    const uint32_t q = f / d;
+    const uint32_t r = f - q * d;
+    const uint32_t w = p.across != 0 ? p.w0 + r : q;
+    const uint32_t i = p.across != 0 ? q : r;
     const int64_t id = lane_id<kCap>(ids, i);
     const uint64_t base = gptr<const uint64_t>(p.storages)[w];
     bool bad = bad_id(id, p.pool_blocks);
@@ -431,17 +436,24 @@ __global__ __launch_bounds__(kThreads) void block_copy_fast_kernel(Args<FastPara
   fast_block<kGather, kOrder, kCap>(args.p, ids_address<FastParams, kCap>(args.p.ids), blockIdx.x);
 }
 
-// Blocks of a whole number of KiB over whole storages, in slices: a wave moves
-// 1 KiB slices of up to 8 blocks with consecutive ids, a workgroup one slice of
-// 32 blocks of one storage, and consecutive workgroups the other slices of those
-// blocks. A workgroup's bytes are thus short pieces of many blocks, which the
-// random side's DRAM serves better than one block at a time. Bound by HBM, per
-// launch: 512 random 32 KiB blocks of 64 storages gathered in 336 us and
-// scattered in 366 (a whole block to a workgroup: 356, sliced in four, and 390),
-// 768 x 160 of 4 KiB gathered in 163 (packed: 177), 0.54 GB of 8 KiB blocks
-// gathered in 172 and scattered in 181 (a workgroup a block: 197 and 214).
-// The last ids of a storage (fewer than 32) are cut the same way, slices of 1 KiB
-// with the id running fastest, 32 to a workgroup, so that every workgroup is full.
+// Blocks of a whole number of KiB over whole storages, in pieces: a workgroup
+// moves one piece of kPiece KiB of each of 32 / kPiece blocks with consecutive
+// ids of one storage, a wave 8 KiB of them. A workgroup's bytes are thus short
+// pieces of several blocks, which the random side's DRAM serves better than one
+// block at a time. Bound by HBM.
+//   kPiece = 1 (gathers, most scatters): consecutive workgroups take the other
+//     slices of the same 32 blocks, storage after storage. 512 random 32 KiB
+//     blocks of 64 storages gathered in 336 us a launch (a whole block to a
+//     workgroup: 356, sliced in four), 768 x 160 of 4 KiB in 163 (packed: 177),
+//     0.54 GB of 8 KiB blocks in 172 (a workgroup a block: 197).
+//   kPiece = 2, 4 and 8 (scatters of 4 to 32 KiB to ids spread over a pool):
+//     consecutive workgroups take the same piece of the same ids in the next
+//     storage, then the next piece. Writes want every storage in flight on some
+//     allocations (512 random 32 KiB blocks of 64 storages, us: a block to a
+//     workgroup, so ordered, 328; this 327; 1 KiB slices storage by storage 396) and
+//     pieces on the others (391, 369, 415).
+// The last ids of a storage (fewer than a group) are cut into 1 KiB slices with
+// the id running fastest, 32 to a workgroup, so that every workgroup is full.
 // The ids and the base are scalar loads, all in flight at once; nothing goes
 // through LDS. A side piece (a scale table) takes the first workgroups.
 constexpr uint32_t kSliceBytes = 1024;                      // 64 lanes x 16 bytes
@@ -456,23 +468,30 @@ struct SlicedParams {
   int64_t pool_blocks;
   uint64_t bytes;      // bytes per block
   uint32_t n;
-  uint32_t w0;         // first storage
-  uint32_t slices;       // slices per block (gridDim.x)
+  uint32_t w0;           // first storage
+  uint32_t slices;       // slices per block
   uint32_t side_wgs;     // workgroups of the side piece and, after them, of
-  uint32_t last_wgs;     // every storage's last ids, in the first extra_planes
-  uint32_t extra_planes; // values of blockIdx.z
+  uint32_t last_wgs;     // every storage's last ids, in the first
+  uint32_t extra_planes; // extra_planes values of blockIdx.z
   uint32_t last_per;     // workgroups of one storage's last ids
   KPiece side;
 };
 
-template <bool kGather, int kCap>
-__global__ __launch_bounds__(kThreads) void block_copy_sliced_kernel(
+// Grid: kPiece = 1: (slices, id groups, extra planes + storages); kPiece > 1:
+// (storages, pieces, extra planes + id groups).
+template <bool kGather, int kPiece, int kCap>
+__global__ __launch_bounds__(kThreads, 4) void block_copy_sliced_kernel(
     Args<SlicedParams, kCap> args) {
   constexpr int V = 16;
+  constexpr uint32_t kIds = kSlices / kPiece;  // ids of a group
+  constexpr uint32_t kPer = kUnroll / kPiece;  // ids of a wave's piece of it
   const SlicedParams& P = args.p;
   const uint64_t ids = ids_address<SlicedParams, kCap>(P.ids);
-  uint32_t wl = blockIdx.z - P.extra_planes;  // the storage
-  uint32_t last = 0;                          // workgroup of its last ids
+  const uint32_t plane = blockIdx.z - P.extra_planes;
+  uint32_t wl = kPiece > 1 ? blockIdx.x : plane;                   // the storage
+  const uint32_t group = kPiece > 1 ? plane : blockIdx.y;
+  const uint32_t piece = kPiece > 1 ? blockIdx.y : blockIdx.x;
+  uint32_t last = 0;                                               // workgroup of its last ids
   const bool whole = blockIdx.z >= P.extra_planes;
   if (!whole) {
     uint32_t g = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
@@ -489,24 +508,25 @@ __global__ __launch_bounds__(kThreads) void block_copy_sliced_kernel(
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const uint32_t lane = (threadIdx.x % 64) * V;
   // The group's first id.
-  const uint32_t first = whole ? blockIdx.y * kSlices : P.n / kSlices * kSlices;
+  const uint32_t first = whole ? group * kIds : P.n / kIds * kIds;
   const uint64_t stg_w = P.staging + w * static_cast<uint64_t>(P.stride_w);
   typename VecT<V>::T v[kUnroll];
   uint64_t pool_at[kUnroll], stg_at[kUnroll];
   bool ok[kUnroll];
   bool all_ok = true, any_bad = false;
   if (whole) {
-    const uint32_t i0 = first + wave * kUnroll;
-    const uint32_t off = blockIdx.x * kSliceBytes;
+    const uint32_t i0 = first + wave * kPer;
+    const uint32_t off = piece * (kPiece * kSliceBytes);
     const uint64_t base = uniform_load<uint64_t>(P.storages, w) + off;
     const uint64_t stg = stg_w + i0 * static_cast<uint64_t>(P.stride_i) + off;
 #pragma unroll
     for (uint32_t u = 0; u < kUnroll; ++u) {
-      const int64_t id = uniform_id<kCap>(ids, i0 + u);
+      const uint32_t i = u / kPiece, sub = u % kPiece * kSliceBytes;
+      const int64_t id = uniform_id<kCap>(ids, i0 + i);
       ok[u] = !bad_id(id, P.pool_blocks);
       all_ok = all_ok && ok[u];
-      pool_at[u] = base + static_cast<uint64_t>(ok[u] ? id : 0) * P.bytes;
-      stg_at[u] = stg + u * static_cast<uint64_t>(P.stride_i);
+      pool_at[u] = base + static_cast<uint64_t>(ok[u] ? id : 0) * P.bytes + sub;
+      stg_at[u] = stg + i * static_cast<uint64_t>(P.stride_i) + sub;
     }
     any_bad = !all_ok;
   } else {
@@ -596,12 +616,49 @@ uint32_t BlocksPerWorkgroup(uint64_t elems) {
   return static_cast<uint32_t>(bpw < 1 ? 1 : bpw);
 }
 
-// Whether a block of `elems` vectors goes whole to a workgroup (else packed).
-// Between device buffers that is one of 4 and more vectors a lane (16 KiB):
-// packed, 10 KB blocks of 64 storages gather 190 against 236 us and scatter 208
-// against 225 (0.54 GB a launch).
-bool WholeBlock(uint64_t elems, bool paged) {
-  return elems >= (paged ? 2 : 4) * kThreads;
+// Launches of fewer bytes have both their sides in the 256 MB last-level cache
+// and no DRAM order to gain from: they keep the kernels that start faster (64 x
+// 64 blocks of 32 KiB scattered in 46.6 us against 48.4 sliced, 256 x 160 of 4
+// KiB, at the line, in 65.0 against 62.6).
+constexpr uint64_t kSlicedMinBytes = 160 << 20;
+
+// Whether a launch goes storage by storage: gathers, and scatters above the
+// cache whose ids fill two fifths of their range (unknown: of the pool) or more.
+// The neighbouring blocks of one storage are then in flight together, which most
+// allocations serve better. Other scatters keep every storage in flight at once,
+// which some allocations need. 512 32 KiB blocks of 64 storages, us, storage by
+// storage and all at once: every id of a range, shuffled, 335 and 368 (five of
+// seven allocations alike), 333 and 327 (the other two); every second 360 and
+// 366, 354 and 329; every third 373 and 368, 363 and 328; random out of 16384 415
+// and 370, 396 and 329. 16 KiB: 166 and 192, 166 and 168; 174 and 194, 173 and
+// 167; 181 and 192, 181 and 167; 207 and 195, 200 and 168. One in two still gains
+// more on the five than it loses on the two, one in three no longer. In the cache
+// dense ids gain little on the five (12 KiB blocks, 80 MiB: 33.0 and 34.1) and lose on
+// the two (32.7 and 29.3).
+bool ByStorage(const CopyLaunch& l, CopyDir dir) {
+  if (dir == CopyDir::kGather) return true;
+  int64_t span = l.id_span;
+  uint64_t total = 0;
+  for (int k = 0; k < l.npieces && k < kMaxPieces; ++k) {
+    const CopyPiece& c = l.pieces[k];
+    if (c.nblocks <= 0 || c.block_bytes <= 0) return false;
+    if (l.id_span <= 0) span = std::max(span, c.pool_blocks);
+    uint64_t bytes = 0;
+    if (__builtin_mul_overflow(static_cast<uint64_t>(c.nblocks),
+                               static_cast<uint64_t>(c.block_bytes), &bytes) ||
+        __builtin_add_overflow(total, bytes, &total)) {
+      total = UINT64_MAX;
+    }
+  }
+  return total >= kSlicedMinBytes && l.n > 0 && l.n <= INT32_MAX && span / 5 * 2 <= l.n;
+}
+
+// Whether a block of `elems` vectors goes whole to a workgroup (else packed):
+// one of 2 and more vectors a lane (8 KiB), but copies between device buffers
+// that go storage by storage pack up to 4 (16 KiB): 10 KB blocks of 64 storages
+// gather in 190 us packed, 236 whole (0.54 GB a launch).
+bool WholeBlock(uint64_t elems, bool paged, bool by_storage) {
+  return elems >= (!paged && by_storage ? 4 : 2) * kThreads;
 }
 
 // Whether a piece's other side is a second paged buffer (host memory that the
@@ -612,7 +669,15 @@ bool Paged(const CopyLaunch& l) {
   return paged;
 }
 
-bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
+// Packed blocks of this size and more take the same id of every storage in turn
+// where a scatter keeps every storage in flight: above the cache, and beside a
+// scale table. us, storage by storage and so, on the two kinds of allocation: 7000
+// bytes, 400 MiB, 178 and 178, 176 and 150; 4 KiB with 8-byte scales, 100 MiB, 44.5
+// and 44.8, 44.9 and 40.1 (6 KiB with 12 43.8 and 44.4, 43.2 and 39.7). 4 KiB
+// alone in the cache: 42.5 and 45.3, 41.6 and 40.1. Smaller ones do not mind
+// (2 KiB with 4-byte scales 163 us on both, 400 MiB).
+constexpr uint64_t kAcrossMinBytes = 4096;
+bool BuildParams(const CopyLaunch& l, bool by_storage, int vec_bytes, KParams* P,
                  uint32_t* grid) {
   if (l.npieces < 1 || l.npieces > kMaxPieces ||
       (l.ids == nullptr && (l.inline_ids == nullptr || l.n > kMaxInlineIds || Paged(l))) ||
@@ -635,10 +700,18 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
     }
     return v;
   };
-  uint64_t total_blocks = 0;
+  uint64_t total_blocks = 0, total_bytes = 0;
   for (int k = 0; k < l.npieces; ++k) {
-    total_blocks += static_cast<uint64_t>(l.pieces[k].nblocks > 0 ? l.pieces[k].nblocks : 0);
+    const uint64_t blocks = l.pieces[k].nblocks > 0 ? l.pieces[k].nblocks : 0;
+    total_blocks += blocks;
+    uint64_t bytes = 0;
+    if (l.pieces[k].block_bytes <= 0 ||
+        __builtin_mul_overflow(blocks, static_cast<uint64_t>(l.pieces[k].block_bytes), &bytes) ||
+        __builtin_add_overflow(total_bytes, bytes, &total_bytes)) {
+      total_bytes = UINT64_MAX;
+    }
   }
+  const bool across = !paged && !by_storage && (l.npieces > 1 || total_bytes >= kSlicedMinBytes);
   // Pieces of smaller blocks (side tables) take the first workgroups, so their
   // few workgroups run alongside the large blocks instead of after them.
   int order[kMaxPieces];
@@ -668,7 +741,7 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
     const uint64_t bytes = static_cast<uint64_t>(c.block_bytes);
     const uint64_t vec = vec_of(bytes);
     uint64_t elems = bytes / vec;
-    const bool whole = WholeBlock(elems, paged);
+    const bool whole = WholeBlock(elems, paged, by_storage);
     if (!whole && bytes % vec != 0) ++elems;
     uint64_t bpw = whole ? 1 : BlocksPerWorkgroup(elems);
     // A launch that does not fill the chip has fewer vectors a lane instead (16
@@ -703,6 +776,11 @@ bool BuildParams(const CopyLaunch& l, int vec_bytes, KParams* P,
     kp.rest = static_cast<uint32_t>(bytes % vec);
     kp.bpw = static_cast<uint32_t>(bpw);
     kp.whole = whole ? 1u : 0u;
+    const uint32_t n = P->n;
+    if (!whole && across && bytes >= kAcrossMinBytes && kp.f0 % n == 0 && kp.nblocks % n == 0) {
+      kp.across = kp.nblocks / n;
+      kp.w0 = kp.f0 / n;
+    }
     kp.wg_begin = static_cast<uint32_t>(wg);
     wg += (static_cast<uint64_t>(c.nblocks) + bpw - 1) / bpw;
     if (wg > INT32_MAX) return false;
@@ -761,29 +839,37 @@ bool BuildFastSideParams(const KParams& K, CopyDir dir, FastParams* F, KPiece* s
   return true;
 }
 
-// Slices of a block when a launch goes sliced, else 0: blocks of 2 KiB and more
-// that are whole KiB, over whole storages, at least one group of 32 ids. Launches
-// whose two sides fit the 256 MB last-level cache have no DRAM order to gain
-// from and keep the other kernels (64 x 64 blocks of 32 KiB scattered in 46.6 us
-// against 48.4 sliced, 256 x 160 of 4 KiB, at the line, in 65.0 against 62.6);
-// gathers of 512 KiB blocks measured 185 us whole and 192 sliced (0.54 GB), 256
-// KiB ones 184 and 177, scatters up to 1 MiB 193 and 184.
-constexpr uint64_t kSlicedMinBytes = 160 << 20;
-uint32_t SlicesOf(const KPiece& p, uint32_t n, CopyDir dir) {
+// KiB of the pieces a launch is cut into when it goes sliced, else 0. Over
+// whole storages, at least 32 ids, and above the cache.
+//   1 KiB: gathers of whole KiB from 2 to 256 KiB (512 KiB blocks measured 185
+// us whole and 192 sliced, 0.54 GB, 256 KiB ones 184 and 177), scatters of dense
+// ids up to 1 MiB (193 and 184), and scatters of 2 and 3 KiB, packed otherwise
+// (480 MB of 3 KiB 170 and 163 us).
+//   Other scatters: blocks of 4, 8, 16 and 32 KiB in halves of up to 8 KiB. us on
+// the two kinds of allocation: 32 KiB whole 391 and so 370, 326 and 328; 16 KiB 202
+// and 195, 168 and 168; 8 KiB 207 and 202, 166 and 168; 4 KiB storage by storage
+// 163 and so 158, 162 and 140. The others stay whole or packed: 6, 12, 20 and
+// 24 KiB in pieces lost on the second kind (141 and 147, 176 and 182, 175 and 181,
+// 166 and 173) and gained little or nothing on the first, 64 KiB 329 and 339.
+uint32_t PieceKib(const KPiece& p, uint32_t n, CopyDir dir, bool by_storage) {
   if (p.others != 0 || p.bytes % kSliceBytes != 0 || p.bytes < 2 * kSliceBytes) return 0;
-  if (p.bytes > (dir == CopyDir::kGather ? 256u << 10 : 1u << 20)) return 0;
   if (n < kSlices || p.f0 % n != 0 || p.nblocks % n != 0) return 0;
   if (p.bytes * p.nblocks < kSlicedMinBytes) return 0;
-  return static_cast<uint32_t>(p.bytes / kSliceBytes);
+  const uint32_t kib = static_cast<uint32_t>(std::min<uint64_t>(p.bytes / kSliceBytes, 1u << 20));
+  if (dir == CopyDir::kGather) return kib <= 256 ? 1 : 0;
+  if (by_storage) return kib <= 1024 ? 1 : 0;
+  if (kib < 4) return 1;
+  return kib == 4 || kib == 8 ? kib / 2 : kib == 16 || kib == 32 ? 8 : 0;
 }
 
 // The sliced launch of one piece, or of one behind a side piece of smaller
 // blocks; *grid receives its workgroups.
-bool BuildSlicedParams(const KParams& K, CopyDir dir, SlicedParams* S, dim3* grid) {
+bool BuildSlicedParams(const KParams& K, CopyDir dir, bool by_storage, SlicedParams* S,
+                       dim3* grid, uint32_t* piece_kib) {
   if (K.npieces > 2) return false;
   const KPiece& p = K.p[K.npieces - 1];
-  const uint32_t slices = SlicesOf(p, K.n, dir);
-  if (slices == 0) return false;
+  const uint32_t kib = PieceKib(p, K.n, dir, by_storage);
+  if (kib == 0) return false;
   if (K.npieces == 2 && (K.p[0].whole || K.p[0].others != 0)) return false;
   *S = SlicedParams{};
   S->storages = p.storages;
@@ -796,26 +882,30 @@ bool BuildSlicedParams(const KParams& K, CopyDir dir, SlicedParams* S, dim3* gri
   S->bytes = p.bytes;
   S->n = K.n;
   S->w0 = p.f0 / K.n;
-  S->slices = slices;
-  // Slices, id groups, storages: the grid's dimensions, so that a workgroup
-  // divides nothing to find its place (two divisions cost a gather 4 %: 0.54 GB
-  // of 32 KiB blocks in 176.5 against 169.6 us). The side piece and the last ids
-  // of the storages fill planes of their own before them.
+  S->slices = static_cast<uint32_t>(p.bytes / kSliceBytes);
+  // Pieces, id groups and storages are the grid's dimensions, so that a
+  // workgroup divides nothing to find its place (two divisions cost a gather 4 %:
+  // 0.54 GB of 32 KiB blocks in 176.5 against 169.6 us). The side piece and the
+  // last ids of the storages fill planes of their own before them.
   const uint64_t W = p.nblocks / K.n;
-  const uint64_t groups = K.n / kSlices;
-  const uint64_t per_plane = slices * groups;
-  S->last_per = (K.n % kSlices * slices + kSlices - 1) / kSlices;
+  const uint32_t ids = kSlices / kib;
+  const uint64_t groups = K.n / ids;
+  const uint64_t pieces = S->slices / kib;
+  const uint64_t x = kib > 1 ? W : pieces, y = kib > 1 ? pieces : groups;
+  const uint64_t z = kib > 1 ? groups : W;
+  S->last_per = (K.n % ids * S->slices + kSlices - 1) / kSlices;
   const uint64_t last_wgs = W * S->last_per;
   if (K.npieces == 2) {
     S->side = K.p[0];
     S->side_wgs = K.p[1].wg_begin;
   }
-  const uint64_t extra = (S->side_wgs + last_wgs + per_plane - 1) / per_plane;
-  const uint64_t planes = extra + W;
+  const uint64_t extra = (S->side_wgs + last_wgs + x * y - 1) / (x * y);
+  const uint64_t planes = extra + z;
   S->last_wgs = static_cast<uint32_t>(last_wgs);
   S->extra_planes = static_cast<uint32_t>(extra);
-  if (groups > 65535 || planes > 65535 || per_plane * planes > INT32_MAX) return false;
-  *grid = dim3(slices, static_cast<uint32_t>(groups), static_cast<uint32_t>(planes));
+  if (y > 65535 || planes > 65535 || x * y * planes > INT32_MAX) return false;
+  *grid = dim3(static_cast<uint32_t>(x), static_cast<uint32_t>(y), static_cast<uint32_t>(planes));
+  *piece_kib = kib;
   return true;
 }
 
@@ -830,36 +920,34 @@ constexpr uint32_t kCapGrid = 2048;
 // LDS the kernels with the small-block path declare (its address tables).
 constexpr uint32_t kStaticLds = 2 * kSmallMaxBlocks * sizeof(uint64_t);
 
-// Whether a scatter with packed or several pieces takes the cap on workgroups
-// per CU: where its blocks are at most 16 KiB (the packed ones and those of 4
-// vectors a lane), or its two sides do not fit the last-level cache. Capped and
-// not, in one process: 2 KiB blocks with 4-byte scales 48.7 and 52.4 us (134
-// MB), 16 KiB with 32-byte ones 48.4 and 49.7 (134 MB), 20000 bytes with 4-byte
-// ones 126.0 and 130.5 (314 MB), 8 and 32 KiB storages 113.8 and 115.5 (315
-// MB). Larger blocks whose launch stays in the cache gain nothing and some lose
-// (17 KiB blocks with scales 28.5 and 27.7 us, 20000 bytes 30.7 and 29.4, both
-// 67 MB; 24 KiB 56.0 and 53.9, 135 MB): they leave the CUs' LDS free.
+// Whether a scatter that is neither sliced nor of one size of whole blocks takes
+// the cap on workgroups per CU: if every piece goes packed. Capped and not, in one
+// process: 2 KiB blocks with 4-byte scales 48.7 and 52.4 us (134 MB). Whole blocks
+// with a scale table lose (us, 150 MiB, on two kinds of allocation: 8 KiB 69.6 and
+// 64.9, 62.4 and 53.5; 12 KiB 69.2 and 64.2, 63.0 and 53.2), those of 16 KiB gain
+// nothing on one (53.8 and 53.1) and 2 % on the other, and the cap takes the CUs'
+// LDS from other streams.
 bool CapScatter(const KParams& P) {
-  uint64_t total = 0, largest = 0;
   for (int k = 0; k < P.npieces; ++k) {
-    total += P.p[k].bytes * P.p[k].nblocks;
-    largest = std::max(largest, P.p[k].bytes);
+    if (P.p[k].whole) return false;
   }
-  return largest <= 4 * kThreads * 16 || total >= kSlicedMinBytes;
+  return true;
 }
 
 // What a launch runs: its kernel, that kernel's parameters (the general kernel
 // takes the KParams as they are), its grid and the LDS it reserves.
 struct Choice {
   enum Kernel { kGeneral, kFast, kFastSide, kSliced } kernel = kGeneral;
-  int order = kStorageMajor;
+  int order = kStorageMajor;  // fast kernels
+  uint32_t piece_kib = 0;     // sliced kernel
   dim3 grid;
   uint32_t lds = 0;
   FastSideParams FS;
   SlicedParams S;
 };
 
-Choice Choose(const KParams& P, uint32_t grid, CopyDir dir, int wg_per_cu, bool capped_grid) {
+Choice Choose(const KParams& P, uint32_t grid, CopyDir dir, bool by_storage, int wg_per_cu,
+              bool capped_grid) {
   const bool gather = dir == CopyDir::kGather;
   Choice c;
   c.grid = dim3(grid);
@@ -879,9 +967,14 @@ Choice Choose(const KParams& P, uint32_t grid, CopyDir dir, int wg_per_cu, bool 
   // The reservation that leaves room for wg_per_cu workgroups on a CU.
   const uint32_t room = wg_per_cu > 0 ? kLdsPerCu / static_cast<uint32_t>(wg_per_cu) : 0;
   const uint32_t side_room = room > kStaticLds ? room - kStaticLds : 0;
-  if (!capped_grid && BuildSlicedParams(P, dir, &c.S, &c.grid)) {
+  if (!capped_grid && BuildSlicedParams(P, dir, by_storage, &c.S, &c.grid, &c.piece_kib)) {
     c.kernel = Choice::kSliced;
     if (c.grid.x * c.grid.y * c.grid.z >= kCapGrid) c.lds = side_room;
+    // All storages at once: half as many (512 x 64 random 32 KiB blocks in 369
+    // us, 378 with 2 a CU; 327 and 327 on the other kind of allocation).
+    if (c.piece_kib > 1 && wg_per_cu > 0) {
+      c.lds = kLdsPerCu / static_cast<uint32_t>((wg_per_cu + 1) / 2) - kStaticLds;
+    }
     return c;
   }
   if (BuildFastParams(P, dir, &F, &c.order)) {
@@ -926,6 +1019,10 @@ struct Launcher {
   hipError_t Fast(const FastParams& F) const {
     return Run<FastParams>(block_copy_fast_kernel<kGather, kOrder, kCap>, F);
   }
+  template <bool kGather, int kPiece>
+  hipError_t Sliced(const SlicedParams& S) const {
+    return Run<SlicedParams>(block_copy_sliced_kernel<kGather, kPiece, kCap>, S);
+  }
   template <bool kGather, int kOrder>
   hipError_t FastSide(const FastSideParams& F) const {
     return Run<FastSideParams>(block_copy_fast_side_kernel<kGather, kOrder, kCap>, F);
@@ -940,14 +1037,18 @@ struct Launcher {
 // whole_vec: vector bytes of the launch's whole-block pieces.
 template <int kCap>
 hipError_t Launch(const KParams& P, const uint32_t* inline_ids, uint32_t grid, CopyDir dir,
-                  int wg_per_cu, bool capped_grid, int whole_vec, hipStream_t stream) {
+                  bool by_storage, int wg_per_cu, bool capped_grid, int whole_vec,
+                  hipStream_t stream) {
   const bool gather = dir == CopyDir::kGather;
-  const Choice c = Choose(P, grid, dir, wg_per_cu, capped_grid);
+  const Choice c = Choose(P, grid, dir, by_storage, wg_per_cu, capped_grid);
   const Launcher<kCap> to{inline_ids, P.n, c.grid, c.lds, stream};
   const FastParams& F = c.FS.fast;
   if (c.kernel == Choice::kSliced) {
-    return gather ? to.template Run<SlicedParams>(block_copy_sliced_kernel<true, kCap>, c.S)
-                  : to.template Run<SlicedParams>(block_copy_sliced_kernel<false, kCap>, c.S);
+    if (gather) return to.template Sliced<true, 1>(c.S);
+    return c.piece_kib == 8   ? to.template Sliced<false, 8>(c.S)
+           : c.piece_kib == 4 ? to.template Sliced<false, 4>(c.S)
+           : c.piece_kib == 2 ? to.template Sliced<false, 2>(c.S)
+                              : to.template Sliced<false, 1>(c.S);
   }
   if (c.kernel == Choice::kFast) {
     if (gather) {
@@ -989,11 +1090,14 @@ int LaunchVectorBytes(const CopyLaunch& l, uint64_t extra_align) {
 bool BlockCopyRouteOf(const CopyLaunch& l, CopyDir dir, int vec_bytes, BlockCopyRoute* route) {
   KParams P;
   uint32_t grid = 0;
-  if (!BuildParams(l, vec_bytes, &P, &grid)) return false;
-  const Choice c = Choose(P, grid, dir, l.gather_workgroups_per_cu, l.max_workgroups > 0);
+  const bool by_storage = ByStorage(l, dir);
+  if (!BuildParams(l, by_storage, vec_bytes, &P, &grid)) return false;
+  const Choice c =
+      Choose(P, grid, dir, by_storage, l.gather_workgroups_per_cu, l.max_workgroups > 0);
   static const char* const kNames[] = {"block_copy_kernel", "block_copy_fast_kernel",
                                        "block_copy_fast_side_kernel", "block_copy_sliced_kernel"};
   route->kernel = kNames[c.kernel];
+  route->piece_kib = c.piece_kib;
   route->workgroups = static_cast<uint64_t>(c.grid.x) * c.grid.y * c.grid.z;
   route->lds_bytes = c.lds;
   return true;
@@ -1003,7 +1107,8 @@ hipError_t LaunchBlockCopy(const CopyLaunch& l, CopyDir dir, int vec_bytes,
                            hipStream_t stream) {
   KParams P;
   uint32_t grid = 0;
-  if (!BuildParams(l, vec_bytes, &P, &grid)) return hipErrorInvalidValue;
+  const bool by_storage = ByStorage(l, dir);
+  if (!BuildParams(l, by_storage, vec_bytes, &P, &grid)) return hipErrorInvalidValue;
   if (l.gather_workgroups_per_cu < 0 || l.gather_workgroups_per_cu > 32) {
     return hipErrorInvalidValue;
   }
@@ -1011,12 +1116,13 @@ hipError_t LaunchBlockCopy(const CopyLaunch& l, CopyDir dir, int vec_bytes,
   if (vec_bytes != 16 && vec_bytes != 4 && vec_bytes != 1) return hipErrorInvalidValue;
   const bool capped = l.max_workgroups > 0;
   if (l.ids == nullptr && l.n <= kFewInlineIds) {
-    return Launch<kFewInlineIds>(P, l.inline_ids, grid, dir, cap, capped, 16, stream);
+    return Launch<kFewInlineIds>(P, l.inline_ids, grid, dir, by_storage, cap, capped, 16, stream);
   }
   if (l.ids == nullptr) {
-    return Launch<kMaxInlineIds>(P, l.inline_ids, grid, dir, cap, capped, 16, stream);
+    return Launch<kMaxInlineIds>(P, l.inline_ids, grid, dir, by_storage, cap, capped, 16, stream);
   }
-  return Launch<0>(P, nullptr, grid, dir, cap, capped, Paged(l) ? vec_bytes : 16, stream);
+  return Launch<0>(P, nullptr, grid, dir, by_storage, cap, capped, Paged(l) ? vec_bytes : 16,
+                   stream);
 }
 
 }  // namespace kvx

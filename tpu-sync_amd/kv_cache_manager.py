@@ -228,10 +228,10 @@ class KVCacheManager:
         so that at most this many of their workgroups share a CU, which serves
         their random side faster but keeps LDS-heavy kernels of other streams
         off those CUs while they run (0: 2; -1: no limit): every gather of one
-        block size from 16 KiB up; of 2048 workgroups and more, other gathers,
-        and scatters of blocks under 16 KiB, of several block sizes none above
-        16 KiB, or of 160 MiB and more (of one block size only if it is whole
-        KiB up to 1 MiB and there are 32 ids).
+        block size from 16 KiB up; other gathers of 2048 workgroups and more;
+        scatters of as many, if their blocks go packed (under 8 KiB) or, from
+        160 MiB on, in slices (whole KiB; half as many of them where the ids lie
+        far apart).
       The remaining reference arguments (ports, worker id, timeout,
       parallelism, unsafe_skip_buffer_lock) configure its networking, which
       this single-GPU build does not have; they are accepted and ignored.
