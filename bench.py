@@ -50,15 +50,26 @@ HBM_PEAK_GBPS = 8000.0
 # second run, WRITE_SIZE (KiB per dispatch), each divided by the factor the
 # same counter reads for a plain 1 GiB device copy in the same runs (FETCH
 # 0.50001, WRITE 1.000): profiles/block_copy_llama3_8b_pmc.txt. Keyed by
-# (kernel, algorithmic bytes per launch).
+# (kernel, algorithmic bytes per launch); the ascending and the shuffled runs of
+# ids were counted together.
 MEASURED_TRAFFIC = {
-    ("gather", 2 * 512 * 64 * 32768): int((524452.0 / 0.50001 + 1048621.8 / 1.0) * 1024),
-    ("scatter", 2 * 512 * 64 * 32768): int((524348.2 / 0.50001 + 1048598.9 / 1.0) * 1024),
-    # The ascending and shuffled runs of ids (profiles/hbm_dram_stall_counters.txt,
-    # calibrated by the same run's 1 GiB copy: 0.500011 / 1.0).
-    ("scatter_contiguous", 2 * 512 * 64 * 32768): int((524345.0 / 0.500011 + 1048587.5) * 1024),
-    ("scatter_shuffled", 2 * 512 * 64 * 32768): int((524345.0 / 0.500011 + 1048604.5) * 1024),
+    ("gather", 2 * 512 * 64 * 32768): int((524419.1 / 0.50001 + 1048593.4) * 1024),
+    ("scatter", 2 * 512 * 64 * 32768): int((524347.9 / 0.50001 + 1048647.7) * 1024),
+    ("scatter_contiguous", 2 * 512 * 64 * 32768): int((524347.2 / 0.50001 + 1048832.6) * 1024),
+    ("scatter_shuffled", 2 * 512 * 64 * 32768): int((524347.2 / 0.50001 + 1048832.6) * 1024),
 }
+
+# What the isolated launches run (tests/test_block_routes.py holds this to the
+# library's dispatch): kernel and KiB of each piece of a block a workgroup moves.
+# Pieces of 1 KiB go storage by storage, the others keep every storage in flight.
+ISOLATED_PIECES = {
+    "gather": ("block_copy_sliced_kernel", 1),
+    "scatter": ("block_copy_sliced_kernel", 8),
+    "scatter_contiguous": ("block_copy_sliced_kernel", 1),
+    "scatter_shuffled": ("block_copy_sliced_kernel", 1),
+}
+ISOLATED_KERNELS = {k: f"{kernel} ({kib} KiB of each of {32 // kib} blocks per workgroup)"
+                    for k, (kernel, kib) in ISOLATED_PIECES.items()}
 
 WORKLOADS = {
     "llama3-8b-kv": dict(layers=32, kv_heads=8, head_dim=128, block_tokens=16,
@@ -925,8 +936,8 @@ def bench_weight_sync_tiled(torch, pkg, dev, args):
            "verified": True,
            # HBM bytes per launch from rocprofv3 FETCH_SIZE / WRITE_SIZE with the
            # same calibration (profiles/tiled_copy_weight_sync_trace.txt).
-           "detile_pack_traffic": int((7844374.1 / 0.50001 + 15684196.2) * 1024),
-           "tile_unpack_traffic": int((7844090.4 / 0.50001 + 15692041.6) * 1024),
+           "detile_pack_traffic": int((7844374.7 / 0.50001 + 15684194.1) * 1024),
+           "tile_unpack_traffic": int((7844084.8 / 0.50001 + 15692903.3) * 1024),
            "d2h_gbps": round(d2h_gbps, 2), "h2d_gbps": round(h2d_gbps, 2),
            "cpu_baseline": {"value": round(cpu[4], 2), "unit": "GB/s", "cores": 4, "kind": "port",
                             "all_threads_gbps": round(cpu[max(cpu)], 2), "all_threads": max(cpu),
@@ -988,8 +999,8 @@ def bench_tiled_int8(torch, pkg, dev, args):
         out[f"{name}_frac_of_box_copy"] = frac_of_box(g, args.box_copy_gbps)
     # HBM bytes per launch from rocprofv3 FETCH_SIZE / WRITE_SIZE with the
     # same calibration (profiles/tiled_copy_weight_sync_trace.txt).
-    out["detile_pack_traffic"] = int((458919.1 / 0.50001 + 917621.9) * 1024)
-    out["tile_unpack_traffic"] = int((458925.5 / 0.50001 + 917616.7) * 1024)
+    out["detile_pack_traffic"] = int((458928.1 / 0.50001 + 917643.9) * 1024)
+    out["tile_unpack_traffic"] = int((458923.6 / 0.50001 + 917686.3) * 1024)
     out["verified"] = True
     ws.close()
     del params, staging
@@ -1788,8 +1799,7 @@ def main():
         for _ in range(2):
             fn(idsets[0], staging, stream=ks_stream).Await()
         # The engine brackets each launch with HIP events on ks_stream (the
-        # stream the kernel runs on); the id-table upload before it is not
-        # inside the bracket.
+        # stream the kernel runs on).
         m.kernel_times(gather, reset=True)
         futs = [fn(idsets[k % len(idsets)], staging, stream=ks_stream) for k in range(launches)]
         for f in futs:
@@ -1822,9 +1832,8 @@ def main():
                      "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBPS, 4),
                      "frac_of_box_copy": frac_of_box(ach, args.box_copy_gbps),
                      "traffic": MEASURED_TRAFFIC.get((name, per_launch)),
-                     "kernel": (("block_copy_sliced_gather_kernel (a quarter of each of 4 ids "
-                                 "per workgroup)" if gather else "block_copy_fast_kernel (scatter)")
-                                + f", {n} ids x {S} storages per launch, {what}"),
+                     "kernel": f"{ISOLATED_KERNELS[name]}, {n} ids x {S} storages per launch, "
+                               f"{what}",
                      "launches": args.steps, "avg_launch_us": round(avg_s * 1e6, 2),
                      "bytes_per_launch": int(per_launch), "verified": True}
         log(f"{name} alone: {ach:.0f} GB/s ({ach / HBM_PEAK_GBPS:.1%} of HBM peak, "

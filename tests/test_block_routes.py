@@ -3,16 +3,19 @@ compiled against libkvx."""
 import os
 import shutil
 import subprocess
+import sys
 
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, ROOT)
+import bench  # noqa: E402
 
 
 def test_block_copy_kernels_and_lds(tmp_path):
     """Which kernel a gather or scatter runs and the LDS it reserves, on both
-    sides of each line of the rule: scatters of blocks above 16 KiB beside
-    other sizes reserve none until they move 160 MiB."""
+    sides of each line of the rule; and what the benchmark says its isolated
+    launches run is what they run."""
     cxx = shutil.which("g++") or shutil.which("c++")
     libdir = os.path.join(ROOT, "tpu-sync_amd")
     if cxx is None or not os.path.exists(os.path.join(libdir, "libkvx.so")):
@@ -29,3 +32,5 @@ def test_block_copy_kernels_and_lds(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120, env=env)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "all checks passed" in r.stdout
+    for name, (kernel, kib) in bench.ISOLATED_PIECES.items():
+        assert f"benchmark {name}: {kernel}, {kib} KiB\n" in r.stdout
