@@ -152,8 +152,8 @@ struct EngineOptions {
   // direction with its own streams, staging ring and SDMA engine (0: leave
   // such copies to the runtime's pageable hipMemcpyAsync).
   int host_copy_threads = 8;
-  // Workgroups of a one-block-per-workgroup gather that may share a CU
-  // (CopyLaunch::gather_workgroups_per_cu; 0: no limit).
+  // Workgroups of a gather, or of a scatter that goes packed or sliced, that may
+  // share a CU (CopyLaunch::gather_workgroups_per_cu; 0: no limit).
   int gather_workgroups_per_cu = kDefaultGatherWorkgroupsPerCu;
 };
 
