@@ -144,7 +144,8 @@ typedef struct kvx_manager_config {
                                    gather of one block size from 16 KiB up;
                                    other gathers of 2048 workgroups and more;
                                    scatters of as many, if their blocks go
-                                   packed (under 8 KiB) or, from 160 MiB on, in
+                                   packed (under 8 KiB; under 16 where dense
+                                   ids move 160 MiB) or, from 160 MiB on, in
                                    slices (whole KiB; half as many of them where
                                    the ids lie far apart); 0 = 2,
                                    -1 = no limit */

@@ -229,9 +229,9 @@ class KVCacheManager:
         their random side faster but keeps LDS-heavy kernels of other streams
         off those CUs while they run (0: 2; -1: no limit): every gather of one
         block size from 16 KiB up; other gathers of 2048 workgroups and more;
-        scatters of as many, if their blocks go packed (under 8 KiB) or, from
-        160 MiB on, in slices (whole KiB; half as many of them where the ids lie
-        far apart).
+        scatters of as many, if their blocks go packed (under 8 KiB; under 16
+        where dense ids move 160 MiB) or, from 160 MiB on, in slices (whole KiB;
+        half as many of them where the ids lie far apart).
       The remaining reference arguments (ports, worker id, timeout,
       parallelism, unsafe_skip_buffer_lock) configure its networking, which
       this single-GPU build does not have; they are accepted and ignored.
